@@ -58,8 +58,8 @@ def listed():
         # the 3D blast on blocks, two refinements, the fused march
         {"name": "blast-fused", "kind": "blast", "root": 8, "levels": 2, "steps": 80, "scheme": "mc",
          "path": "fused", "bins": 0},
-        # the same physics with per-block timesteps (two cycles of eight substeps)
-        {"name": "blast-bins", "kind": "blast", "root": 4, "levels": 2, "steps": 16, "scheme": "mc",
+        # the same physics with per-block timesteps (eight cycles of eight substeps)
+        {"name": "blast-bins", "kind": "blast", "root": 4, "levels": 2, "steps": 64, "scheme": "mc",
          "path": "passes", "bins": 3},
         # the published adaptive 2D run's mesh (256^2 root cells, finest 4096^2), default scheme
         {"name": "shear-4096-koren", "kind": "shear", "root": 16, "levels": 4, "steps": 100, "scheme": "koren",
@@ -110,7 +110,7 @@ def draw(rng):
     if kind == "blast":
         bins = rng.choice([0, 0, 0, 2, 3])
         return {"kind": "blast", "root": rng.randint(3, 6), "levels": rng.randint(1, 2),
-                "steps": 2 << bins if bins else _log_int(rng, 10, 60), "scheme": "mc" if bins else scheme,
+                "steps": 8 << bins if bins else _log_int(rng, 10, 60), "scheme": "mc" if bins else scheme,
                 "path": "passes" if bins else "fused", "bins": bins}
     regrid = rng.choice([0, 0, 8])
     return {"kind": "shear", "root": rng.randint(4, 14), "levels": rng.randint(1, 2 if regrid else 3),
