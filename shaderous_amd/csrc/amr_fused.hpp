@@ -92,8 +92,8 @@ __device__ __forceinline__ Half<T> half_at_source(const Params<T>& P, const int*
   sl[1] = axis_slope<T, LIM, ISEN>(P, ym, q, yp, nullptr, nullptr);
   sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
   const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
-  const T jump = tmax(jump_of(xm.p, xp.p), tmax(jump_of(ym.p, yp.p), jump_of(zm.p, zp.p)));
-  return hancock(P, q, sl, conv, jump, dt);
+  const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
+  return hancock<T, LIM>(P, q, sl, conv, jump, dt);
 }
 
 // Flux register: per coarse-fine face of a leaf, its 16 x 16 faces' fluxes (8 values each), in
@@ -463,8 +463,8 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
             scale_inc(sl[2].s, (!oz && (c == 0 || c == AMR_BS - 1)) ? T(0) : T(1));
           }
           const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (pp.vz - pm.vz);
-          const T jump = tmax(jump_of(xm.p, xp.p), tmax(jump_of(ym.p, yp.p), jump_of(pm.p, pp.p)));
-          hc = hancock(P, pc, sl, conv, jump, dt);
+          const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, pm.p, pp.p)));
+          hc = hancock<T, LIM>(P, pc, sl, conv, jump, dt);
         } else {
           // another block's cell (same level, refined, or this block's boundary image): its half
           // step was formed in the shell pass

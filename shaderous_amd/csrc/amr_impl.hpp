@@ -186,6 +186,12 @@ __device__ __forceinline__ Cons<T> mid_cons(const Params<T>& P, const AmrBins& B
 template <int LIM>
 constexpr int prolong_lim() { return (LIM == LIM_MINMOD || LIM == LIM_VANLEER) ? LIM : LIM_MC; }
 
+// The limited slope across a cell: twice its increment toward a face
+template <typename T, int PL>
+__device__ __forceinline__ T slope1(T below, T above) {
+  return T(2) * sym_edge<T, PL>(below, above);
+}
+
 // slope_between with mom_slope (amr/cons.wgsl:57-74): limited slopes of every conserved value,
 // momentum by the product rule from the density and velocity slopes
 template <typename T, int LIM>
@@ -193,19 +199,19 @@ __device__ __forceinline__ Cons<T> slope_between(const Params<T>& P, const Cons<
                                                  const Cons<T>& p) {
   constexpr int PL = prolong_lim<LIM>();
   Cons<T> s;
-  s.a.x = edge1<T, PL>(c.a.x - m.a.x, p.a.x - c.a.x, T(0));
-  s.a.y = edge1<T, PL>(c.a.y - m.a.y, p.a.y - c.a.y, T(0));
-  s.a.z = edge1<T, PL>(c.a.z - m.a.z, p.a.z - c.a.z, T(0));
-  s.a.w = edge1<T, PL>(c.a.w - m.a.w, p.a.w - c.a.w, T(0));
-  s.b.x = edge1<T, PL>(c.b.x - m.b.x, p.b.x - c.b.x, T(0));
-  s.b.y = edge1<T, PL>(c.b.y - m.b.y, p.b.y - c.b.y, T(0));
-  s.b.z = edge1<T, PL>(c.b.z - m.b.z, p.b.z - c.b.z, T(0));
-  s.b.w = edge1<T, PL>(c.b.w - m.b.w, p.b.w - c.b.w, T(0));
+  s.a.x = slope1<T, PL>(c.a.x - m.a.x, p.a.x - c.a.x);
+  s.a.y = slope1<T, PL>(c.a.y - m.a.y, p.a.y - c.a.y);
+  s.a.z = slope1<T, PL>(c.a.z - m.a.z, p.a.z - c.a.z);
+  s.a.w = slope1<T, PL>(c.a.w - m.a.w, p.a.w - c.a.w);
+  s.b.x = slope1<T, PL>(c.b.x - m.b.x, p.b.x - c.b.x);
+  s.b.y = slope1<T, PL>(c.b.y - m.b.y, p.b.y - c.b.y);
+  s.b.z = slope1<T, PL>(c.b.z - m.b.z, p.b.z - c.b.z);
+  s.b.w = slope1<T, PL>(c.b.w - m.b.w, p.b.w - c.b.w);
   const T dc = tmax(c.a.x, P.rho_floor), dm = tmax(m.a.x, P.rho_floor), dp = tmax(p.a.x, P.rho_floor);
   const T vcx = tdiv(c.a.y, dc), vcy = tdiv(c.a.z, dc), vcz = tdiv(c.a.w, dc);
-  const T svx = edge1<T, PL>(vcx - tdiv(m.a.y, dm), tdiv(p.a.y, dp) - vcx, T(0));
-  const T svy = edge1<T, PL>(vcy - tdiv(m.a.z, dm), tdiv(p.a.z, dp) - vcy, T(0));
-  const T svz = edge1<T, PL>(vcz - tdiv(m.a.w, dm), tdiv(p.a.w, dp) - vcz, T(0));
+  const T svx = slope1<T, PL>(vcx - tdiv(m.a.y, dm), tdiv(p.a.y, dp) - vcx);
+  const T svy = slope1<T, PL>(vcy - tdiv(m.a.z, dm), tdiv(p.a.z, dp) - vcy);
+  const T svz = slope1<T, PL>(vcz - tdiv(m.a.w, dm), tdiv(p.a.w, dp) - vcz);
   s.a.y = vcx * s.a.x + c.a.x * svx;
   s.a.z = vcy * s.a.x + c.a.x * svy;
   s.a.w = vcz * s.a.x + c.a.x * svz;
@@ -496,8 +502,8 @@ __device__ __forceinline__ Half<T> predict_texel(const Params<T>& P, const T4<T>
     s.rho *= mk[a]; s.vx *= mk[a]; s.vy *= mk[a]; s.vz *= mk[a]; s.p *= mk[a]; s.s *= mk[a];
   }
   const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
-  const T jump = tmax(jump_of(xm.p, xp.p), tmax(jump_of(ym.p, yp.p), jump_of(zm.p, zp.p)));
-  return hancock(P, q, sl, conv, jump, dt);
+  const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
+  return hancock<T, LIM>(P, q, sl, conv, jump, dt);
 }
 
 template <typename T, int LIM, bool ISEN, int D = 3>

@@ -7,6 +7,15 @@
 //
 // The arithmetic follows the reference's WGSL with every optional module off; each function
 // cites the file and lines it follows (paths under the reference's src/).
+//
+// The fused kernels are bound by VALU issue, and a reciprocal, root, log or exp takes the issue
+// slots of four other instructions, so the formulas here are arranged for few of both: one set of
+// expressions for every state a face can have (riemann), Koren's weight once per channel for both
+// edges, increments kept at the size they are used at, no root or quotient where a product tells
+// the same. Against the reference's own arrangement, with the same tiles and launches: turbulence
+// 256^3 (MC) 0.578 -> 0.52 ms per step, KH 2048^2 (Koren + isentropic) 0.182 -> 0.146, Sedov 128^3
+// (the same scheme) 0.157 -> 0.121, turbulence 96^3 in FP64 0.316 -> 0.275; the error against 64
+// bits after 100 to 200 steps as before (2e-7 to 3e-7), half for Sedov.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -133,141 +142,151 @@ __device__ __forceinline__ T bc_vel(T v, int flip, int side) {
 }
 
 // ---- limiters: hydro/limiters/*.wgsl, per channel ----
-// Koren's smoothness measure of a channel against its natural scale s = 0.01 scale: the
-// difference energy over s^2 (koren.wgsl:274-292), or, where s^2 over- or underflows, the
-// differences scaled by 1/|s| first. What depends on the scale alone is formed once per scale
-// (a cell's six channels have four: rho, c_s three times, p, none) and shared by its edges.
+// Increments are kept as the step from a cell's centre to its face, half of the reference's
+// (which halves them at each use): every factor left out is a power of two, so the values are
+// the same, and the symmetric limiters lose two doublings per channel.
+//
+// Koren's smoothness measure of a channel (koren.wgsl:274-292) is the difference energy over the
+// square of its natural scale s = 0.01 scale. Here the differences are scaled by 1/|s| and then
+// squared, which neither over- nor underflows; a zero scale stands for 1e-15, the root of the
+// reference's smallest s^2. It depends on the scale alone and is formed once per scale (a cell's
+// six channels have four: rho, c_s three times, p, none).
 template <typename T>
-struct EdgeScale { T s2inv; T k; bool as_is; };
-
-template <typename T>
-__device__ __forceinline__ EdgeScale<T> edge_scale(T scale) {
-  const T SMOOTH = T(0.01);
-  T s = SMOOTH * scale;
-  T s2 = s * s;
-  EdgeScale<T> e;
-  e.as_is = (s2 >= T(1e-30) && s2 < T(1e30)) || (s == T(0));
-  e.s2inv = tmax(s2, T(1e-30));
-  if constexpr (sizeof(T) == 4) e.s2inv = trcp(e.s2inv);   // tdiv(q, ss) = q rcp(ss) in FP32
-  e.k = trcp(tmax(tabs(s), T(1e-37)));
-  return e;
+__device__ __forceinline__ T edge_scale(T scale) {
+  const T s = tabs(T(0.01) * scale);
+  return s == T(0) ? T(1e15) : trcp(tmax(s, T(1e-37)));
 }
 
-// Twice the edge increment from the differences (far, near) and the channel's scale.
-// Koren (koren.wgsl:274-292): its early return gives exactly the blend's value per channel
-// (the blend weight is 1 for a smooth channel), so each channel is formed on its own.
+// Koren's blend weight of a channel from its two differences: the same for the cell's up and
+// down edges, so a pair of edges forms it once.
+template <typename T>
+__device__ __forceinline__ T koren_weight(T below, T above, T k) {
+  const T b = below * k, a = above * k;
+  return tclamp(T(1.5) - (b * b + a * a), T(0), T(1));
+}
+// Koren's increment toward the face `near` lies on, blended by w from the limited value to the
+// plain one (w = 1 gives the plain one exactly: the limited value is no larger). The early return
+// of koren.wgsl gives the blend's value per channel, so each channel is formed on its own.
+template <typename T>
+__device__ __forceinline__ T koren_edge(T far, T near, T w) {
+  const T fr = (far + T(2) * near) * T(1.0 / 6.0);
+  // sign(near) min(|far|, |near|, |fr|) where far and near share a sign (fr then does too)
+  const T lim = minmod(far, minmod(near, fr));
+  return tmix(lim, fr, w);
+}
+// The symmetric limiters' increment from the two differences, the same toward both faces
 template <typename T, int LIM>
-__device__ __forceinline__ T edge1(T far, T near, const EdgeScale<T>& sc) {
-  if constexpr (LIM == LIM_KOREN) {
-    T fr = (far + T(2) * near) * T(1.0 / 3.0);
-    T q = far * far + near * near;
-    T eta;
-    if (sc.as_is) {
-      // FP32: q times the reciprocal (tdiv's form); FP64: the quotient (s2inv holds ss)
-      if constexpr (sizeof(T) == 4) eta = q * sc.s2inv;
-      else eta = tdiv(q, sc.s2inv);
-    } else {
-      T fk = far * sc.k, nk = near * sc.k;
-      eta = fk * fk + nk * nk;
-    }
-    // sign(near) min(2|far|, 2|near|, |fr|) where far and near share a sign (fr then does too)
-    T lim = minmod(T(2) * far, minmod(T(2) * near, fr));
-    T w = tclamp(T(1.5) - eta, T(0), T(1));
-    return (w == T(1)) ? fr : tmix(lim, fr, w);
-  } else if constexpr (LIM == LIM_MC) {
-    // sign(far) min(2|far|, 2|near|, |far + near| / 2) where far and near share a sign
-    return minmod(T(2) * far, minmod(T(2) * near, T(0.5) * (far + near)));
+__device__ __forceinline__ T sym_edge(T below, T above) {
+  if constexpr (LIM == LIM_MC) {
+    // sign min(|below|, |above|, |below + above| / 4) where the two share a sign
+    return minmod(below, minmod(above, T(0.25) * (below + above)));
   } else if constexpr (LIM == LIM_MINMOD) {
-    return minmod(far, near);
+    return T(0.5) * minmod(below, above);
   } else {
-    return same_sign(far, near) ? T(2) * far * tdiv(near, far + near) : T(0);
+    return same_sign(below, above) ? below * tdiv(above, below + above) : T(0);
   }
-}
-// The same from the scale itself (callers with one channel per scale)
-template <typename T, int LIM>
-__device__ __forceinline__ T edge1(T far, T near, T scale) {
-  EdgeScale<T> sc{};
-  if constexpr (LIM == LIM_KOREN) sc = edge_scale(scale);
-  return edge1<T, LIM>(far, near, sc);
 }
 template <int LIM> constexpr bool lim_symmetric() { return LIM != LIM_KOREN; }
 
-// Twice the increment of each reconstructed channel (rho, vx, vy, vz, p, s) toward a face.
+// The increment of one channel toward the upper (UP) or lower face; k: edge_scale of the
+// channel's scale (Koren)
+template <typename T, int LIM, bool UP>
+__device__ __forceinline__ T edge1(T below, T above, T k) {
+  if constexpr (LIM == LIM_KOREN) {
+    const T w = koren_weight(below, above, k);
+    return UP ? koren_edge(below, above, w) : koren_edge(above, below, w);
+  } else {
+    return sym_edge<T, LIM>(below, above);
+  }
+}
+
+// The increment of each reconstructed channel (rho, vx, vy, vz, p, s) toward a face.
 template <typename T>
 struct Inc { T rho, vx, vy, vz, p, s; };
 
 // isen_inc / isen_blend (hydro/q.wgsl:183-213) with no reference state and no potential, in two
 // parts: what depends only on the three cells (the densities along the adiabat through the
 // centre, the smoothness, adiabat and shear switches), shared by a cell's up and down edges, and
-// the edge's own blend.
+// the edge's own blend. Everything that divides by the centre's pressure shares one reciprocal:
+// (p_c / p)^(1/gamma) is taken as (p / p_c)^(-1/gamma).
 template <typename T>
-struct IsenCommon { bool ok; T gi, tl, tr, room; };
+struct IsenCommon { bool ok; T gi, ipc, tl, tr, bound; };
 
 template <typename T>
 __device__ __forceinline__ IsenCommon<T> isen_common(const Params<T>& P, const Prim<T>& l, const Prim<T>& c,
                                                      const Prim<T>& r) {
-  const T ISEN_SMOOTH = T(0.2), ISEN_ADIABAT = T(0.01), ISEN_SHEAR = T(0.1), ISEN_ROOM = T(0.01);
+  const T ISEN_SMOOTH = T(0.2), ISEN_ADIABAT = T(0.01), ISEN_SHEAR = T(0.1), ISEN_ROOM = T(0.01), ISEN_CAP = T(0.25);
   IsenCommon<T> k;
-  k.ok = l.rho > T(0) && l.p > T(0) && c.rho > T(0) && c.p > T(0) && r.rho > T(0) && r.p > T(0);
+  // (the unassembled edge texels of a block are zeros)
+  k.ok = tmin(tmin(tmin(l.rho, l.p), tmin(c.rho, c.p)), tmin(r.rho, r.p)) > T(0);
   k.gi = trcp(P.gamma);
-  k.tl = l.rho * tpow(tdiv(c.p, l.p), k.gi) - c.rho;
-  k.tr = r.rho * tpow(tdiv(c.p, r.p), k.gi) - c.rho;
-  T ks = tclamp(T(2) - tdiv(tmax(tabs(l.p - c.p), tabs(r.p - c.p)), ISEN_SMOOTH * c.p), T(0), T(1));
+  k.ipc = trcp(c.p);
+  k.tl = l.rho * tpow(l.p * k.ipc, -k.gi) - c.rho;
+  k.tr = r.rho * tpow(r.p * k.ipc, -k.gi) - c.rho;
+  T ks = tclamp(T(2) - tmax(tabs(l.p - c.p), tabs(r.p - c.p)) * (k.ipc * T(1.0 / ISEN_SMOOTH)), T(0), T(1));
   T ka = tclamp(T(2) - tdiv(tmax(tabs(k.tl), tabs(k.tr)), ISEN_ADIABAT * c.rho), T(0), T(1));
   T dxr = r.vx - c.vx, dyr = r.vy - c.vy, dzr = r.vz - c.vz;
   T dxl = c.vx - l.vx, dyl = c.vy - l.vy, dzl = c.vz - l.vz;
-  T dvr = tsqrt(dxr * dxr + dyr * dyr + dzr * dzr);
-  T dvl = tsqrt(dxl * dxl + dyl * dyl + dzl * dzl);
-  T kv = tclamp(T(2) - tdiv(tmax(dvr, dvl), ISEN_SHEAR * tmax(c.cs, T(1e-30))), T(0), T(1));
-  k.room = ISEN_ROOM * c.rho * ks * ka * kv;
+  T dv = tsqrt(tmax(dxr * dxr + dyr * dyr + dzr * dzr, dxl * dxl + dyl * dyl + dzl * dzl));
+  T kv = tclamp(T(2) - tdiv(dv, ISEN_SHEAR * tmax(c.cs, T(1e-30))), T(0), T(1));
+  // how far the blend may move the density, as an increment
+  const T room = (T(0.5) * ISEN_ROOM) * c.rho * ks * ka * kv;
+  k.bound = tmax((T(0.5) * ISEN_CAP) * tmin(tabs(c.rho - l.rho), tabs(r.rho - c.rho)), room);
   return k;
 }
 
-template <typename T, int LIM>
-__device__ __forceinline__ T isen_blend(const IsenCommon<T>& k, const EdgeScale<T>& srho, const Prim<T>& l,
-                                        const Prim<T>& c, const Prim<T>& r, T x, T bx, T sgn) {
-  const T ISEN_CAP = T(0.25);
-  if (!k.ok) return x + tclamp(T(0) - x, T(0), T(0));
-  T far = sgn > T(0) ? -k.tl : k.tr;
-  T near = sgn > T(0) ? k.tr : -k.tl;
-  T d = edge1<T, LIM>(far, near, srho);
-  T pf = c.p + T(0.5) * sgn * bx;
-  T wn = sgn > T(0) ? r.rho : l.rho;
-  T rf = tclamp((c.rho + T(0.5) * sgn * d) * tpow(tdiv(tmax(pf, T(1e-30)), c.p), k.gi), tmin(c.rho, wn),
-                tmax(c.rho, wn));
-  T bound = tmax(ISEN_CAP * tmin(tabs(c.rho - l.rho), tabs(r.rho - c.rho)), k.room);
-  T i0 = T(2) * sgn * (rf - c.rho);
-  return x + tclamp(i0 - x, -bound, bound);
+// x, bx: the increments of density and pressure toward the face; d: the limited increment of the
+// densities along the adiabat; wn: the density beyond the face
+template <typename T, bool UP>
+__device__ __forceinline__ T isen_blend(const IsenCommon<T>& k, const Prim<T>& c, T wn, T x, T bx, T d) {
+  const T sgn = UP ? T(1) : T(-1);
+  const T pf = c.p + sgn * bx;
+  const T rf = tclamp((c.rho + sgn * d) * tpow(tmax(pf, T(1e-30)) * k.ipc, k.gi), tmin(c.rho, wn), tmax(c.rho, wn));
+  const T i0 = sgn * (rf - c.rho);
+  return k.ok ? x + tclamp(i0 - x, -k.bound, k.bound) : x;
+}
+
+// What one axis's edges of a cell share: the differences to its two neighbours, Koren's scales,
+// the isentropic terms.
+template <typename T>
+struct EdgeTerms {
+  Inc<T> below, above;
+  T krho, kv, kp, k0;
+  IsenCommon<T> isen;
+};
+
+template <typename T, int LIM, bool ISEN>
+__device__ __forceinline__ EdgeTerms<T> edge_terms(const Params<T>& P, const Prim<T>& l, const Prim<T>& c,
+                                                   const Prim<T>& r) {
+  EdgeTerms<T> e{};
+  e.below = Inc<T>{c.rho - l.rho, c.vx - l.vx, c.vy - l.vy, c.vz - l.vz, c.p - l.p, c.s - l.s};
+  e.above = Inc<T>{r.rho - c.rho, r.vx - c.vx, r.vy - c.vy, r.vz - c.vz, r.p - c.p, r.s - c.s};
+  if constexpr (LIM == LIM_KOREN) {
+    e.krho = edge_scale(c.rho); e.kv = edge_scale(c.cs); e.kp = edge_scale(c.p); e.k0 = edge_scale(T(0));
+  }
+  if constexpr (ISEN) e.isen = isen_common(P, l, c, r);
+  return e;
 }
 
 // edge_up (UP) / edge_dn (hydro/q.wgsl:214-239), no potential.
 template <typename T, int LIM, bool ISEN, bool UP>
-__device__ __forceinline__ Inc<T> edge_k(const Params<T>& P, const Prim<T>& l, const Prim<T>& c, const Prim<T>& r,
-                                         const IsenCommon<T>& k) {
+__device__ __forceinline__ Inc<T> edge_of(const EdgeTerms<T>& e, const Prim<T>& l, const Prim<T>& c, const Prim<T>& r) {
   Inc<T> o;
-  constexpr bool fwd = UP || lim_symmetric<LIM>();
-  auto e = [&](T lo, T mid, T hi, const EdgeScale<T>& sc) {
-    T below = mid - lo, above = hi - mid;
-    return fwd ? edge1<T, LIM>(below, above, sc) : edge1<T, LIM>(above, below, sc);
-  };
-  EdgeScale<T> srho{}, sv{}, sp{}, s0{};
-  if constexpr (LIM == LIM_KOREN) {
-    srho = edge_scale(c.rho); sv = edge_scale(c.cs); sp = edge_scale(c.p); s0 = edge_scale(T(0));
+  o.rho = edge1<T, LIM, UP>(e.below.rho, e.above.rho, e.krho);
+  o.vx = edge1<T, LIM, UP>(e.below.vx, e.above.vx, e.kv);
+  o.vy = edge1<T, LIM, UP>(e.below.vy, e.above.vy, e.kv);
+  o.vz = edge1<T, LIM, UP>(e.below.vz, e.above.vz, e.kv);
+  o.p = edge1<T, LIM, UP>(e.below.p, e.above.p, e.kp);
+  o.s = edge1<T, LIM, UP>(e.below.s, e.above.s, e.k0);
+  if constexpr (ISEN) {
+    const T d = edge1<T, LIM, UP>(-e.isen.tl, e.isen.tr, e.krho);
+    o.rho = isen_blend<T, UP>(e.isen, c, UP ? r.rho : l.rho, o.rho, o.p, d);
   }
-  o.rho = e(l.rho, c.rho, r.rho, srho);
-  o.vx = e(l.vx, c.vx, r.vx, sv);
-  o.vy = e(l.vy, c.vy, r.vy, sv);
-  o.vz = e(l.vz, c.vz, r.vz, sv);
-  o.p = e(l.p, c.p, r.p, sp);
-  o.s = e(l.s, c.s, r.s, s0);
-  if constexpr (ISEN) o.rho = isen_blend<T, LIM>(k, srho, l, c, r, o.rho, o.p, UP ? T(1) : T(-1));
   return o;
 }
 template <typename T, int LIM, bool ISEN, bool UP>
 __device__ __forceinline__ Inc<T> edge(const Params<T>& P, const Prim<T>& l, const Prim<T>& c, const Prim<T>& r) {
-  IsenCommon<T> k{};
-  if constexpr (ISEN) k = isen_common(P, l, c, r);
-  return edge_k<T, LIM, ISEN, UP>(P, l, c, r, k);
+  return edge_of<T, LIM, ISEN, UP>(edge_terms<T, LIM, ISEN>(P, l, c, r), l, c, r);
 }
 
 // Half-step state (hydro/predictor.wgsl:46-209): rho, v, p, s at t + dt/2, the shock flag and
@@ -275,7 +294,9 @@ __device__ __forceinline__ Inc<T> edge(const Params<T>& P, const Prim<T>& l, con
 template <typename T>
 struct Half { T rho, vx, vy, vz, p, s, shock, fo; };
 
-// One axis's contribution to the predictor: the face-to-face slope and the positivity terms.
+// One axis's contribution to the predictor: the slope (the up increment of a symmetric limiter,
+// half of the face-to-face slope; the sum of Koren's two, all of it: slope_step takes the factor)
+// and the positivity terms.
 template <typename T>
 struct AxisSlope { Inc<T> s; T big; T fall; };
 
@@ -283,42 +304,55 @@ template <typename T, int LIM, bool ISEN>
 __device__ __forceinline__ AxisSlope<T> axis_slope(const Params<T>& P, const Prim<T>& m, const Prim<T>& q,
                                                    const Prim<T>& p, Inc<T>* up_out, Inc<T>* dn_out) {
   AxisSlope<T> r;
-  // a cell's up and down edges share the isentropic terms of its three cells
-  IsenCommon<T> k{};
-  if constexpr (ISEN) k = isen_common(P, m, q, p);
-  Inc<T> u = edge_k<T, LIM, ISEN, true>(P, m, q, p, k);
+  // a cell's up and down edges share their differences, Koren's weights and the isentropic terms
+  const EdgeTerms<T> e = edge_terms<T, LIM, ISEN>(P, m, q, p);
+  const Inc<T> u = edge_of<T, LIM, ISEN, true>(e, m, q, p);
   if constexpr (lim_symmetric<LIM>()) {
     r.s = u;
     r.big = tabs(u.p);
-    r.fall = T(-0.5) * tabs(u.rho);
+    r.fall = -tabs(u.rho);
     if (up_out) *up_out = u;
     if (dn_out) *dn_out = u;
   } else {
-    Inc<T> d = edge_k<T, LIM, ISEN, false>(P, m, q, p, k);
-    r.s.rho = T(0.5) * (u.rho + d.rho);
-    r.s.vx = T(0.5) * (u.vx + d.vx);
-    r.s.vy = T(0.5) * (u.vy + d.vy);
-    r.s.vz = T(0.5) * (u.vz + d.vz);
-    r.s.p = T(0.5) * (u.p + d.p);
-    r.s.s = T(0.5) * (u.s + d.s);
+    const Inc<T> d = edge_of<T, LIM, ISEN, false>(e, m, q, p);
+    r.s.rho = u.rho + d.rho;
+    r.s.vx = u.vx + d.vx;
+    r.s.vy = u.vy + d.vy;
+    r.s.vz = u.vz + d.vz;
+    r.s.p = u.p + d.p;
+    r.s.s = u.s + d.s;
     r.big = tmax(tabs(u.p), tabs(d.p));
-    r.fall = tmin(T(0.5) * u.rho, T(-0.5) * d.rho);
+    r.fall = tmin(u.rho, -d.rho);
     if (up_out) *up_out = u;
     if (dn_out) *dn_out = d;
   }
   return r;
 }
+// What the half step multiplies an axis's slope by: half a step's dt / dx for a whole slope
+template <typename T, int LIM>
+__device__ __forceinline__ T slope_step(const Params<T>& P, T dt) {
+  return lim_symmetric<LIM>() ? dt / P.dx : T(0.5) * dt / P.dx;
+}
 
-// The Hancock half step from the cell, its six neighbours' pressures and normal velocities
-// (for the shock detector) and the three axis slopes.
+// Shock detector (predictor.wgsl:114-134): converging flow and a relative pressure jump across
+// the cell above the threshold, |p+ - p-| / min(p+, p-) > thresh. jump_over is positive where
+// that holds along an axis (the product form: no reciprocal).
 template <typename T>
+__device__ __forceinline__ T jump_over(const Params<T>& P, T pm, T pp) {
+  return tabs(pp - pm) - P.shock_thresh * tmin(pp, pm);
+}
+
+// The Hancock half step from the cell, the three axis slopes, and for the shock detector the
+// convergence and the largest jump_over. gamma p is the rho c_s^2 of predictor.wgsl, without the
+// sound speed's root.
+template <typename T, int LIM>
 __device__ __forceinline__ Half<T> hancock(const Params<T>& P, const Prim<T>& q, const AxisSlope<T> sl[3],
                                            T conv, T jump, T dt) {
   Half<T> o;
-  T big = tmax(tmax(tmax(T(0), sl[0].big), sl[1].big), sl[2].big);
+  T big = tmax(tmax(sl[0].big, sl[1].big), sl[2].big);
   T fall = tmin(tmin(tmin(T(0), sl[0].fall), sl[1].fall), sl[2].fall);
-  T shock = (conv < T(0) && jump > P.shock_thresh) ? T(1) : T(0);
-  T h = T(0.5) * dt / P.dx;
+  T shock = (conv < T(0) && jump > T(0)) ? T(1) : T(0);
+  T h = slope_step<T, LIM>(P, dt);
   T rho = q.rho;
   const Inc<T>& sx = sl[0].s;
   const Inc<T>& sy = sl[1].s;
@@ -335,24 +369,17 @@ __device__ __forceinline__ Half<T> hancock(const Params<T>& P, const Prim<T>& q,
   o.vx = q.vx - h * (da1 + sx.p * ir);
   o.vy = q.vy - h * (da2 + sy.p * ir);
   o.vz = q.vz - h * (da3 + sz.p * ir);
-  o.p = q.p - h * (db0 + rho * q.cs * q.cs * dv);
+  o.p = q.p - h * (db0 + P.gamma * q.p * dv);
   o.s = q.s - h * db1;
   o.shock = shock;
   T rmin = o.rho + fall;
-  T pmin = o.p - T(0.5) * big;
+  T pmin = o.p - big;
   o.fo = T(0);
   if (!(rmin > T(0) && pmin > T(0))) {
     o.rho = q.rho; o.vx = q.vx; o.vy = q.vy; o.vz = q.vz; o.p = q.p; o.s = q.s;
     o.fo = T(1);
   }
   return o;
-}
-
-// Shock detector (predictor.wgsl:114-134): converging flow and the largest relative pressure
-// jump across the cell.
-template <typename T>
-__device__ __forceinline__ T jump_of(T pm, T pp) {
-  return tdiv(tabs(pp - pm), tmin(pp, pm));
 }
 
 // The half step of a cell of a flat grid (one layer along z) from its four neighbours: hancock
@@ -367,12 +394,12 @@ __device__ __forceinline__ Half<T> half_flat(const Params<T>& P, const Prim<T>& 
   const AxisSlope<T> ax = axis_slope<T, LIM, ISEN>(P, xm, q, xp, ixu, ixd);
   const AxisSlope<T> ay = axis_slope<T, LIM, ISEN>(P, ym, q, yp, iyu, iyd);
   const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy);
-  const T jump = tmax(jump_of(xm.p, xp.p), jump_of(ym.p, yp.p));
+  const T jump = tmax(jump_over(P, xm.p, xp.p), jump_over(P, ym.p, yp.p));
   Half<T> o;
-  T big = tmax(tmax(T(0), ax.big), ay.big);
+  T big = tmax(ax.big, ay.big);
   T fall = tmin(tmin(T(0), ax.fall), ay.fall);
-  T shock = (conv < T(0) && jump > P.shock_thresh) ? T(1) : T(0);
-  T h = T(0.5) * dt / P.dx;
+  T shock = (conv < T(0) && jump > T(0)) ? T(1) : T(0);
+  T h = slope_step<T, LIM>(P, dt);
   T rho = q.rho;
   const Inc<T>& sx = ax.s;
   const Inc<T>& sy = ay.s;
@@ -388,11 +415,11 @@ __device__ __forceinline__ Half<T> half_flat(const Params<T>& P, const Prim<T>& 
   o.vx = q.vx - h * (da1 + sx.p * ir);
   o.vy = q.vy - h * (da2 + sy.p * ir);
   o.vz = q.vz - h * da3;
-  o.p = q.p - h * (db0 + rho * q.cs * q.cs * dv);
+  o.p = q.p - h * (db0 + P.gamma * q.p * dv);
   o.s = q.s - h * db1;
   o.shock = shock;
   T rmin = o.rho + fall;
-  T pmin = o.p - T(0.5) * big;
+  T pmin = o.p - big;
   o.fo = T(0);
   if (!(rmin > T(0) && pmin > T(0))) {
     o.rho = q.rho; o.vx = q.vx; o.vy = q.vy; o.vz = q.vz; o.p = q.p; o.s = q.s;
@@ -406,9 +433,9 @@ template <typename T>
 struct Flux { T m, mx, my, mz, e, ei, s, vn; };
 
 // One side of a face (to_side, flux.wgsl:60-85) in the face frame: n normal, t1/t2 the
-// cyclically following components (rot, flux.wgsl:37-41).
+// cyclically following components (rot, flux.wgsl:37-41); pr = p / rho.
 template <typename T>
-struct Side { T rho, vn, vt1, vt2, p, s, cs, eint; };
+struct Side { T rho, vn, vt1, vt2, p, s, cs, pr; };
 
 template <typename T>
 __device__ __forceinline__ Side<T> make_side(const Params<T>& P, T rho, T vn, T vt1, T vt2, T p, T s, T lo_rho, T lo_p) {
@@ -417,108 +444,91 @@ __device__ __forceinline__ Side<T> make_side(const Params<T>& P, T rho, T vn, T 
   o.vn = vn; o.vt1 = vt1; o.vt2 = vt2;
   o.s = s;
   o.p = tmax(p, tmax(lo_p, P.p_floor));
-  o.cs = tsqrt(tdiv(P.gamma * o.p, o.rho));
-  o.eint = o.p * P.igm1;
+  o.pr = tdiv(o.p, o.rho);
+  o.cs = tsqrt(P.gamma * o.pr);
   return o;
 }
 
-// HLLC blended toward HLL by w (riemann/hllc.wgsl:4-85), or HLL (riemann/hll.wgsl:87-121).
-// A side's total energy, momentum and normal flux (hllc.wgsl:7-28), each from the side's own
-// primitives in one fixed expression
+// A side's total energy, momentum and normal flux (hllc.wgsl:7-28), for the HLL state
 template <typename T>
 struct SideFlux { T E, m0, m1, m2, f0, f1, f2, fe; };
 template <typename T>
-__device__ __forceinline__ SideFlux<T> side_flux(T rho, T vn, T vt1, T vt2, T p, T eint) {
+__device__ __forceinline__ SideFlux<T> side_flux(const Params<T>& P, const Side<T>& q) {
   SideFlux<T> o;
-  o.E = eint + T(0.5) * rho * (vn * vn + vt1 * vt1 + vt2 * vt2);
-  o.m0 = rho * vn; o.m1 = rho * vt1; o.m2 = rho * vt2;
-  o.f0 = o.m0 * vn + p; o.f1 = o.m1 * vn; o.f2 = o.m2 * vn;
-  o.fe = (o.E + p) * vn;
+  o.E = q.p * P.igm1 + T(0.5) * q.rho * (q.vn * q.vn + q.vt1 * q.vt1 + q.vt2 * q.vt2);
+  o.m0 = q.rho * q.vn; o.m1 = q.rho * q.vt1; o.m2 = q.rho * q.vt2;
+  o.f0 = o.m0 * q.vn + q.p; o.f1 = o.m1 * q.vn; o.f2 = o.m2 * q.vn;
+  o.fe = (o.E + q.p) * q.vn;
   return o;
 }
 
-// HLLC blended toward HLL by w (riemann/hllc.wgsl:4-85), or HLL (riemann/hll.wgsl:87-121).
-// Each branch forms only the side quantities it uses: the upwind side's on a supersonic face,
-// the star side's on a subsonic one, both where the HLL state is needed.
+// HLLC blended toward HLL by w (riemann/hllc.wgsl:4-85; w is a flag, 0 or 1), or HLL
+// (riemann/hll.wgsl:87-121).
+//
+// The supersonic and the two star states go through one set of expressions, so that a wave whose
+// faces differ in them does not run each in turn: the side K the face's fluxes come from, its
+// wave speed S, and u the normal velocity of the state at the face, which is the contact's speed
+// sm between the waves and K's own where K is supersonic (the star state is then K's state itself,
+// taken as it is). With d = S - u_K and 1/(S - u),
+//   rho* = rho d / (S - u),  p* = p + rho d (u - u_K),  E* = (E d - p u_K + p* u) / (S - u)
+// and the flux is (rho* u, rho* u^2 + p*, rho* u v_t, (E* + p*) u): the star flux of
+// hllc.wgsl:52-74 by the jump conditions, with one reciprocal where that form takes three. The
+// mass flux has the sign of u, which is also what K was picked by, so the internal energy and the
+// scalar it carries are K's.
 template <typename T, int RS>
-__device__ __forceinline__ Flux<T> riemann(const Side<T>& l, const Side<T>& r, T w_hll) {
-  T sl = tmin(l.vn - l.cs, r.vn - r.cs);
-  T sr = tmax(l.vn + l.cs, r.vn + r.cs);
+__device__ __forceinline__ Flux<T> riemann(const Params<T>& P, const Side<T>& l, const Side<T>& r, T w_hll) {
+  const T sl = tmin(l.vn - l.cs, r.vn - r.cs);
+  const T sr = tmax(l.vn + l.cs, r.vn + r.cs);
+  const T ql = l.rho * (sl - l.vn);
+  const T qr = r.rho * (sr - r.vn);
+  const T sm = tdiv(r.p - l.p + l.vn * ql - r.vn * qr, ql - qr);
+  const bool up_l = sl >= T(0), up_r = sr <= T(0), super = up_l || up_r;
+  const bool left = up_l || (!up_r && sm >= T(0));
+  const T S = left ? sl : sr;
+  const T rho = left ? l.rho : r.rho;
+  const T un = left ? l.vn : r.vn;
+  const T u1 = left ? l.vt1 : r.vt1;
+  const T u2 = left ? l.vt2 : r.vt2;
+  const T p = left ? l.p : r.p;
+  const T E = p * P.igm1 + T(0.5) * rho * (un * un + u1 * u1 + u2 * u2);
+  const T u = super ? un : sm;
+  const T d = S - un;
+  const T inv = trcp(S - u);
+  const T ps = p + (rho * d) * (u - un);
+  const T rs = super ? rho : rho * d * inv;
+  const T es = super ? E : (E * d - p * un + ps * u) * inv;
   Flux<T> o;
-  if (sl >= T(0) || sr <= T(0)) {
-    // supersonic: the upwind side's own flux
-    const bool up_l = sl >= T(0);
-    const SideFlux<T> u = side_flux(up_l ? l.rho : r.rho, up_l ? l.vn : r.vn, up_l ? l.vt1 : r.vt1,
-                                    up_l ? l.vt2 : r.vt2, up_l ? l.p : r.p, up_l ? l.eint : r.eint);
-    o.m = u.m0; o.mx = u.f0; o.my = u.f1; o.mz = u.f2; o.e = u.fe; o.vn = up_l ? l.vn : r.vn;
-  } else {
-    T ql = l.rho * (sl - l.vn);
-    T qr = r.rho * (sr - r.vn);
-    const bool star = RS != RS_HLL && ql < T(0) && qr > T(0);
-    // The HLL state between the waves: the flux itself where the star densities are not
-    // positive (and for HLL), the blend's other end where the face is flagged; a subsonic
-    // unflagged face (w = 0: the blend is the star flux exactly) skips it.
-    T hm, hp0, hp1, hp2, he;
-    if (!star || w_hll != T(0)) {
-      const SideFlux<T> a = side_flux(l.rho, l.vn, l.vt1, l.vt2, l.p, l.eint);
-      const SideFlux<T> b = side_flux(r.rho, r.vn, r.vt1, r.vt2, r.p, r.eint);
-      T inv = trcp(sr - sl);
-      T slsr = sl * sr;
-      hm = (sr * a.m0 - sl * b.m0 + slsr * (r.rho - l.rho)) * inv;
-      hp0 = (sr * a.f0 - sl * b.f0 + slsr * (b.m0 - a.m0)) * inv;
-      hp1 = (sr * a.f1 - sl * b.f1 + slsr * (b.m1 - a.m1)) * inv;
-      hp2 = (sr * a.f2 - sl * b.f2 + slsr * (b.m2 - a.m2)) * inv;
-      he = (sr * a.fe - sl * b.fe + slsr * (b.E - a.E)) * inv;
-    }
-    if constexpr (RS == RS_HLL) {
-      o.m = hm; o.mx = hp0; o.my = hp1; o.mz = hp2; o.e = he;
-      o.vn = tdiv(r.p - l.p + l.vn * ql - r.vn * qr, ql - qr);
-    } else {
-      if (!star) {
-        o.m = hm; o.mx = hp0; o.my = hp1; o.mz = hp2; o.e = he;
-        o.vn = T(0.5) * (l.vn + r.vn);
-      } else {
-        T sm = tdiv(r.p - l.p + l.vn * ql - r.vn * qr, ql - qr);
-        // the star state as differences from the outer state (hllc.wgsl:52-74)
-        bool left = sm >= T(0);
-        T S = left ? sl : sr;
-        T rho = left ? l.rho : r.rho;
-        T un = left ? l.vn : r.vn;
-        T u1 = left ? l.vt1 : r.vt1;
-        T u2 = left ? l.vt2 : r.vt2;
-        T p = left ? l.p : r.p;
-        T q = left ? ql : qr;
-        const SideFlux<T> c = side_flux(rho, un, u1, u2, p, left ? l.eint : r.eint);
-        T k = tdiv(sm - un, S - sm);
-        T dr = rho * k;
-        T f = rho + dr;
-        T cm = c.m0 + S * dr;
-        T c0 = c.f0 + S * (sm * dr + rho * (sm - un));
-        T c1 = c.f1 + S * (dr * u1);
-        T c2 = c.f2 + S * (dr * u2);
-        T ce = c.fe + S * (c.E * k + f * (sm - un) * (sm + tdiv(p, q)));
-        if (w_hll != T(0)) {
-          o.m = tmix(cm, hm, w_hll);
-          o.mx = tmix(c0, hp0, w_hll);
-          o.my = tmix(c1, hp1, w_hll);
-          o.mz = tmix(c2, hp2, w_hll);
-          o.e = tmix(ce, he, w_hll);
-        } else {
-          o.m = cm; o.mx = c0; o.my = c1; o.mz = c2; o.e = ce;
-        }
-        o.vn = sm;
-      }
-    }
+  o.m = rs * u;
+  o.mx = o.m * u + ps;
+  o.my = o.m * u1;
+  o.mz = o.m * u2;
+  o.e = (es + ps) * u;
+  o.ei = o.m * ((left ? l.pr : r.pr) * P.igm1);
+  o.s = o.m * (left ? l.s : r.s);
+  o.vn = u;
+  // The HLL state between the waves: the flux itself where the star densities are not positive
+  // (and for HLL) and where the face is flagged.
+  const bool star = ql < T(0) && qr > T(0);
+  if (!super && (RS == RS_HLL || !star || w_hll != T(0))) {
+    const SideFlux<T> a = side_flux(P, l);
+    const SideFlux<T> b = side_flux(P, r);
+    const T ih = trcp(sr - sl);
+    const T slsr = sl * sr;
+    o.m = (sr * a.m0 - sl * b.m0 + slsr * (r.rho - l.rho)) * ih;
+    o.mx = (sr * a.f0 - sl * b.f0 + slsr * (b.m0 - a.m0)) * ih;
+    o.my = (sr * a.f1 - sl * b.f1 + slsr * (b.m1 - a.m1)) * ih;
+    o.mz = (sr * a.f2 - sl * b.f2 + slsr * (b.m2 - a.m2)) * ih;
+    o.e = (sr * a.fe - sl * b.fe + slsr * (b.E - a.E)) * ih;
+    if (RS != RS_HLL && !star) o.vn = T(0.5) * (l.vn + r.vn);
+    const bool up = o.m >= T(0);
+    o.ei = o.m * ((up ? l.pr : r.pr) * P.igm1);
+    o.s = o.m * (up ? l.s : r.s);
   }
-  // internal energy and the scalar ride on the mass flux, upwinded
-  bool up = o.m >= T(0);
-  o.ei = o.m * tdiv(up ? l.eint : r.eint, up ? l.rho : r.rho);
-  o.s = o.m * (up ? l.s : r.s);
   return o;
 }
 
 // One cell's side of a face before the face's own lower bound and floors: the half-step state
-// plus half the edge increment toward the face (to_side, flux.wgsl:60-63; zero increment for a
+// plus the edge increment toward the face (to_side, flux.wgsl:60-63; zero increment for a
 // first-order cell), with the cell's half-step density and pressure (for the face's lower bound,
 // flux.wgsl:109-117) and its shock flag (flux.wgsl:93).
 template <typename T>
@@ -527,7 +537,7 @@ struct SideData { T rho, vx, vy, vz, p, s, hrho, hp, shock; };
 // sgn = +1 for the cell's upper face (il its up increment), -1 for its lower face.
 template <typename T>
 __device__ __forceinline__ SideData<T> side_of(const Half<T>& h, const Inc<T>& inc, T sgn) {
-  T hs = T(0.5) * sgn * (T(1) - h.fo);
+  T hs = sgn * (T(1) - h.fo);
   SideData<T> o;
   o.rho = h.rho + hs * inc.rho;
   o.vx = h.vx + hs * inc.vx;
@@ -556,7 +566,7 @@ __device__ __forceinline__ Flux<T> face_from_sides(const Params<T>& P, const Sid
   else { ln = L.vz; l1 = L.vx; l2 = L.vy; rn = R.vz; r1 = R.vx; r2 = R.vy; }
   Side<T> sl = make_side(P, L.rho, ln, l1, l2, L.p, L.s, lo_rho, lo_p);
   Side<T> sr = make_side(P, R.rho, rn, r1, r2, R.p, R.s, lo_rho, lo_p);
-  Flux<T> F = riemann<T, RS>(sl, sr, w);
+  Flux<T> F = riemann<T, RS>(P, sl, sr, w);
   // unrot: the face frame's (n, t1, t2) back to grid components
   T n = F.mx, t1 = F.my, t2 = F.mz;
   if (axis == 0) { F.mx = n; F.my = t1; F.mz = t2; }
@@ -584,7 +594,7 @@ __device__ __forceinline__ Flux<T> face_from_sides_rt(const Params<T>& P, SideDa
   return F;
 }
 
-// face_flux between the half-step states hl (left) and hr (right), given twice the increments
+// face_flux between the half-step states hl (left) and hr (right), given the increments
 // from each cell toward the face (il: the left cell's up increment, ir: the right cell's down
 // increment), along a run-time axis.
 template <typename T, int RS>
@@ -649,8 +659,7 @@ __device__ __forceinline__ Flux<T> net_of(const Flux<T>& xl, const Flux<T>& xh, 
 // The signal rate of a cell (hydro/rates.wgsl:60-62).
 template <typename T>
 __device__ __forceinline__ T rate_of(const Params<T>& P, const Prim<T>& w) {
-  T signal = tsqrt(w.cs * w.cs);
-  return tabs(w.vx) + tabs(w.vy) + tabs(w.vz) + P.ndim * signal;
+  return tabs(w.vx) + tabs(w.vy) + tabs(w.vz) + P.ndim * w.cs;
 }
 
 // Non-negative floats order as their bit patterns: the reductions compare those.

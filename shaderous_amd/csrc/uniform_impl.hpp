@@ -206,8 +206,8 @@ __device__ __forceinline__ void predict_cell(const Params<T>& P, const T4<T>* __
   sl[1] = axis_slope<T, LIM, ISEN>(P, ym, q, yp, nullptr, nullptr);
   sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
   T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
-  T jump = tmax(jump_of(xm.p, xp.p), tmax(jump_of(ym.p, yp.p), jump_of(zm.p, zp.p)));
-  Half<T> h = hancock(P, q, sl, conv, jump, dt);
+  T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
+  Half<T> h = hancock<T, LIM>(P, q, sl, conv, jump, dt);
   a.x = h.rho; a.y = h.vx; a.z = h.vy; a.w = h.vz;
   b.x = h.p; b.y = h.s; b.z = h.shock; b.w = h.fo;
 }
@@ -543,8 +543,8 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
       Half<T> hc;
       if (!MAPBC || !mapped) {
         T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (pp.vz - pm.vz);
-        T jump = tmax(jump_of(xm.p, xp.p), tmax(jump_of(ym.p, yp.p), jump_of(pm.p, pp.p)));
-        hc = hancock(P, pc, sl, conv, jump, dt);
+        T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, pm.p, pp.p)));
+        hc = hancock<T, LIM>(P, pc, sl, conv, jump, dt);
       } else {
         // the mapped cell's own stencil: its centre and z neighbours are this column's
         // primitives seen unflipped; its x/y neighbours are in LDS
@@ -559,8 +559,8 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
         ms[1] = axis_slope<T, LIM, ISEN>(P, sym, qc, syp, nullptr, nullptr);
         ms[2] = axis_slope<T, LIM, ISEN>(P, qm, qc, qp, nullptr, nullptr);
         T conv = (sxp.vx - sxm.vx) + (syp.vy - sym.vy) + (qp.vz - qm.vz);
-        T jump = tmax(jump_of(sxm.p, sxp.p), tmax(jump_of(sym.p, syp.p), jump_of(qm.p, qp.p)));
-        hc = hancock(P, qc, ms, conv, jump, dt);
+        T jump = tmax(jump_over(P, sxm.p, sxp.p), tmax(jump_over(P, sym.p, syp.p), jump_over(P, qm.p, qp.p)));
+        hc = hancock<T, LIM>(P, qc, ms, conv, jump, dt);
         hc.vx = bc_vel(hc.vx, mx.flip, mx.side);
         hc.vy = bc_vel(hc.vy, my.flip, my.side);
       }

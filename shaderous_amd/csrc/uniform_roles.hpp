@@ -211,8 +211,8 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::NTH), (RoleTile<TX, TY>::MINW)) 
       Half<T> hc;
       if (!MAPBC || !mapped) {
         T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (pp.vz - pm.vz);
-        T jump = tmax(jump_of(xm.p, xp.p), tmax(jump_of(ym.p, yp.p), jump_of(pm.p, pp.p)));
-        hc = hancock(P, pc, sl, conv, jump, dt);
+        T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, pm.p, pp.p)));
+        hc = hancock<T, LIM>(P, pc, sl, conv, jump, dt);
       } else {
         Prim<T> qc = pc, qm = pm, qp = pp;
         qc.vx = bc_vel(qc.vx, mx.flip, 0); qc.vy = bc_vel(qc.vy, my.flip, 0);
@@ -225,8 +225,8 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::NTH), (RoleTile<TX, TY>::MINW)) 
         ms[1] = axis_slope<T, LIM, ISEN>(P, sym, qc, syp, nullptr, nullptr);
         ms[2] = axis_slope<T, LIM, ISEN>(P, qm, qc, qp, nullptr, nullptr);
         T conv = (sxp.vx - sxm.vx) + (syp.vy - sym.vy) + (qp.vz - qm.vz);
-        T jump = tmax(jump_of(sxm.p, sxp.p), tmax(jump_of(sym.p, syp.p), jump_of(qm.p, qp.p)));
-        hc = hancock(P, qc, ms, conv, jump, dt);
+        T jump = tmax(jump_over(P, sxm.p, sxp.p), tmax(jump_over(P, sym.p, syp.p), jump_over(P, qm.p, qp.p)));
+        hc = hancock<T, LIM>(P, qc, ms, conv, jump, dt);
         hc.vx = bc_vel(hc.vx, mx.flip, mx.side);
         hc.vy = bc_vel(hc.vy, my.flip, my.side);
       }
