@@ -93,7 +93,7 @@ __device__ __forceinline__ Half<T> half_at_source(const Params<T>& P, const int*
   sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
   const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
   const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
-  return hancock<T, LIM>(P, q, sl, conv, jump, dt);
+  return hancock<T, LIM>(P, q, sl, conv, jump, slope_step<T, LIM>(P, dt));
 }
 
 // Flux register: per coarse-fine face of a leaf, its 16 x 16 faces' fluxes (8 values each), in
@@ -373,7 +373,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     // this block's cell size (P is the kernel's own copy: its dx is the block's from here on)
     const T dx = dx0 * (T(1) / T(1 << bt(tab, s, BT_LEVEL)));
     P.dx = dx;
-    const T dtdx = dt / dx;
+    const T dtdx = wave_uniform(dt / dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
     const bool cells = cells0 && act_blk, ghosts = ghosts0 && act_blk;
     // beside a coarser block (-1): its ghosts are predicted in place; elsewhere they are another
     // block's cells, whose half steps come from the shell
@@ -422,6 +422,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     __syncthreads();
 
     SideData<T> zs_prev;
+    T hp_prev = T(0);
     Flux<T> fz_lo = zero_flux<T>();
     Flux<T> axy_prev = zero_flux<T>();
 
@@ -436,6 +437,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
       //    (c = -1, 16) in the cell waves; the face ghosts of the cell planes in the ghost wave
       const bool oz = c < 0 || c >= AMR_BS;
       SideData<T> sxl, syl, szl, szu;
+      T hp = T(0);
       if (cells || (ghosts && !oz)) {
         Prim<T> pc = lds_prim<T, NT>(Lq, t);
         pc.cs = cs_c;
@@ -464,7 +466,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
           }
           const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (pp.vz - pm.vz);
           const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, pm.p, pp.p)));
-          hc = hancock<T, LIM>(P, pc, sl, conv, jump, dt);
+          hc = hancock<T, LIM>(P, pc, sl, conv, jump, hstep);
         } else {
           // another block's cell (same level, refined, or this block's boundary image): its half
           // step was formed in the shell pass
@@ -473,12 +475,13 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
           hc.rho = a.x; hc.vx = a.y; hc.vy = a.z; hc.vz = a.w;
           hc.p = b.x; hc.s = b.y; hc.shock = b.z; hc.fo = b.w;
         }
-        sxl = side_of(hc, ixd, T(-1));
-        syl = side_of(hc, iyd, T(-1));
-        szl = side_of(hc, izd, T(-1));
-        szu = side_of(hc, izu, T(1));
-        lds_put_side<T, NT>(L, LY::SX, t, side_of(hc, ixu, T(1)));
-        lds_put_side<T, NT>(L, LY::SY, t, side_of(hc, iyu, T(1)));
+        hp = hc.p;
+        sxl = side_of(P, hc, ixd, T(-1));
+        syl = side_of(P, hc, iyd, T(-1));
+        szl = side_of(P, hc, izd, T(-1));
+        szu = side_of(P, hc, izu, T(1));
+        lds_put_side<T, NT>(L, LY::SX, t, side_of(P, hc, ixu, T(1)));
+        lds_put_side<T, NT>(L, LY::SY, t, side_of(P, hc, iyu, T(1)));
       }
       // plane c + 1 into the slot plane c - 1 leaves
       lds_put_prim6<T, NT>(Lm, t, pp);
@@ -536,13 +539,14 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
           net.s = axy_prev.s + (fz_lo.s - fz.s);
           net.vn = axy_prev.vn + (fz_lo.vn - fz.vn);
           T4<T> o1, o2;
-          advance(P, U1[o], U2[o], net, zs_prev.hp, dtdx, o1, o2);
+          advance(P, U1[o], U2[o], net, hp_prev, dtdx, o1, o2);
           O1[o] = o1;
           O2[o] = o2;
           // the next step's rate / dx (assemble's leaf-cell rate, amr/assemble.wgsl:77-154)
           rate_max = tmax(rate_max, rate_of(P, prim_from_cons(P, o1, o2)) / dx);
         }
         zs_prev = szu;
+        hp_prev = hp;
         fz_lo = fz;
         axy_prev = axy;
       }

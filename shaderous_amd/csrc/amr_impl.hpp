@@ -503,7 +503,7 @@ __device__ __forceinline__ Half<T> predict_texel(const Params<T>& P, const T4<T>
   }
   const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
   const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
-  return hancock<T, LIM>(P, q, sl, conv, jump, dt);
+  return hancock<T, LIM>(P, q, sl, conv, jump, slope_step<T, LIM>(P, dt));
 }
 
 template <typename T, int LIM, bool ISEN, int D = 3>

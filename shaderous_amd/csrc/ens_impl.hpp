@@ -81,7 +81,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 2 : 1)) void k_ens_fused(
     const long long off = SINGLE ? 0ll : inst[w.inst].off;
     const int nx = P.n[0], ny = P.n[1];
     const T dt = step_dt(P, C, w.inst);
-    const T dtdx = dt / P.dx;
+    const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
     const int x = w.x0 + tx - 2, y = w.y0 + ty - 2;
     const AxisMap mx = map_axis(x, nx, P.bc_lo[0], P.bc_hi[0]);
     const AxisMap my = map_axis(y, ny, P.bc_lo[1], P.bc_hi[1]);
@@ -114,7 +114,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 2 : 1)) void k_ens_fused(
       const Prim<T> xm = lds_prim<T, NT>(L + LY::Q, t - 1), xp = lds_prim<T, NT>(L + LY::Q, t + 1);
       const Prim<T> ym = lds_prim<T, NT>(L + LY::Q, t - BX), yp = lds_prim<T, NT>(L + LY::Q, t + BX);
       Inc<T> ixu, ixd, iyu, iyd;
-      Half<T> hc = half_flat<T, LIM, ISEN>(P, pc, xm, xp, ym, yp, dt, &ixu, &ixd, &iyu, &iyd);
+      Half<T> hc = half_flat<T, LIM, ISEN>(P, pc, xm, xp, ym, yp, hstep, &ixu, &ixd, &iyu, &iyd);
       if (mapped) {
         // the mapped cell's own stencil: its centre is this column's primitives seen unflipped
         Prim<T> qc = pc;
@@ -122,15 +122,15 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 2 : 1)) void k_ens_fused(
         qc.vy = bc_vel(qc.vy, my.flip, 0);
         const Prim<T> sxm = lds_prim<T, NT>(L + LY::Q, ts - 1), sxp = lds_prim<T, NT>(L + LY::Q, ts + 1);
         const Prim<T> sym = lds_prim<T, NT>(L + LY::Q, ts - BX), syp = lds_prim<T, NT>(L + LY::Q, ts + BX);
-        hc = half_flat<T, LIM, ISEN>(P, qc, sxm, sxp, sym, syp, dt, nullptr, nullptr, nullptr, nullptr);
+        hc = half_flat<T, LIM, ISEN>(P, qc, sxm, sxp, sym, syp, hstep, nullptr, nullptr, nullptr, nullptr);
         hc.vx = bc_vel(hc.vx, mx.flip, mx.side);
         hc.vy = bc_vel(hc.vy, my.flip, my.side);
       }
       hp = hc.p;
-      sxl = side_of(hc, ixd, T(-1));
-      syl = side_of(hc, iyd, T(-1));
-      lds_put_side<T, NT>(L, LY::SX, t, side_of(hc, ixu, T(1)));
-      lds_put_side<T, NT>(L, LY::SY, t, side_of(hc, iyu, T(1)));
+      sxl = side_of(P, hc, ixd, T(-1));
+      syl = side_of(P, hc, iyd, T(-1));
+      lds_put_side<T, NT>(L, LY::SX, t, side_of(P, hc, ixu, T(1)));
+      lds_put_side<T, NT>(L, LY::SY, t, side_of(P, hc, iyu, T(1)));
     }
     __syncthreads();
 
@@ -229,7 +229,7 @@ __global__ __launch_bounds__(64) void k_ens_rows(const EnsInst<float>* __restric
   const long long off = inst[w.inst].off;
   const int nx = P.n[0], ny = P.n[1];
   const T dt = step_dt(P, C, w.inst);
-  const T dtdx = dt / P.dx;
+  const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
   const int lane = threadIdx.x;
   if (blockIdx.x == 0)
     for (int i = lane; i < ninst; i += 64) step_clock_advance(inst[i].P, C, i);
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(64) void k_ens_rows(const EnsInst<float>* __restric
     const Prim<T> pp = row(c + 1);
     const Prim<T> xm = prim_beside<true>(pc), xp = prim_beside<false>(pc);
     Inc<T> ixu, ixd, iyu, iyd;
-    Half<T> hc = half_flat<T, LIM, ISEN>(P, pc, xm, xp, pm, pp, dt, &ixu, &ixd, &iyu, &iyd);
+    Half<T> hc = half_flat<T, LIM, ISEN>(P, pc, xm, xp, pm, pp, hstep, &ixu, &ixd, &iyu, &iyd);
     // a ghost row above: the last row's half step
     const bool ghost_hi = ymap_hi && c == ny;
     if (ghost_hi) {
@@ -283,11 +283,11 @@ __global__ __launch_bounds__(64) void k_ens_rows(const EnsInst<float>* __restric
         hc.vx = bc_vel(hc.vx, mx.flip, mx.side);
       }
     }
-    const SideData<T> sxl = side_of(hc, ixd, T(-1));
-    const SideData<T> syl = side_of(hc, iyd, T(-1));
-    const SideData<T> syu = side_of(hc, iyu, T(1));
+    const SideData<T> sxl = side_of(P, hc, ixd, T(-1));
+    const SideData<T> syl = side_of(P, hc, iyd, T(-1));
+    const SideData<T> syu = side_of(P, hc, iyu, T(1));
     // the x face on this lane's left (every lane, for the shifts)
-    const Flux<T> Fx = face_from_sides<T, RS>(P, side_from_left(side_of(hc, ixu, T(1))), sxl, 0);
+    const Flux<T> Fx = face_from_sides<T, RS>(P, side_from_left(side_of(P, hc, ixu, T(1))), sxl, 0);
     const Flux<T> xh = flux_from_right(Fx);
     Flux<T> axy;
     axy.m = Fx.m - xh.m; axy.mx = Fx.mx - xh.mx; axy.my = Fx.my - xh.my; axy.mz = Fx.mz - xh.mz;
@@ -303,7 +303,7 @@ __global__ __launch_bounds__(64) void k_ens_rows(const EnsInst<float>* __restric
           const AxisMap my = map_axis(-1, ny, P.bc_lo[1], P.bc_hi[1]);
           Half<T> hg = hc;
           hg.vy = bc_vel(hg.vy, my.flip, my.side);
-          lo = side_of(hg, iyu_ghost, T(1));
+          lo = side_of(P, hg, iyu_ghost, T(1));
         }
         fy = face_from_sides<T, RS>(P, lo, syl, 1);
       }

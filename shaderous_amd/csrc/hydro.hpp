@@ -52,8 +52,29 @@ __device__ __forceinline__ float tmax(float a, float b) { return __builtin_fmaxf
 __device__ __forceinline__ double tmax(double a, double b) { return __builtin_fmax(a, b); }
 __device__ __forceinline__ float tabs(float a) { return __builtin_fabsf(a); }
 __device__ __forceinline__ double tabs(double a) { return __builtin_fabs(a); }
+// The same for operands that come from memory or LDS, where the compiler would first quiet each
+// one (v_max x, x) in case it is a signaling NaN: arithmetic makes none, and states are checked
+// finite when they are set
+__device__ __forceinline__ float raw_min(float a, float b) {
+  float r;
+  asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double raw_min(double a, double b) { return tmin(a, b); }
+__device__ __forceinline__ float raw_max(float a, float b) {
+  float r;
+  asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ double raw_max(double a, double b) { return tmax(a, b); }
 template <typename T> __device__ __forceinline__ T tsign(T a) { return a > T(0) ? T(1) : (a < T(0) ? T(-1) : T(0)); }
-template <typename T> __device__ __forceinline__ T tclamp(T x, T lo, T hi) { return tmin(tmax(x, lo), hi); }
+// x held to [lo, hi] (lo <= hi; a NaN x gives lo): in FP32 the median, one instruction, and between
+// the constants 0 and 1 the output modifier of the instruction that forms x
+__device__ __forceinline__ float tclamp(float x, float lo, float hi) { return __builtin_amdgcn_fmed3f(x, lo, hi); }
+__device__ __forceinline__ double tclamp(double x, double lo, double hi) { return tmin(tmax(x, lo), hi); }
+// x held between a and b, whichever is the smaller
+__device__ __forceinline__ float tbetween(float x, float a, float b) { return __builtin_amdgcn_fmed3f(x, a, b); }
+__device__ __forceinline__ double tbetween(double x, double a, double b) { return tclamp(x, tmin(a, b), tmax(a, b)); }
 // Single precision: the hardware reciprocal and square root (v_rcp_f32, v_sqrt_f32, ~1 ulp;
 // WGSL allows 2.5 ulp for division). Double precision: correctly rounded.
 __device__ __forceinline__ float trcp(float b) { return __builtin_amdgcn_rcpf(b); }
@@ -66,7 +87,11 @@ __device__ __forceinline__ double tsqrt(double x) { return __builtin_sqrt(x); }
 // hardware's log2 and exp2 (v_log_f32, v_exp_f32): the library powf's exact-case handling costs
 // ~40 instructions a call, and the isentropic reconstruction makes six calls per axis.
 __device__ __forceinline__ float tpow(float a, float b) { return __builtin_amdgcn_exp2f(b * __builtin_amdgcn_logf(a)); }
-__device__ __forceinline__ double tpow(double a, double b) { return pow(a, b); }
+// Double precision: the library's, as a call. Inlined at each of the twelve uses of a plane (and in
+// every role's loop) it made kernels of up to 347 KB, several times the instruction cache; one
+// that large (isentropic reconstruction beside reflecting faces) also came out of the compiler
+// wrong. Turbulence 96^3 in FP64, Koren + isentropic: 0.78 -> 0.50 ms per step.
+__device__ __attribute__((noinline)) inline double tpow(double a, double b) { return pow(a, b); }
 // WGSL mix(x, y, a) = x (1 - a) + y a
 template <typename T> __device__ __forceinline__ T tmix(T x, T y, T a) { return x * (T(1) - a) + y * a; }
 // sign(a) * sign(b) > 0, formed from the signs so that small products do not underflow
@@ -92,7 +117,7 @@ struct Prim {
 template <typename T>
 __device__ __forceinline__ Prim<T> prim_from_cons(const Params<T>& P, T4<T> u1, T4<T> u2) {
   Prim<T> q;
-  T rho = tmax(u1.x, P.rho_floor);
+  T rho = raw_max(u1.x, P.rho_floor);
   T p = P.gm1 * u2.y;
   if (!(p >= P.p_floor)) p = P.p_floor;
   T ir = trcp(rho);
@@ -162,17 +187,17 @@ __device__ __forceinline__ T edge_scale(T scale) {
 template <typename T>
 __device__ __forceinline__ T koren_weight(T below, T above, T k) {
   const T b = below * k, a = above * k;
-  return tclamp(T(1.5) - (b * b + a * a), T(0), T(1));
+  const T e = T(1.5) - b * b;
+  return tclamp(e - a * a, T(0), T(1));
 }
-// Koren's increment toward the face `near` lies on, blended by w from the limited value to the
+// Koren's increment toward the face `near` lies on (least: the minmod of the two), blended by w from the limited value to the
 // plain one (w = 1 gives the plain one exactly: the limited value is no larger). The early return
 // of koren.wgsl gives the blend's value per channel, so each channel is formed on its own.
 template <typename T>
-__device__ __forceinline__ T koren_edge(T far, T near, T w) {
+__device__ __forceinline__ T koren_edge(T far, T near, T least, T w) {
   const T fr = (far + T(2) * near) * T(1.0 / 6.0);
   // sign(near) min(|far|, |near|, |fr|) where far and near share a sign (fr then does too)
-  const T lim = minmod(far, minmod(near, fr));
-  return tmix(lim, fr, w);
+  return tmix(minmod(least, fr), fr, w);
 }
 // The symmetric limiters' increment from the two differences, the same toward both faces
 template <typename T, int LIM>
@@ -194,7 +219,8 @@ template <typename T, int LIM, bool UP>
 __device__ __forceinline__ T edge1(T below, T above, T k) {
   if constexpr (LIM == LIM_KOREN) {
     const T w = koren_weight(below, above, k);
-    return UP ? koren_edge(below, above, w) : koren_edge(above, below, w);
+    const T least = minmod(below, above);
+    return UP ? koren_edge(below, above, least, w) : koren_edge(above, below, least, w);
   } else {
     return sym_edge<T, LIM>(below, above);
   }
@@ -218,7 +244,7 @@ __device__ __forceinline__ IsenCommon<T> isen_common(const Params<T>& P, const P
   const T ISEN_SMOOTH = T(0.2), ISEN_ADIABAT = T(0.01), ISEN_SHEAR = T(0.1), ISEN_ROOM = T(0.01), ISEN_CAP = T(0.25);
   IsenCommon<T> k;
   // (the unassembled edge texels of a block are zeros)
-  k.ok = tmin(tmin(tmin(l.rho, l.p), tmin(c.rho, c.p)), tmin(r.rho, r.p)) > T(0);
+  k.ok = raw_min(raw_min(raw_min(l.rho, l.p), raw_min(c.rho, c.p)), raw_min(r.rho, r.p)) > T(0);
   k.gi = trcp(P.gamma);
   k.ipc = trcp(c.p);
   k.tl = l.rho * tpow(l.p * k.ipc, -k.gi) - c.rho;
@@ -241,7 +267,7 @@ template <typename T, bool UP>
 __device__ __forceinline__ T isen_blend(const IsenCommon<T>& k, const Prim<T>& c, T wn, T x, T bx, T d) {
   const T sgn = UP ? T(1) : T(-1);
   const T pf = c.p + sgn * bx;
-  const T rf = tclamp((c.rho + sgn * d) * tpow(tmax(pf, T(1e-30)) * k.ipc, k.gi), tmin(c.rho, wn), tmax(c.rho, wn));
+  const T rf = tbetween((c.rho + sgn * d) * tpow(tmax(pf, T(1e-30)) * k.ipc, k.gi), c.rho, wn);
   const T i0 = sgn * (rf - c.rho);
   return k.ok ? x + tclamp(i0 - x, -k.bound, k.bound) : x;
 }
@@ -339,20 +365,19 @@ __device__ __forceinline__ T slope_step(const Params<T>& P, T dt) {
 // that holds along an axis (the product form: no reciprocal).
 template <typename T>
 __device__ __forceinline__ T jump_over(const Params<T>& P, T pm, T pp) {
-  return tabs(pp - pm) - P.shock_thresh * tmin(pp, pm);
+  return tabs(pp - pm) - P.shock_thresh * raw_min(pp, pm);
 }
 
 // The Hancock half step from the cell, the three axis slopes, and for the shock detector the
-// convergence and the largest jump_over. gamma p is the rho c_s^2 of predictor.wgsl, without the
+// convergence and the largest jump_over; h: slope_step. gamma p is the rho c_s^2 of predictor.wgsl, without the
 // sound speed's root.
 template <typename T, int LIM>
 __device__ __forceinline__ Half<T> hancock(const Params<T>& P, const Prim<T>& q, const AxisSlope<T> sl[3],
-                                           T conv, T jump, T dt) {
+                                           T conv, T jump, T h) {
   Half<T> o;
   T big = tmax(tmax(sl[0].big, sl[1].big), sl[2].big);
   T fall = tmin(tmin(tmin(T(0), sl[0].fall), sl[1].fall), sl[2].fall);
   T shock = (conv < T(0) && jump > T(0)) ? T(1) : T(0);
-  T h = slope_step<T, LIM>(P, dt);
   T rho = q.rho;
   const Inc<T>& sx = sl[0].s;
   const Inc<T>& sy = sl[1].s;
@@ -389,7 +414,7 @@ __device__ __forceinline__ Half<T> hancock(const Params<T>& P, const Prim<T>& q,
 // increments.
 template <typename T, int LIM, bool ISEN>
 __device__ __forceinline__ Half<T> half_flat(const Params<T>& P, const Prim<T>& q, const Prim<T>& xm,
-                                             const Prim<T>& xp, const Prim<T>& ym, const Prim<T>& yp, T dt,
+                                             const Prim<T>& xp, const Prim<T>& ym, const Prim<T>& yp, T h,
                                              Inc<T>* ixu, Inc<T>* ixd, Inc<T>* iyu, Inc<T>* iyd) {
   const AxisSlope<T> ax = axis_slope<T, LIM, ISEN>(P, xm, q, xp, ixu, ixd);
   const AxisSlope<T> ay = axis_slope<T, LIM, ISEN>(P, ym, q, yp, iyu, iyd);
@@ -399,7 +424,6 @@ __device__ __forceinline__ Half<T> half_flat(const Params<T>& P, const Prim<T>& 
   T big = tmax(ax.big, ay.big);
   T fall = tmin(tmin(T(0), ax.fall), ay.fall);
   T shock = (conv < T(0) && jump > T(0)) ? T(1) : T(0);
-  T h = slope_step<T, LIM>(P, dt);
   T rho = q.rho;
   const Inc<T>& sx = ax.s;
   const Inc<T>& sy = ay.s;
@@ -433,17 +457,18 @@ template <typename T>
 struct Flux { T m, mx, my, mz, e, ei, s, vn; };
 
 // One side of a face (to_side, flux.wgsl:60-85) in the face frame: n normal, t1/t2 the
-// cyclically following components (rot, flux.wgsl:37-41); pr = p / rho.
+// cyclically following components (rot, flux.wgsl:37-41); pr = p / rho. lo_rho, lo_p: the face's
+// lower bounds, floors included.
 template <typename T>
 struct Side { T rho, vn, vt1, vt2, p, s, cs, pr; };
 
 template <typename T>
 __device__ __forceinline__ Side<T> make_side(const Params<T>& P, T rho, T vn, T vt1, T vt2, T p, T s, T lo_rho, T lo_p) {
   Side<T> o;
-  o.rho = tmax(rho, tmax(lo_rho, P.rho_floor));
+  o.rho = raw_max(rho, lo_rho);
   o.vn = vn; o.vt1 = vt1; o.vt2 = vt2;
   o.s = s;
-  o.p = tmax(p, tmax(lo_p, P.p_floor));
+  o.p = raw_max(p, lo_p);
   o.pr = tdiv(o.p, o.rho);
   o.cs = tsqrt(P.gamma * o.pr);
   return o;
@@ -462,8 +487,8 @@ __device__ __forceinline__ SideFlux<T> side_flux(const Params<T>& P, const Side<
   return o;
 }
 
-// HLLC blended toward HLL by w (riemann/hllc.wgsl:4-85; w is a flag, 0 or 1), or HLL
-// (riemann/hll.wgsl:87-121).
+// HLLC, taken to HLL where w is not zero (riemann/hllc.wgsl:4-85, whose blend weight is a flag), or
+// HLL (riemann/hll.wgsl:87-121).
 //
 // The supersonic and the two star states go through one set of expressions, so that a wave whose
 // faces differ in them does not run each in turn: the side K the face's fluxes come from, its
@@ -529,14 +554,14 @@ __device__ __forceinline__ Flux<T> riemann(const Params<T>& P, const Side<T>& l,
 
 // One cell's side of a face before the face's own lower bound and floors: the half-step state
 // plus the edge increment toward the face (to_side, flux.wgsl:60-63; zero increment for a
-// first-order cell), with the cell's half-step density and pressure (for the face's lower bound,
-// flux.wgsl:109-117) and its shock flag (flux.wgsl:93).
+// first-order cell), with the cell's share of the face's lower bounds, half its half-step density
+// and pressure and at least the floors (flux.wgsl:109-117), and its shock flag (flux.wgsl:93).
 template <typename T>
 struct SideData { T rho, vx, vy, vz, p, s, hrho, hp, shock; };
 
 // sgn = +1 for the cell's upper face (il its up increment), -1 for its lower face.
 template <typename T>
-__device__ __forceinline__ SideData<T> side_of(const Half<T>& h, const Inc<T>& inc, T sgn) {
+__device__ __forceinline__ SideData<T> side_of(const Params<T>& P, const Half<T>& h, const Inc<T>& inc, T sgn) {
   T hs = sgn * (T(1) - h.fo);
   SideData<T> o;
   o.rho = h.rho + hs * inc.rho;
@@ -545,8 +570,8 @@ __device__ __forceinline__ SideData<T> side_of(const Half<T>& h, const Inc<T>& i
   o.vz = h.vz + hs * inc.vz;
   o.p = h.p + hs * inc.p;
   o.s = h.s + hs * inc.s;
-  o.hrho = h.rho;
-  o.hp = h.p;
+  o.hrho = tmax(T(0.5) * h.rho, P.rho_floor);
+  o.hp = tmax(T(0.5) * h.p, P.p_floor);
   o.shock = h.shock;
   return o;
 }
@@ -556,9 +581,9 @@ __device__ __forceinline__ SideData<T> side_of(const Half<T>& h, const Inc<T>& i
 template <typename T, int RS>
 __device__ __forceinline__ Flux<T> face_from_sides(const Params<T>& P, const SideData<T>& L, const SideData<T>& R,
                                                    int axis) {
-  T w = tmax(L.shock, R.shock);
-  T lo_rho = T(0.5) * tmin(L.hrho, R.hrho);
-  T lo_p = T(0.5) * tmin(L.hp, R.hp);
+  T w = L.shock + R.shock;   // flags: zero where neither cell has one
+  T lo_rho = raw_min(L.hrho, R.hrho);
+  T lo_p = raw_min(L.hp, R.hp);
   // rot (flux.wgsl:37-41): axis 0 -> (x, y, z), 1 -> (y, z, x), 2 -> (z, x, y)
   T ln, l1, l2, rn, r1, r2;
   if (axis == 0) { ln = L.vx; l1 = L.vy; l2 = L.vz; rn = R.vx; r1 = R.vy; r2 = R.vz; }
@@ -600,7 +625,7 @@ __device__ __forceinline__ Flux<T> face_from_sides_rt(const Params<T>& P, SideDa
 template <typename T, int RS>
 __device__ __forceinline__ Flux<T> face_flux(const Params<T>& P, const Half<T>& hl, const Inc<T>& il,
                                              const Half<T>& hr, const Inc<T>& ir, int axis) {
-  return face_from_sides_rt<T, RS>(P, side_of(hl, il, T(1)), side_of(hr, ir, T(-1)), axis);
+  return face_from_sides_rt<T, RS>(P, side_of(P, hl, il, T(1)), side_of(P, hr, ir, T(-1)), axis);
 }
 
 // advance (hydro/advance.wgsl:31-52), dual_energy (hydro/dual_energy.wgsl:73-87) and the

@@ -194,8 +194,9 @@ __device__ __forceinline__ void predict_cell(const Params<T>& P, const T4<T>* __
   Prim<T> q = load_q(P, U1, U2, i, j, k);
   Prim<T> xm = load_q(P, U1, U2, i - 1, j, k), xp = load_q(P, U1, U2, i + 1, j, k);
   Prim<T> ym = load_q(P, U1, U2, i, j - 1, k), yp = load_q(P, U1, U2, i, j + 1, k);
+  const T hstep = slope_step<T, LIM>(P, dt);
   if (P.flat) {
-    const Half<T> h = half_flat<T, LIM, ISEN>(P, q, xm, xp, ym, yp, dt, nullptr, nullptr, nullptr, nullptr);
+    const Half<T> h = half_flat<T, LIM, ISEN>(P, q, xm, xp, ym, yp, hstep, nullptr, nullptr, nullptr, nullptr);
     a.x = h.rho; a.y = h.vx; a.z = h.vy; a.w = h.vz;
     b.x = h.p; b.y = h.s; b.z = h.shock; b.w = h.fo;
     return;
@@ -207,7 +208,7 @@ __device__ __forceinline__ void predict_cell(const Params<T>& P, const T4<T>* __
   sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
   T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
   T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
-  Half<T> h = hancock<T, LIM>(P, q, sl, conv, jump, dt);
+  Half<T> h = hancock<T, LIM>(P, q, sl, conv, jump, hstep);
   a.x = h.rho; a.y = h.vx; a.z = h.vy; a.w = h.vz;
   b.x = h.p; b.y = h.s; b.z = h.shock; b.w = h.fo;
 }
@@ -456,7 +457,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
   const int z0 = blockIdx.z * zc;
   const int z1 = min(z0 + zc, nz);
   const T dt = step_dt(P, C, 0);
-  const T dtdx = dt / P.dx;
+  const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
   if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && t == 0) step_clock_advance(P, C, 0);
 
   // this column's source through the x/y boundaries (clamped in range for the ragged rim,
@@ -509,6 +510,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
   b1 = U1[o0]; b2 = U2[o0];
 
   SideData<T> zs_prev;                 // the upper z side of plane c - 1
+  T hp_prev = T(0);                    // and its half-step pressure
   Flux<T> fz_lo = zero_flux<T>();      // the z face below plane c - 1
   Flux<T> axy_prev = zero_flux<T>();   // plane c - 1's (x_lo - x_hi) + (y_lo - y_hi)
   T rate_max = T(0);
@@ -530,6 +532,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
 
     // 2. half step and sides of plane c (hydro/predictor.wgsl:46-209)
     SideData<T> sxl, syl, szl, szu;
+    T hp = T(0);
     if (in_r1) {
       Prim<T> pc = lds_prim_c<T, NT>(Lq, t);
       Prim<T> pm = lds_prim<T, NT>(Lm, t);
@@ -544,7 +547,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
       if (!MAPBC || !mapped) {
         T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (pp.vz - pm.vz);
         T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, pm.p, pp.p)));
-        hc = hancock<T, LIM>(P, pc, sl, conv, jump, dt);
+        hc = hancock<T, LIM>(P, pc, sl, conv, jump, hstep);
       } else {
         // the mapped cell's own stencil: its centre and z neighbours are this column's
         // primitives seen unflipped; its x/y neighbours are in LDS
@@ -560,18 +563,19 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
         ms[2] = axis_slope<T, LIM, ISEN>(P, qm, qc, qp, nullptr, nullptr);
         T conv = (sxp.vx - sxm.vx) + (syp.vy - sym.vy) + (qp.vz - qm.vz);
         T jump = tmax(jump_over(P, sxm.p, sxp.p), tmax(jump_over(P, sym.p, syp.p), jump_over(P, qm.p, qp.p)));
-        hc = hancock<T, LIM>(P, qc, ms, conv, jump, dt);
+        hc = hancock<T, LIM>(P, qc, ms, conv, jump, hstep);
         hc.vx = bc_vel(hc.vx, mx.flip, mx.side);
         hc.vy = bc_vel(hc.vy, my.flip, my.side);
       }
       if (zbc && tile) zghost_half(P, ZA, ZB, c, (size_t)y * nx + x, hc);
-      sxl = side_of(hc, ixd, T(-1));
-      syl = side_of(hc, iyd, T(-1));
-      szl = side_of(hc, izd, T(-1));
-      szu = side_of(hc, izu, T(1));
+      hp = hc.p;
+      sxl = side_of(P, hc, ixd, T(-1));
+      syl = side_of(P, hc, iyd, T(-1));
+      szl = side_of(P, hc, izd, T(-1));
+      szu = side_of(P, hc, izu, T(1));
       // what the neighbours above need
-      lds_put_side<T, NT>(L, LY::SX, t, side_of(hc, ixu, T(1)));
-      lds_put_side<T, NT>(L, LY::SY, t, side_of(hc, iyu, T(1)));
+      lds_put_side<T, NT>(L, LY::SX, t, side_of(P, hc, ixu, T(1)));
+      lds_put_side<T, NT>(L, LY::SY, t, side_of(P, hc, iyu, T(1)));
     }
     // plane c + 1 into the slot plane c - 1 leaves (only this column reads its own c - 1 entry)
     lds_put_prim<T, NT>(Lm, t, pp);
@@ -623,7 +627,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
         net.ei = axy_prev.ei + (fz_lo.ei - fz.ei);
         net.s = axy_prev.s + (fz_lo.s - fz.s);
         net.vn = axy_prev.vn + (fz_lo.vn - fz.vn);
-        advance(P, U1[o], U2[o], net, zs_prev.hp, dtdx, o1, o2);
+        advance(P, U1[o], U2[o], net, hp_prev, dtdx, o1, o2);
         // the next step's signal rate (hydro/rates.wgsl:60-62), from the state just made
         Prim<T> w = prim_from_cons(P, o1, o2);
         rate_max = tmax(rate_max, rate_of(P, w));
@@ -633,6 +637,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
     }
     // rotate
     zs_prev = szu;
+    hp_prev = hp;
     fz_lo = fz;
     axy_prev = axy;
   }
@@ -717,7 +722,7 @@ struct UniformImpl {
     bool mapbc = za != nullptr;
     for (int a = 0; a < 2; a++) mapbc |= P.bc_lo[a] != BC_PERIODIC || P.bc_hi[a] != BC_PERIODIC;
 #define SHX_FUSED_R(D, M)                                                                                            \
-  hipLaunchKernelGGL((k_fused_r<T, LIM, RS, ISEN, TX, TY, D, M>), g, dim3(RoleTile<TX, TY>::NTH), 0, L.stream, P,     \
+  hipLaunchKernelGGL((k_fused_r<T, LIM, RS, ISEN, TX, TY, D, M>), g, dim3(RoleTile<TX, TY>::template launch<T>()), 0, L.stream, P,     \
                      (const T4<T>*)u1, (const T4<T>*)u2, (T4<T>*)o1, (T4<T>*)o2, step_clock<T>(ck), (const T4<T>*)za, \
                      (const T4<T>*)zb, zc)
     if (debug) { if (mapbc) SHX_FUSED_R(true, true); else SHX_FUSED_R(true, false); }
@@ -727,9 +732,14 @@ struct UniformImpl {
   // za, zb: the half steps of planes 0 and nz - 1 for a non-periodic z face (null: z periodic)
   static void fused(const Launch& L, int tile, const void* u1, const void* u2, void* o1, void* o2, const ClockRefs& ck,
                     const void* za, const void* zb, int zc, bool debug) {
+    // the role kernel addresses a plane with 32 bits: beyond 4 GiB a plane, the raster tiles
+    const Params<T>& P = *static_cast<const Params<T>*>(L.params);
+    const bool wide = (size_t)P.n[0] * P.n[1] * sizeof(T4<T>) >= (size_t)1 << 32;
     if constexpr (sizeof(T) == 8) {
-      fused_tile<20, 20>(L, u1, u2, o1, o2, ck, za, zb, zc, debug);
+      if (wide) fused_tile<20, 20>(L, u1, u2, o1, o2, ck, za, zb, zc, debug);
+      else fused_roles<16, 16>(L, u1, u2, o1, o2, ck, za, zb, zc, debug);
     } else {
+      if (wide) tile = FUSED_32x16;
       switch (tile) {
         case FUSED_R32x16: fused_roles<32, 16>(L, u1, u2, o1, o2, ck, za, zb, zc, debug); break;
         case FUSED_R32x8: fused_roles<32, 8>(L, u1, u2, o1, o2, ck, za, zb, zc, debug); break;

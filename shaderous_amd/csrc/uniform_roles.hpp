@@ -1,19 +1,24 @@
 // The fused uniform-grid step with threads by role (k_fused_r): the same arithmetic as k_fused,
-// with a different map of threads to the tile's columns and two barriers per plane instead of
-// four. A tile is TX x TY cells (32 x 16, 32 x 8 or 16 x 16, so 256^3 and other power-of-two
-// grids split into whole tiles); of its (TX + 4) x (TY + 4) columns, threads own, in this order:
+// with a different map of threads to the tile's columns. A tile is TX x TY cells (32 x 16, 32 x 8
+// or 16 x 16, so 256^3 and other power-of-two grids split into whole tiles); of its
+// (TX + 4) x (TY + 4) columns, threads own, in this order:
 //   [0, TX TY)               the cell columns, x fastest: whole waves of cell work
 //   the next 2 TX + 2 TY     ring 1 without its corners (half steps): the top row and the right
 //                            column first (they also solve the faces they share with the tile's
 //                            cells), then the bottom row and the left column
-//   the next 4               ring 1's corners (loads only: their primitives feed the transverse
-//                            slopes of ring 1's ends)
 //   the last 2 TX + 2 TY     ring 2 without its corners (loads only); ring 2's corners are never
-//                            read
-// The cell waves never carry halo lanes; at 16 x 16 the 64 half-step lanes of ring 1 are one
-// wave. LDS holds the plane data in raster order of the columns, with the x/y fluxes apart from
-// the sides (RoleLayout), so a plane needs one barrier after the half steps and one after the
-// fluxes.
+//                            read. The last four threads load ring 1's corners as well (their
+//                            primitives feed the transverse slopes of ring 1's ends), so that
+//                            they take no wave of their own: 16 x 16 cells are six waves.
+// Each role runs its own loop over the planes (a scalar branch per wave, the barriers in step): the
+// cell waves never carry halo lanes or their registers, and the planes before the first and after
+// the last one, which need only the cells' z sides, cost the other waves a conversion.
+//
+// Bound by VALU issue. Against one loop for every role with its stages behind lane masks, the
+// state re-read at its use and single-value LDS accesses, per step: 256^3 MC 0.515 -> 0.342 ms
+// (3.1 TB/s of state read and written once), Koren + isentropic 0.795 -> 0.656; 128^3 0.073 ->
+// 0.053 and 0.124 -> 0.102; FP64 96^3 MC 0.147 (raster tiles) -> 0.104. 32 x 16 is the tile of large
+// grids: its two ring waves land on two SIMDs, beside two cell waves each.
 #pragma once
 
 namespace shx {
@@ -24,15 +29,28 @@ struct RoleTile {
   static constexpr int NCELL = TX * TY;
   static constexpr int NHALF = NCELL + 2 * TX + 2 * TY;          // threads that form half steps
   static constexpr int NFACE = NCELL + TX + TY;                  // threads that solve x/y faces
-  static constexpr int NTH = NHALF + 4 + 2 * TX + 2 * TY;        // threads
-  // waves per SIMD the launch bound asks for: one 12-wave workgroup per CU at 32 x 16 (168
-  // VGPRs), two 7-wave workgroups otherwise (128 VGPRs)
-  static constexpr int MINW = NCELL > 256 ? 3 : 4;
+  static constexpr int NTH = NHALF + 2 * TX + 2 * TY;            // threads with a role
+  // At 16 x 16 the ring wave and the load wave are the fifth and sixth of a workgroup, and waves go
+  // to a CU's SIMDs in turn: two workgroups would put both ring waves on the first SIMD (0.523
+  // against 0.383 ms at 256^3). So a workgroup is launched with eight waves, of which the last
+  // four hold those two roles in the fifth and sixth or, in every second run of 256 workgroups (as
+  // many as there are CUs), in the seventh and eighth; the other two end at once.
+  // (FP64 has the LDS for one workgroup per CU.)
+  template <typename T>
+  static constexpr bool paired() { return sizeof(T) == 4 && NCELL == 256 && NTH == 384; }
+  template <typename T>
+  static constexpr int launch() { return paired<T>() ? 512 : NTH; }
+  // waves per SIMD the launch bound asks for in FP32: one 11-wave workgroup per CU at 32 x 16 (up
+  // to 168 VGPRs), two otherwise (128 VGPRs); one at 16 x 16 where Koren's edges need more
+  // registers than that (it serves the grids with too few tiles for two), and in FP64
+  template <typename T, int LIM>
+  static constexpr int minw() {
+    return sizeof(T) == 8 || (paired<T>() && !lim_symmetric<LIM>()) ? 2 : (NCELL > 256 ? 3 : 4);
+  }
 };
 
-// LDS of k_fused_r, per column: primitives of two planes (rho, v, p, s: the centre's sound speed
-// stays in a register), x and y sides, x and y fluxes: 46 values (132 KB at 32 x 16 cells, one
-// workgroup per CU; 79.5 KB at 32 x 8, two per CU)
+// The block march's LDS (k_amr_fused), per column: primitives of two planes (rho, v, p, s: the
+// centre's sound speed stays in a register), x and y sides, x and y fluxes: 46 values
 template <int NT>
 struct RoleLayout {
   static constexpr int Q0 = 0, Q1 = 6 * NT, SX = 12 * NT, SY = 21 * NT, FX = 30 * NT, FY = 38 * NT;
@@ -50,15 +68,8 @@ template <int TX, int TY>
 __device__ __forceinline__ void role_column(int t, int& cx, int& cy) {
   using RT = RoleTile<TX, TY>;
   if (t < RT::NCELL) {
-    if constexpr (TX == 16) {
-      // a wave holds a 4-wide strip of 16 rows: with the LDS rows 20 columns apart its lanes
-      // then reach distinct banks (4 rows of 16 would meet in a third of them)
-      cx = 4 * (t >> 6) + (t & 3);
-      cy = (t & 63) >> 2;
-    } else {
-      cx = t % TX;
-      cy = t / TX;
-    }
+    cx = t % TX;
+    cy = t / TX;
     return;
   }
   t -= RT::NCELL;
@@ -70,8 +81,6 @@ __device__ __forceinline__ void role_column(int t, int& cx, int& cy) {
   t -= TX;
   if (t < TY) { cx = -1; cy = t; return; }             // the left column
   t -= TY;
-  if (t < 4) { cx = (t & 1) ? TX : -1; cy = (t & 2) ? TY : -1; return; }   // the corners
-  t -= 4;
   if (t < TX) { cx = t; cy = -2; return; }             // ring 2: bottom, top, left, right
   t -= TX;
   if (t < TX) { cx = t; cy = TY + 1; return; }
@@ -81,28 +90,166 @@ __device__ __forceinline__ void role_column(int t, int& cx, int& cy) {
   cx = TX + 1; cy = t;
 }
 
-// Launch bound: 32 x 16, 708 threads (12 waves), one workgroup per CU at up to 168 VGPRs;
-// 32 x 8 (420 threads) and 16 x 16 (388), 7 waves, two per CU at up to 128 VGPRs.
+// The planes in LDS: per column the primitives of two planes (rho, v | p, s; the centre's sound
+// speed stays in a register), the upper x and y sides (rho, v | p, s, half-step rho and p) with the
+// cell's shock flag, and the fluxes of the x and y faces below the column: 45 values, kept as
+// 4- and 2-vectors so that a neighbour is two or three LDS instructions and not six to nine.
+template <typename T> struct Vec2;
+template <> struct Vec2<float> { using type = float2; };
+template <> struct Vec2<double> { using type = double2; };
+template <typename T, int NT>
+struct PlaneLds {
+  static constexpr int QA = 0, QB = 4 * NT, QN = 6 * NT;      // + QN: the other plane
+  static constexpr int SX = 12 * NT, SY = 20 * NT, SK = 28 * NT, FX = 29 * NT, FY = 37 * NT, SIZE = 45 * NT;
+  using V4 = T4<T>;
+  using V2 = typename Vec2<T>::type;
+  // A column's byte offsets in the arrays of 4-, 2- and 1-vectors, each kept as a value of its own
+  // (the empty asm): the compiler derives one from another by a quarter-rate multiplication per
+  // plane otherwise. off: a column so many to the right.
+  struct At {
+    unsigned int a, b, c;
+    __device__ __forceinline__ At off(int d) const {
+      return At{a + (unsigned int)(d * (int)sizeof(V4)), b + (unsigned int)(d * (int)sizeof(V2)),
+                c + (unsigned int)(d * (int)sizeof(T))};
+    }
+  };
+  static __device__ __forceinline__ At at(int t) {
+    At k{(unsigned int)(t * (int)sizeof(V4)), (unsigned int)(t * (int)sizeof(V2)), (unsigned int)(t * (int)sizeof(T))};
+    asm("" : "+v"(k.a));
+    asm("" : "+v"(k.b));
+    asm("" : "+v"(k.c));
+    return k;
+  }
+  template <typename V>
+  static __device__ __forceinline__ V& ref(T* L, int base, unsigned int off) {
+    return *reinterpret_cast<V*>(reinterpret_cast<char*>(L + base) + off);
+  }
+  static __device__ __forceinline__ void put_prim(T* L, int q, const At& t, const Prim<T>& w) {
+    V4 a; a.x = w.rho; a.y = w.vx; a.z = w.vy; a.w = w.vz;
+    V2 b; b.x = w.p; b.y = w.s;
+    ref<V4>(L, q + QA, t.a) = a;
+    ref<V2>(L, q + QB, t.b) = b;
+  }
+  static __device__ __forceinline__ Prim<T> prim(T* L, int q, const At& t) {
+    const V4 a = ref<V4>(L, q + QA, t.a);
+    const V2 b = ref<V2>(L, q + QB, t.b);
+    Prim<T> w;
+    w.rho = a.x; w.vx = a.y; w.vy = a.z; w.vz = a.w; w.p = b.x; w.s = b.y; w.cs = T(0);
+    return w;
+  }
+  static __device__ __forceinline__ void put_side(T* L, int s, const At& t, const SideData<T>& d) {
+    V4 a; a.x = d.rho; a.y = d.vx; a.z = d.vy; a.w = d.vz;
+    V4 b; b.x = d.p; b.y = d.s; b.z = d.hrho; b.w = d.hp;
+    ref<V4>(L, s, t.a) = a;
+    ref<V4>(L, s + 4 * NT, t.a) = b;
+  }
+  static __device__ __forceinline__ void put_shock(T* L, const At& t, T shock) { ref<T>(L, SK, t.c) = shock; }
+  static __device__ __forceinline__ SideData<T> side(T* L, int s, const At& t) {
+    const V4 a = ref<V4>(L, s, t.a), b = ref<V4>(L, s + 4 * NT, t.a);
+    SideData<T> d;
+    d.rho = a.x; d.vx = a.y; d.vy = a.z; d.vz = a.w; d.p = b.x; d.s = b.y; d.hrho = b.z; d.hp = b.w;
+    d.shock = ref<T>(L, SK, t.c);
+    return d;
+  }
+  static __device__ __forceinline__ void put_flux(T* L, int f, const At& t, const Flux<T>& F) {
+    V4 a; a.x = F.m; a.y = F.mx; a.z = F.my; a.w = F.mz;
+    V4 b; b.x = F.e; b.y = F.ei; b.z = F.s; b.w = F.vn;
+    ref<V4>(L, f, t.a) = a;
+    ref<V4>(L, f + 4 * NT, t.a) = b;
+  }
+  static __device__ __forceinline__ Flux<T> flux(T* L, int f, const At& t) {
+    const V4 a = ref<V4>(L, f, t.a), b = ref<V4>(L, f + 4 * NT, t.a);
+    Flux<T> F;
+    F.m = a.x; F.mx = a.y; F.my = a.z; F.mz = a.w; F.e = b.x; F.ei = b.y; F.s = b.z; F.vn = b.w;
+    return F;
+  }
+};
+
+// A cell of a plane by its byte offset, through a buffer resource over the plane (a scalar base and
+// one 32-bit vector offset; the resource covers 4 GiB, beyond what offsets reach)
+typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t plane_rsrc(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0xffffffff, 0x00020000);
+}
+template <typename T>
+__device__ __forceinline__ T4<T> plane_load(const T4<T>* base, unsigned int off) {
+  const __amdgpu_buffer_rsrc_t r = plane_rsrc(base);
+  struct Words { u32x4 w[sizeof(T4<T>) / 16]; } k;
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(T4<T>) / 16); i++) k.w[i] = __builtin_amdgcn_raw_buffer_load_b128(r, off + 16 * i, 0, 0);
+  return __builtin_bit_cast(T4<T>, k);
+}
+template <typename T>
+__device__ __forceinline__ void plane_store(T4<T>* base, unsigned int off, T4<T> v) {
+  const __amdgpu_buffer_rsrc_t r = plane_rsrc(base);
+  struct Words { u32x4 w[sizeof(T4<T>) / 16]; } k = __builtin_bit_cast(Words, v);
+#pragma unroll
+  for (int i = 0; i < (int)(sizeof(T4<T>) / 16); i++) __builtin_amdgcn_raw_buffer_store_b128(k.w[i], r, off + 16 * i, 0, 0);
+}
+
+// The net inflow of a plane's x and y faces, and with the z faces' (lower lo, upper hi)
+template <typename T>
+__device__ __forceinline__ Flux<T> net_xy(const Flux<T>& xl, const Flux<T>& xh, const Flux<T>& yl, const Flux<T>& yh) {
+  Flux<T> n;
+  n.m = (xl.m - xh.m) + (yl.m - yh.m);
+  n.mx = (xl.mx - xh.mx) + (yl.mx - yh.mx);
+  n.my = (xl.my - xh.my) + (yl.my - yh.my);
+  n.mz = (xl.mz - xh.mz) + (yl.mz - yh.mz);
+  n.e = (xl.e - xh.e) + (yl.e - yh.e);
+  n.ei = (xl.ei - xh.ei) + (yl.ei - yh.ei);
+  n.s = (xl.s - xh.s) + (yl.s - yh.s);
+  n.vn = (xl.vn - xh.vn) + (yl.vn - yh.vn);
+  return n;
+}
+template <typename T>
+__device__ __forceinline__ Flux<T> net_z(const Flux<T>& xy, const Flux<T>& lo, const Flux<T>& hi) {
+  Flux<T> n;
+  n.m = xy.m + (lo.m - hi.m);
+  n.mx = xy.mx + (lo.mx - hi.mx);
+  n.my = xy.my + (lo.my - hi.my);
+  n.mz = xy.mz + (lo.mz - hi.mz);
+  n.e = xy.e + (lo.e - hi.e);
+  n.ei = xy.ei + (lo.ei - hi.ei);
+  n.s = xy.s + (lo.s - hi.s);
+  n.vn = xy.vn + (lo.vn - hi.vn);
+  return n;
+}
+
 // z: periodic, or through a non-periodic face as k_fused (ZA, ZB: the boundary planes' half steps).
+// Columns beyond the grid (a ragged tile's) compute on the cells they map to and store nothing.
 // Barriers: the half steps of plane c (sides, and plane c + 1's primitives) are visible after
 // the first, its x/y fluxes after the second. The sides of plane c + 1 overwrite those of plane c
 // after the second barrier of plane c (the last reads of sides were before it); the fluxes of
 // plane c + 1 overwrite those of plane c after the first barrier of plane c + 1; each primitive
-// buffer is rewritten a plane after its neighbours were last read from it.
+// buffer is rewritten a plane after its neighbours were last read from it. The z faces and the
+// update of plane c - 1 need nothing of LDS: they go before the first barrier, and the state they
+// update is loaded a half step ahead.
+// A plane's byte offsets fit 32 bits (the launcher's rule), so a load is a scalar base and one
+// vector offset.
 template <typename T, int LIM, int RS, bool ISEN, int TX, int TY, bool DEBUG, bool MAPBC>
-__global__ __launch_bounds__((RoleTile<TX, TY>::NTH), (RoleTile<TX, TY>::MINW)) void k_fused_r(
+__global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile<TX, TY>::template minw<T, LIM>())) void k_fused_r(
     Params<T> P, const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, T4<T>* __restrict__ O1,
     T4<T>* __restrict__ O2, StepClock<T> C, const T4<T>* __restrict__ ZA, const T4<T>* __restrict__ ZB, int zc) {
   using RT = RoleTile<TX, TY>;
-  constexpr int NT = RT::NC, BX = RT::CX, BY = RT::CY;
-  using LY = RoleLayout<NT>;
-  __shared__ T L[LY::SIZE];
-  __shared__ T red[NT / 64 + 1];
-  const int tid = threadIdx.x;
+  constexpr int NT = RT::NC, BX = RT::CX, NW = (RT::NTH + 63) / 64;
+  using PL = PlaneLds<T, NT>;
+  __shared__ T4<T> LV[PL::SIZE / 4];
+  __shared__ T red[NW];
+  T* const L = reinterpret_cast<T*>(LV);
+  const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+  // the wave's role, a scalar
+  int wave = __builtin_amdgcn_readfirstlane(threadIdx.x) >> 6;
+  if constexpr (RT::template paired<T>()) {
+    if (wave >= 4) {
+      if (((wave >> 1) & 1) != ((lin >> 8) & 1)) return;
+      wave = 4 | (wave & 1);
+    }
+  }
+  const int tid = wave * 64 + (threadIdx.x & 63);
+  const bool cells = wave < RT::NCELL / 64, rings = !cells && wave * 64 < RT::NHALF;
   int cx, cy;
   role_column<TX, TY>(tid, cx, cy);
-  const int t = (cy + 2) * BX + (cx + 2);          // raster index of the column
-  const bool cell = tid < RT::NCELL;               // wave-uniform
+  const typename PL::At t = PL::at((cy + 2) * BX + (cx + 2));   // the column, in raster order
   const int nx = P.n[0], ny = P.n[1], nz = P.n[2];
   // XCD-aware tile order: the dispatcher deals workgroups to the 8 XCDs in turn (workgroup i to
   // XCD i mod 8), so XCD k takes the k-th of 8 contiguous runs of tiles (the first n mod 8 runs
@@ -111,52 +258,42 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::NTH), (RoleTile<TX, TY>::MINW)) 
   int bx, by, bz;
   {
     const int ntile = gridDim.x * gridDim.y * gridDim.z;
-    const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
     const int k = lin & 7, q = ntile >> 3, r = ntile & 7;
     const int m = k * q + min(k, r) + (lin >> 3);
     bx = m % gridDim.x;
     by = (m / gridDim.x) % gridDim.y;
     bz = m / (gridDim.x * gridDim.y);
   }
-  const int x = bx * TX + cx;
-  const int y = by * TY + cy;
   const int z0 = bz * zc;
   const int z1 = min(z0 + zc, nz);
   const T dt = step_dt(P, C, 0);
-  const T dtdx = dt / P.dx;
+  const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
   if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && tid == 0) step_clock_advance(P, C, 0);
 
-  AxisMap mx = map_axis(x, nx, P.bc_lo[0], P.bc_hi[0]);
-  AxisMap my = map_axis(y, ny, P.bc_lo[1], P.bc_hi[1]);
-  const size_t col = (size_t)my.i * nx + mx.i;
   const size_t plane = (size_t)nx * ny;
-
-  const bool in_r1 = tid < RT::NHALF;              // cells and ring 1 without its corners
-  const bool ring_face = !cell && tid < RT::NFACE; // ring 1's top row and right column
-  const bool real_x = x >= 0 && x < nx, real_y = y >= 0 && y < ny;
-  const bool upd = cell && real_x && real_y;
-  const bool xface = cx >= 0 && cx <= TX && cy >= 0 && cy < TY && x <= nx && real_y;
-  const bool yface = cy >= 0 && cy <= TY && cx >= 0 && cx < TX && y <= ny && real_x;
-  // a ghost column beyond a non-periodic face takes the half step of the cell it maps to
-  // (load_pred, hydro/update.wgsl:47-63): that cell's stencil sits inward in the tile
-  int sx = cx, sy = cy;
-  if (!real_x && ((x < 0 && P.bc_lo[0] != BC_PERIODIC) || (x >= nx && P.bc_hi[0] != BC_PERIODIC))) sx = cx + (mx.i - x);
-  if (!real_y && ((y < 0 && P.bc_lo[1] != BC_PERIODIC) || (y >= ny && P.bc_hi[1] != BC_PERIODIC))) sy = cy + (my.i - y);
-  const bool mapped = MAPBC && ((sx != cx) || (sy != cy));
-  const int ts = (min(max(sy, -1), TY) + 2) * BX + (min(max(sx, -1), TX) + 2);
-
   // z: periodic, or (ZA given) a non-periodic face that ghost planes map through
   const bool zbc = MAPBC && ZA != nullptr;
-  auto plane_of = [&](int z) {
-    const int zi = zbc ? map_axis(z, nz, P.bc_lo[2], P.bc_hi[2]).i : ((z % nz) + nz) % nz;
-    return (size_t)zi * plane + col;
+  auto plane_of = [&](int z) -> size_t {
+    if (zbc) return (size_t)map_axis(z, nz, P.bc_lo[2], P.bc_hi[2]).i * plane;
+    while (z < 0) z += nz;
+    while (z >= nz) z -= nz;
+    return (size_t)z * plane;
   };
-  auto prim_of = [&](T4<T> u1, T4<T> u2, int z) {
+  // a column of the tile: the byte offset in a plane of the cell it maps to, and whether that cell
+  // is seen through a reflecting x or y face (its velocity turns; outflow-only faces, which clip
+  // it, are not run here)
+  struct Column { unsigned int at; bool fx, fy; };
+  auto column = [&](int cx, int cy) {
+    const AxisMap mx = map_axis(bx * TX + cx, nx, P.bc_lo[0], P.bc_hi[0]);
+    const AxisMap my = map_axis(by * TY + cy, ny, P.bc_lo[1], P.bc_hi[1]);
+    return Column{(unsigned int)(my.i * nx + mx.i) * (unsigned int)sizeof(T4<T>), mx.flip < 0, my.flip < 0};
+  };
+  auto at = [](const T4<T>* base, unsigned int off) { return plane_load<T>(base, off); };
+  auto prim_of = [&](const Column& k, T4<T> u1, T4<T> u2, int z) {
     Prim<T> q = prim_from_cons(P, u1, u2);
     if constexpr (MAPBC) {
-      // (x and y periodic: every column's map has flip 1 and side 0, which bc_vel leaves as is)
-      q.vx = bc_vel(q.vx, mx.flip, mx.side);
-      q.vy = bc_vel(q.vy, my.flip, my.side);
+      q.vx = k.fx ? -q.vx : q.vx;
+      q.vy = k.fy ? -q.vy : q.vy;
     }
     if (zbc && (z < 0 || z >= nz)) {
       const AxisMap mz = map_axis(z, nz, P.bc_lo[2], P.bc_hi[2]);
@@ -164,157 +301,261 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::NTH), (RoleTile<TX, TY>::MINW)) 
     }
     return q;
   };
-
-  T4<T> b1, b2;
-  size_t o0 = plane_of(z0 - 2);
-  lds_put_prim6<T, NT>(L + LY::Q0, t, prim_of(U1[o0], U2[o0], z0 - 2));
-  o0 = plane_of(z0 - 1);
-  T cs_c;   // this column's sound speed in plane c
+  const Column K = column(cx, cy);
+  // a ghost column beyond a non-periodic face takes the half step of the cell it maps to
+  // (load_pred, hydro/update.wgsl:47-63): that cell's stencil sits inward in the tile
+  int sx = cx, sy = cy;
   {
-    Prim<T> q = prim_of(U1[o0], U2[o0], z0 - 1);
-    lds_put_prim6<T, NT>(L + LY::Q1, t, q);
-    cs_c = q.cs;
+    const int x = bx * TX + cx, y = by * TY + cy;
+    if ((x < 0 && P.bc_lo[0] != BC_PERIODIC) || (x >= nx && P.bc_hi[0] != BC_PERIODIC))
+      sx = cx + (map_axis(x, nx, P.bc_lo[0], P.bc_hi[0]).i - x);
+    if ((y < 0 && P.bc_lo[1] != BC_PERIODIC) || (y >= ny && P.bc_hi[1] != BC_PERIODIC))
+      sy = cy + (map_axis(y, ny, P.bc_lo[1], P.bc_hi[1]).i - y);
   }
-  o0 = plane_of(z0);
-  b1 = U1[o0]; b2 = U2[o0];
-  __syncthreads();
+  const bool mapped = MAPBC && ((sx != cx) || (sy != cy));
+  const bool any_mapped = MAPBC && __ballot(mapped) != 0;
+  const typename PL::At ts = PL::at((min(max(sy, -1), TY) + 2) * BX + (min(max(sx, -1), TX) + 2));
 
-  SideData<T> zs_prev;
-  Flux<T> fz_lo = zero_flux<T>();
-  Flux<T> axy_prev = zero_flux<T>();
-  T rate_max = T(0);
-
-  for (int c = z0 - 1; c <= z1; c++) {
-    Prim<T> pp = prim_of(b1, b2, c + 1);
-    if (c + 2 <= z1 + 1) {
-      size_t o = plane_of(c + 2);
-      b1 = U1[o];
-      b2 = U2[o];
+  // the half step of this column in the plane whose primitives are at q (those of the plane below
+  // at m, of the plane above in pp), and its edge increments (hydro/predictor.wgsl:46-209)
+  struct Edges { Inc<T> xu, xd, yu, yd, zu, zd; };
+  auto half_at = [&](int q, const typename PL::At& at, Prim<T> pc, const Prim<T>& pm, const Prim<T>& pp, Edges& e) {
+    AxisSlope<T> sl[3];
+    // axis by axis: the scheduler would read every neighbour first, at 12 more registers an axis
+    T conv, jump;
+    {
+      const Prim<T> xm = PL::prim(L, q, at.off(-1)), xp = PL::prim(L, q, at.off(1));
+      sl[0] = axis_slope<T, LIM, ISEN>(P, xm, pc, xp, &e.xu, &e.xd);
+      conv = xp.vx - xm.vx;
+      jump = jump_over(P, xm.p, xp.p);
     }
-    const bool odd = ((c - z0 + 1) & 1) != 0;
-    const T* Lq = L + (odd ? LY::Q0 : LY::Q1);
-    T* Lm = L + (odd ? LY::Q1 : LY::Q0);
-
-    // 2. half step and sides of plane c (hydro/predictor.wgsl:46-209)
-    SideData<T> sxl, syl, szl, szu;
-    if (in_r1) {
-      Prim<T> pc = lds_prim<T, NT>(Lq, t);
-      pc.cs = cs_c;
-      Prim<T> pm = lds_prim<T, NT>(Lm, t);
-      Prim<T> xm = lds_prim<T, NT>(Lq, t - 1), xp = lds_prim<T, NT>(Lq, t + 1);
-      Prim<T> ym = lds_prim<T, NT>(Lq, t - BX), yp = lds_prim<T, NT>(Lq, t + BX);
-      Inc<T> ixu, ixd, iyu, iyd, izu, izd;
-      AxisSlope<T> sl[3];
-      sl[0] = axis_slope<T, LIM, ISEN>(P, xm, pc, xp, &ixu, &ixd);
-      sl[1] = axis_slope<T, LIM, ISEN>(P, ym, pc, yp, &iyu, &iyd);
-      sl[2] = axis_slope<T, LIM, ISEN>(P, pm, pc, pp, &izu, &izd);
-      Half<T> hc;
-      if (!MAPBC || !mapped) {
-        T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (pp.vz - pm.vz);
-        T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, pm.p, pp.p)));
-        hc = hancock<T, LIM>(P, pc, sl, conv, jump, dt);
-      } else {
+    __builtin_amdgcn_sched_barrier(0);
+    {
+      const Prim<T> ym = PL::prim(L, q, at.off(-BX)), yp = PL::prim(L, q, at.off(BX));
+      sl[1] = axis_slope<T, LIM, ISEN>(P, ym, pc, yp, &e.yu, &e.yd);
+      conv = conv + (yp.vy - ym.vy);
+      jump = tmax(jump, jump_over(P, ym.p, yp.p));
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    sl[2] = axis_slope<T, LIM, ISEN>(P, pm, pc, pp, &e.zu, &e.zd);
+    __builtin_amdgcn_sched_barrier(0);
+    conv = conv + (pp.vz - pm.vz);
+    return hancock<T, LIM>(P, pc, sl, conv, tmax(jump, jump_over(P, pm.p, pp.p)), hstep);
+  };
+  auto half_of = [&](int q, int m, T cs, const Prim<T>& pp, Edges& e) {
+    Prim<T> pc = PL::prim(L, q, t);
+    pc.cs = cs;
+    const Prim<T> pm = PL::prim(L, m, t);
+    if constexpr (!MAPBC) {
+      return half_at(q, t, pc, pm, pp, e);
+    } else {
+      // where a lane of the wave is mapped: first every lane's half step at the cell it maps to (the
+      // column itself if it maps to none), its centre being this column's primitives seen
+      // unflipped, then the increments and the half step here. One body, two turns.
+      Half<T> h, hm;
+#pragma unroll 1
+      for (int k = any_mapped ? 0 : 1; k < 2; k++) {
+        const bool first = k == 0;
         Prim<T> qc = pc, qm = pm, qp = pp;
-        qc.vx = bc_vel(qc.vx, mx.flip, 0); qc.vy = bc_vel(qc.vy, my.flip, 0);
-        qm.vx = bc_vel(qm.vx, mx.flip, 0); qm.vy = bc_vel(qm.vy, my.flip, 0);
-        qp.vx = bc_vel(qp.vx, mx.flip, 0); qp.vy = bc_vel(qp.vy, my.flip, 0);
-        Prim<T> sxm = lds_prim<T, NT>(Lq, ts - 1), sxp = lds_prim<T, NT>(Lq, ts + 1);
-        Prim<T> sym = lds_prim<T, NT>(Lq, ts - BX), syp = lds_prim<T, NT>(Lq, ts + BX);
-        AxisSlope<T> ms[3];
-        ms[0] = axis_slope<T, LIM, ISEN>(P, sxm, qc, sxp, nullptr, nullptr);
-        ms[1] = axis_slope<T, LIM, ISEN>(P, sym, qc, syp, nullptr, nullptr);
-        ms[2] = axis_slope<T, LIM, ISEN>(P, qm, qc, qp, nullptr, nullptr);
-        T conv = (sxp.vx - sxm.vx) + (syp.vy - sym.vy) + (qp.vz - qm.vz);
-        T jump = tmax(jump_over(P, sxm.p, sxp.p), tmax(jump_over(P, sym.p, syp.p), jump_over(P, qm.p, qp.p)));
-        hc = hancock<T, LIM>(P, qc, ms, conv, jump, dt);
-        hc.vx = bc_vel(hc.vx, mx.flip, mx.side);
-        hc.vy = bc_vel(hc.vy, my.flip, my.side);
-      }
-      if (zbc && upd) zghost_half(P, ZA, ZB, c, (size_t)y * nx + x, hc);
-      sxl = side_of(hc, ixd, T(-1));
-      syl = side_of(hc, iyd, T(-1));
-      szl = side_of(hc, izd, T(-1));
-      szu = side_of(hc, izu, T(1));
-      lds_put_side<T, NT>(L, LY::SX, t, side_of(hc, ixu, T(1)));
-      lds_put_side<T, NT>(L, LY::SY, t, side_of(hc, iyu, T(1)));
-    }
-    lds_put_prim6<T, NT>(Lm, t, pp);
-    cs_c = pp.cs;
-    __syncthreads();
-
-    // 3. the x and y faces below this column, and the z face below plane c
-    const bool live = c >= z0 && c < z1;
-    Flux<T> Fx = zero_flux<T>(), Fy = zero_flux<T>(), fz = zero_flux<T>();
-    if (cell) {
-      if (live && xface) Fx = face_from_sides<T, RS>(P, lds_get_side<T, NT>(L, LY::SX, t - 1), sxl, 0);
-      if (live && yface) Fy = face_from_sides<T, RS>(P, lds_get_side<T, NT>(L, LY::SY, t - BX), syl, 1);
-      if (upd && c >= z0) fz = face_from_sides<T, RS>(P, zs_prev, szl, 2);
-      // 4. the x/y fluxes into LDS
-      if (live && xface) lds_put_flux<T, NT>(L, LY::FX, t, Fx);
-      if (live && yface) lds_put_flux<T, NT>(L, LY::FY, t, Fy);
-    } else if (ring_face && live && (xface || yface)) {
-      // ring 1: the right column's x face or the top row's y face, one solve along the lane's axis
-      const bool ax = xface;
-      const Flux<T> F = face_from_sides_rt<T, RS>(
-          P, lds_get_side<T, NT>(L, ax ? LY::SX : LY::SY, ax ? t - 1 : t - BX), ax ? sxl : syl, ax ? 0 : 1);
-      lds_put_flux<T, NT>(L, ax ? LY::FX : LY::FY, t, F);
-    }
-    __syncthreads();
-
-    // 5. this plane's x/y net inflow, and the update of plane c - 1
-    if (cell) {
-      Flux<T> axy = zero_flux<T>();
-      if (live && upd) {
-        Flux<T> xh = lds_get_flux<T, NT>(L, LY::FX, t + 1);
-        Flux<T> yh = lds_get_flux<T, NT>(L, LY::FY, t + BX);
-        if constexpr (DEBUG) {
-          axy.m = Fx.m; axy.mx = xh.m; axy.my = Fy.m; axy.mz = yh.m;
-        } else {
-          axy.m = (Fx.m - xh.m) + (Fy.m - yh.m);
-          axy.mx = (Fx.mx - xh.mx) + (Fy.mx - yh.mx);
-          axy.my = (Fx.my - xh.my) + (Fy.my - yh.my);
-          axy.mz = (Fx.mz - xh.mz) + (Fy.mz - yh.mz);
-          axy.e = (Fx.e - xh.e) + (Fy.e - yh.e);
-          axy.ei = (Fx.ei - xh.ei) + (Fy.ei - yh.ei);
-          axy.s = (Fx.s - xh.s) + (Fy.s - yh.s);
-          axy.vn = (Fx.vn - xh.vn) + (Fy.vn - yh.vn);
+        if (first) {
+          qc.vx = K.fx ? -qc.vx : qc.vx; qc.vy = K.fy ? -qc.vy : qc.vy;
+          qm.vx = K.fx ? -qm.vx : qm.vx; qm.vy = K.fy ? -qm.vy : qm.vy;
+          qp.vx = K.fx ? -qp.vx : qp.vx; qp.vy = K.fy ? -qp.vy : qp.vy;
+        }
+        h = half_at(q, first ? ts : t, qc, qm, qp, e);
+        if (first) {
+          hm = h;
+          hm.vx = K.fx ? -hm.vx : hm.vx;
+          hm.vy = K.fy ? -hm.vy : hm.vy;
         }
       }
-      if (upd && c - 1 >= z0 && c - 1 < z1) {
-        size_t o = (size_t)(c - 1) * plane + col;
-        T4<T> o1, o2;
-        if constexpr (DEBUG) {
-          o1.x = axy_prev.m; o1.y = axy_prev.mx; o1.z = axy_prev.my; o1.w = axy_prev.mz;
-          o2.x = fz_lo.m; o2.y = fz.m; o2.z = T(0); o2.w = T(0);
-        } else {
-          Flux<T> net;
-          net.m = axy_prev.m + (fz_lo.m - fz.m);
-          net.mx = axy_prev.mx + (fz_lo.mx - fz.mx);
-          net.my = axy_prev.my + (fz_lo.my - fz.my);
-          net.mz = axy_prev.mz + (fz_lo.mz - fz.mz);
-          net.e = axy_prev.e + (fz_lo.e - fz.e);
-          net.ei = axy_prev.ei + (fz_lo.ei - fz.ei);
-          net.s = axy_prev.s + (fz_lo.s - fz.s);
-          net.vn = axy_prev.vn + (fz_lo.vn - fz.vn);
-          advance(P, U1[o], U2[o], net, zs_prev.hp, dtdx, o1, o2);
-          Prim<T> w = prim_from_cons(P, o1, o2);
-          rate_max = tmax(rate_max, rate_of(P, w));
-        }
-        O1[o] = o1;
-        O2[o] = o2;
+      if (mapped) h = hm;
+      return h;
+    }
+  };
+  // the buffer of plane c's primitives: plane z0 - 2 and z0 in the first, z0 - 1 and z0 + 1 in the
+  // second, and so on
+  auto buf = [&](int c) { return ((c - z0) & 1) ? PL::QN : 0; };
+
+  T rate_max = T(0);
+  if (cells) {
+    const bool upd = bx * TX + cx < nx && by * TY + cy < ny;
+    T4<T> b1, b2;
+    auto load = [&](int z) {
+      const size_t o = plane_of(z);
+      b1 = at(U1 + o, K.at);
+      b2 = at(U2 + o, K.at);
+    };
+    load(z0 - 2);
+    PL::put_prim(L, buf(z0 - 2), t, prim_of(K, b1, b2, z0 - 2));
+    load(z0 - 1);
+    Prim<T> pp = prim_of(K, b1, b2, z0 - 1);
+    PL::put_prim(L, buf(z0 - 1), t, pp);
+    T cs = pp.cs;   // this column's sound speed in plane c
+    load(z0);
+    __syncthreads();
+    SideData<T> zs;           // the upper z side of the plane below
+    T hp;                     // and its half-step pressure
+    Flux<T> fz_lo, xy;        // the z face below and the x/y net inflow of that plane
+    auto update = [&](int c, T4<T> u1, T4<T> u2, const Flux<T>& fz) {
+      T4<T> o1, o2;
+      if constexpr (DEBUG) {
+        o1.x = xy.m; o1.y = xy.mx; o1.z = xy.my; o1.w = xy.mz;
+        o2.x = fz_lo.m; o2.y = fz.m; o2.z = T(0); o2.w = T(0);
+      } else {
+        advance(P, u1, u2, net_z(xy, fz_lo, fz), hp, dtdx, o1, o2);
       }
-      zs_prev = szu;
+      if (upd) {
+        const size_t o = (size_t)c * plane;
+        plane_store<T>(O1 + o, K.at, o1);
+        plane_store<T>(O2 + o, K.at, o2);
+        if constexpr (!DEBUG) rate_max = tmax(rate_max, rate_of(P, prim_from_cons(P, o1, o2)));
+      }
+    };
+    {
+      // plane z0 - 1: its upper z sides
+      pp = prim_of(K, b1, b2, z0);
+      load(z0 + 1);
+      Edges e;
+      Half<T> h = half_of(buf(z0 - 1), buf(z0 - 2), cs, pp, e);
+      if (zbc && upd) zghost_half(P, ZA, ZB, z0 - 1, K.at / sizeof(T4<T>), h);
+      zs = side_of(P, h, e.zu, T(1));
+      hp = h.p;
+      PL::put_prim(L, buf(z0), t, pp);
+      cs = pp.cs;
+    }
+    __syncthreads();
+    for (int c = z0; c < z1; c++) {
+      pp = prim_of(K, b1, b2, c + 1);
+      Edges e;
+      const Half<T> h = half_of(buf(c), buf(c - 1), cs, pp, e);
+      __builtin_amdgcn_sched_barrier(0);
+      T4<T> u1, u2;
+      if (c > z0) {
+        const size_t o = (size_t)(c - 1) * plane;
+        u1 = at(U1 + o, K.at);
+        u2 = at(U2 + o, K.at);
+      }
+      PL::put_side(L, PL::SX, t, side_of(P, h, e.xu, T(1)));
+      PL::put_side(L, PL::SY, t, side_of(P, h, e.yu, T(1)));
+      PL::put_shock(L, t, h.shock);
+      PL::put_prim(L, buf(c + 1), t, pp);
+      cs = pp.cs;
+      __builtin_amdgcn_sched_barrier(0);
+      const Flux<T> fz = face_from_sides<T, RS>(P, zs, side_of(P, h, e.zd, T(-1)), 2);
+      __builtin_amdgcn_sched_barrier(0);
+      if (c > z0) update(c - 1, u1, u2, fz);
       fz_lo = fz;
-      axy_prev = axy;
+      zs = side_of(P, h, e.zu, T(1));
+      hp = h.p;
+      __builtin_amdgcn_sched_barrier(0);
+      load(c + 2);
+      __syncthreads();
+      const Flux<T> Fx = face_from_sides<T, RS>(P, PL::side(L, PL::SX, t.off(-1)), side_of(P, h, e.xd, T(-1)), 0);
+      PL::put_flux(L, PL::FX, t, Fx);
+      __builtin_amdgcn_sched_barrier(0);
+      const Flux<T> Fy = face_from_sides<T, RS>(P, PL::side(L, PL::SY, t.off(-BX)), side_of(P, h, e.yd, T(-1)), 1);
+      PL::put_flux(L, PL::FY, t, Fy);
+      __syncthreads();
+      const Flux<T> xh = PL::flux(L, PL::FX, t.off(1)), yh = PL::flux(L, PL::FY, t.off(BX));
+      if constexpr (DEBUG) {
+        xy.m = Fx.m; xy.mx = xh.m; xy.my = Fy.m; xy.mz = yh.m;
+      } else {
+        xy = net_xy(Fx, xh, Fy, yh);
+      }
+    }
+    {
+      // plane z1: its lower z sides, and the update of plane z1 - 1
+      pp = prim_of(K, b1, b2, z1 + 1);
+      const size_t o = (size_t)(z1 - 1) * plane;
+      const T4<T> u1 = at(U1 + o, K.at), u2 = at(U2 + o, K.at);
+      Edges e;
+      Half<T> h = half_of(buf(z1), buf(z1 - 1), cs, pp, e);
+      if (zbc && upd) zghost_half(P, ZA, ZB, z1, K.at / sizeof(T4<T>), h);
+      update(z1 - 1, u1, u2, face_from_sides<T, RS>(P, zs, side_of(P, h, e.zd, T(-1)), 2));
+    }
+  } else if (rings) {
+    // ring 1 (and, in a mixed wave, ring 2's first lanes, which only load)
+    const bool ring1 = tid < RT::NHALF, face = tid < RT::NFACE;
+    const bool ax = cx == TX;      // the right column's x faces, else the top row's y faces
+    T4<T> b1, b2;
+    auto load = [&](int z) {
+      const size_t o = plane_of(z);
+      b1 = at(U1 + o, K.at);
+      b2 = at(U2 + o, K.at);
+    };
+    load(z0 - 1);
+    Prim<T> pp = prim_of(K, b1, b2, z0 - 1);
+    PL::put_prim(L, buf(z0 - 1), t, pp);
+    load(z0);
+    __syncthreads();
+    pp = prim_of(K, b1, b2, z0);
+    load(z0 + 1);
+    PL::put_prim(L, buf(z0), t, pp);
+    T cs = pp.cs;
+    __syncthreads();
+    for (int c = z0; c < z1; c++) {
+      pp = prim_of(K, b1, b2, c + 1);
+      if (c + 2 <= z1) load(c + 2);
+      SideData<T> lo;
+      if (ring1) {
+        Edges e;
+        const Half<T> h = half_of(buf(c), buf(c - 1), cs, pp, e);
+        PL::put_side(L, PL::SX, t, side_of(P, h, e.xu, T(1)));
+        PL::put_side(L, PL::SY, t, side_of(P, h, e.yu, T(1)));
+        PL::put_shock(L, t, h.shock);
+        const SideData<T> sxl = side_of(P, h, e.xd, T(-1)), syl = side_of(P, h, e.yd, T(-1));
+        lo = ax ? sxl : syl;
+      }
+      PL::put_prim(L, buf(c + 1), t, pp);
+      cs = pp.cs;
+      __syncthreads();
+      if (face) {
+        const Flux<T> F = face_from_sides_rt<T, RS>(P, PL::side(L, ax ? PL::SX : PL::SY, t.off(ax ? -1 : -BX)), lo, ax ? 0 : 1);
+        PL::put_flux(L, ax ? PL::FX : PL::FY, t, F);
+      }
+      __syncthreads();
+    }
+  } else {
+    // ring 2, and by the last four threads ring 1's corners
+    const int e = tid - (RT::NTH - 4);
+    const bool corner = e >= 0;
+    const int ex = (e & 1) ? TX : -1, ey = (e & 2) ? TY : -1;
+    const typename PL::At te = PL::at((ey + 2) * BX + (ex + 2));
+    const Column KE = column(ex, ey);
+    T4<T> b1, b2, c1, c2;
+    auto load = [&](int z) {
+      const size_t o = plane_of(z);
+      b1 = at(U1 + o, K.at);
+      b2 = at(U2 + o, K.at);
+      if (corner) {
+        c1 = at(U1 + o, KE.at);
+        c2 = at(U2 + o, KE.at);
+      }
+    };
+    auto put = [&](int z) {
+      PL::put_prim(L, buf(z), t, prim_of(K, b1, b2, z));
+      if (corner) PL::put_prim(L, buf(z), te, prim_of(KE, c1, c2, z));
+    };
+    load(z0);
+    __syncthreads();
+    put(z0);
+    if (z0 + 1 < z1) load(z0 + 1);
+    __syncthreads();
+    for (int c = z0; c < z1; c++) {
+      if (c + 1 < z1) put(c + 1);
+      if (c + 2 < z1) load(c + 2);
+      __syncthreads();
+      __syncthreads();
     }
   }
   if constexpr (!DEBUG) {
     T v = wave_max(rate_max);
-    if ((tid & 63) == 0) red[tid >> 6] = v;
+    if ((tid & 63) == 0) red[wave] = v;
     __syncthreads();
     if (tid == 0) {
       T m = T(0);
-      for (int w = 0; w < (NT + 63) / 64; w++) m = tmax(m, red[w]);
+      for (int w = 0; w < RT::NCELL / 64; w++) m = tmax(m, red[w]);
       max_slot(C.next(0), (unsigned long long)order_bits(m));
     }
   }
