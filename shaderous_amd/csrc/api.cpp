@@ -70,6 +70,7 @@ struct shx_sim {
   void* etiles[ENS_NTILES] = {};          // the grid's tiles (strips) for every 2D tile shape
   int entiles[ENS_NTILES] = {};
   int etile = ENS_ROWS16;
+  int rows_fit = 16;                      // the rows of ENS_ROWSFIT
   int egrid = 1024;                       // persistent grid of the tile kernel
 };
 
@@ -150,6 +151,11 @@ int reset_rates(shx_sim* s) {
     s->ops.rates(L, s->U1[s->cur], s->U2[s->cur], s->slot);
   }
   return SHX_OK;
+}
+
+// The 3D march's shapes for a configuration, cheapest first (none for a raster tile)
+std::vector<FusedShape> shapes_of(const shx_config& c, int cus, int tile, int zc) {
+  return fused_shapes(c.n[0], c.n[1], c.n[2], cus, c.precision == 64, c.limiter == SHX_LIM_KOREN, tile, zc);
 }
 
 bool fused_supported(const shx_config& c) {
@@ -414,28 +420,30 @@ int shx_create(const shx_config* cfg, shx_sim** out) {
   s->pf = make_params<float>(c);
   s->pd = make_params<double>(c);
   s->fused = c.path == SHX_PATH_FUSED && fused_supported(c);
-  s->tile = s->es == 8 ? FUSED_20x20 : FUSED_32x16;
-  s->zc = 32;
-  if (c.tile[0] > 0) {
-    for (int k = 0; k < FUSED_NTILES; k++) {
-      int tx, ty;
-      fused_tile_cells(k, tx, ty);
-      if (tx == c.tile[0] && ty == c.tile[1]) s->tile = k;
-    }
-    if (s->es == 8) s->tile = FUSED_20x20;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device) != hipSuccess || cus < 1) cus = 256;
+  // the 3D march's tile and chunk: as asked for, the rest by what it is expected to cost
+  int asked = -1;
+  for (int k = 0; c.tile[0] > 0 && s->es == 4 && k < FUSED_NTILES; k++) {
+    int tx, ty;
+    fused_tile_cells(k, tx, ty);
+    if (tx == c.tile[0] && ty == c.tile[1]) asked = k;
   }
-  if (c.tile[2] > 0) s->zc = c.tile[2];
-  if (s->zc > c.n[2]) s->zc = c.n[2];
+  const auto shapes = shapes_of(c, cus, asked, c.tile[2]);
+  s->tile = shapes.empty() ? asked : shapes[0].tile;
+  s->zc = shapes.empty() ? std::min(c.tile[2] > 0 ? c.tile[2] : 32, c.n[2]) : shapes[0].zc;
   if (s->fused && c.n[2] == 1) {
     const int isen = c.isentropic ? 1 : 0;
     s->eops = s->es == 8 ? ens_ops_f64(c.limiter, c.riemann, isen) : ens_ops_f32(c.limiter, c.riemann, isen);
     s->flat2d = s->eops.fused != nullptr;
-    if (s->es == 8) s->etile = ENS_20x20;   // the FP64 2D kernel's one tile
   }
+  s->etile = s->es == 8 ? ENS_20x20 : ens_default_tile(c.n[0], c.n[1], c.limiter == SHX_LIM_KOREN);
+  s->rows_fit = ens_fit_rows(&c.n[0], &c.n[1], 1, 4 * cus);
+  if (c.tile[0] == ENS_STRIP && c.tile[1] > 0) s->rows_fit = c.tile[1];
   if (s->flat2d && s->es == 4 && c.tile[0] > 0)
-    for (int k = 0; k < ENS_NTILES; k++) {
+    for (int k = ENS_NTILES - 1; k >= 0; k--) {
       int tx, ty;
-      ens_tile_cells(k, tx, ty);
+      ens_tile_cells(k, s->rows_fit, tx, ty);
       if (tx == c.tile[0] && ty == c.tile[1]) s->etile = k;
     }
 
@@ -453,13 +461,11 @@ int shx_create(const shx_config* cfg, shx_sim** out) {
        alloc((void**)&s->diag_out, DIAG_CH * 8);
   std::vector<EnsTile> lists[ENS_NTILES];
   if (s->flat2d) {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device) != hipSuccess || cus < 1) cus = 256;
     s->egrid = 4 * cus;
     ok = ok && alloc(&s->einst, s->es == 8 ? sizeof(EnsInst<double>) : sizeof(EnsInst<float>));
     for (int k = 0; k < ENS_NTILES; k++) {
       int tx, ty;
-      ens_tile_cells(k, tx, ty);
+      ens_tile_cells(k, s->rows_fit, tx, ty);
       for (int y0 = 0; y0 < c.n[1]; y0 += ty)
         for (int x0 = 0; x0 < c.n[0]; x0 += tx) lists[k].push_back(EnsTile{0, x0, y0, std::min(y0 + ty, c.n[1])});
       s->entiles[k] = (int)lists[k].size();
@@ -658,10 +664,9 @@ int shx_profile(shx_sim* s, int steps, double ms[5]) {
 
 int shx_kernel_name(shx_sim* s, char* buf, size_t len) {
   if (!s || !buf || len == 0) return fail(SHX_EINVAL, "bad argument");
-  // threads by role: the FP32 tiles 32 x 16, 32 x 8 and 16 x 16
-  const bool roles = s->es == 4 && (s->tile == FUSED_R32x16 || s->tile == FUSED_R32x8 || s->tile == FUSED_20x20);
-  const bool rows = s->etile == ENS_ROWS8 || s->etile == ENS_ROWS16 || s->etile == ENS_ROWS32;
-  const char* fused = s->flat2d ? (rows ? "k_ens_rows" : "k_ens_fused") : (roles ? "k_fused_r" : "k_fused");
+  // threads by role: tiles of 32 x 16, 32 x 8 and 16 x 16
+  const bool roles = s->tile == FUSED_R32x16 || s->tile == FUSED_R32x8 || s->tile == FUSED_20x20;
+  const char* fused = s->flat2d ? (ens_is_rows(s->etile) ? "k_ens_rows" : "k_ens_fused") : (roles ? "k_fused_r" : "k_fused");
   snprintf(buf, len, "%s", !s->fused ? "k_update" : fused);
   return SHX_OK;
 }
@@ -669,6 +674,7 @@ int shx_kernel_name(shx_sim* s, char* buf, size_t len) {
 int shx_autotune(shx_sim* s, int reps, int chosen[3]) {
   if (!s) return fail(SHX_EINVAL, "null sim");
   if (!s->fused || s->es == 8) {
+    // FP64 has one tile, its chunk chosen when the sim is made
     if (chosen) { chosen[0] = 0; chosen[1] = 0; chosen[2] = s->zc; }
     return SHX_OK;
   }
@@ -691,36 +697,57 @@ int shx_autotune(shx_sim* s, int reps, int chosen[3]) {
     HIPCHK(hipMemcpyAsync(s->clk, clk_saved.data(), clk_saved.size(), hipMemcpyHostToDevice, s->stream));
     return SHX_OK;
   };
-  const int tiles3[] = {FUSED_R32x16, FUSED_R32x8, FUSED_32x32, FUSED_32x16, FUSED_20x20};
-  const int tiles2[] = {ENS_32x32, ENS_32x16, ENS_20x20, ENS_ROWS8, ENS_ROWS16, ENS_ROWS32};
-  std::vector<int> tiles = s->flat2d ? std::vector<int>(tiles2, tiles2 + 6) : std::vector<int>(tiles3, tiles3 + 5);
-  const int zcs[] = {16, 32, 64, 128};
+  // candidates: the 2D shapes, or the three likeliest chunks of each 3D tile
+  std::vector<FusedShape> cands;
+  if (s->flat2d) {
+    for (int k : {ENS_32x32, ENS_32x16, ENS_20x20, ENS_ROWS8, ENS_ROWS16, ENS_ROWS32, ENS_ROWSFIT})
+      cands.push_back(FusedShape{k, 1, 0});
+  } else {
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->cfg.device) != hipSuccess || cus < 1) cus = 256;
+    for (int k : {FUSED_R32x16, FUSED_R32x8, FUSED_20x20}) {
+      const auto of = shapes_of(s->cfg, cus, k, 0);
+      cands.insert(cands.end(), of.begin(), of.begin() + std::min<size_t>(of.size(), 3));
+    }
+  }
+  // the shape in use goes first, and another has to beat it by more than timing noise
   double best = 1e30;
   int bt = s->flat2d ? s->etile : s->tile, bz = s->zc;
+  cands.insert(cands.begin(), FusedShape{bt, bz, 0});
   Launch L = launch_of(s);
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
-  for (int ti : tiles)
-    for (int z : zcs) {
-      // the 2D kernels have no plane chunk: one candidate per tile; a chunk beyond the grid's
-      // planes is the whole grid, timed once
-      if (s->flat2d ? z != zcs[0] : (z > s->cfg.n[2] && z != zcs[0])) continue;
-      int rc = restore();
-      if (rc) return rc;
-      // a warm step, then `reps` timed steps (each with its boundary planes' half steps)
-      for (int r = 0, p = start; r <= reps; r++, p = 1 - p) {
-        if (r == 1) HIPCHK(hipEventRecord(e0, s->stream));
-        if (s->zbc) s->ops.zplanes(L, s->U1[p], s->U2[p], s->PA, s->PB, clock_refs(s, p));
-        enqueue_fused(s, p, ti, z, false);
-      }
-      HIPCHK(hipEventRecord(e1, s->stream));
-      HIPCHK(hipEventSynchronize(e1));
-      HIPCHK(hipGetLastError());
-      float t;
-      HIPCHK(hipEventElapsedTime(&t, e0, e1));
-      if (t < best) { best = t; bt = ti; bz = z; }
+  // milliseconds a step: from the saved state a warm step, then n timed ones (each with its
+  // boundary planes' half steps)
+  auto timed = [&](int ti, int z, int n, double* ms) -> int {
+    int rc = restore();
+    if (rc) return rc;
+    for (int r = 0, p = start; r <= n; r++, p = 1 - p) {
+      if (r == 1) HIPCHK(hipEventRecord(e0, s->stream));
+      if (s->zbc) s->ops.zplanes(L, s->U1[p], s->U2[p], s->PA, s->PB, clock_refs(s, p));
+      enqueue_fused(s, p, ti, z, false);
     }
+    HIPCHK(hipEventRecord(e1, s->stream));
+    HIPCHK(hipEventSynchronize(e1));
+    HIPCHK(hipGetLastError());
+    float t;
+    HIPCHK(hipEventElapsedTime(&t, e0, e1));
+    *ms = t / n;
+    return SHX_OK;
+  };
+  // (the first series only wakes the device and tells how many steps of a small grid to time)
+  double ms;
+  int rc = timed(bt, bz, reps, &ms);
+  if (rc) return rc;
+  const int n = std::max(reps, (int)std::min(32.0, 0.3 / std::max(ms, 1e-3)));
+  for (size_t i = 0; i < cands.size(); i++) {
+    const int ti = cands[i].tile, z = cands[i].zc;
+    if (i > 0 && ti == cands[0].tile && z == cands[0].zc) continue;
+    rc = timed(ti, z, n, &ms);
+    if (rc) return rc;
+    if (ms < best) { best = i == 0 ? 0.97 * ms : ms; bt = ti; bz = z; }
+  }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (s->flat2d) {
@@ -729,7 +756,7 @@ int shx_autotune(shx_sim* s, int reps, int chosen[3]) {
     s->tile = bt;
     s->zc = std::min(bz, s->cfg.n[2]);
   }
-  int rc = restore();
+  rc = restore();
   if (rc) return rc;
   HIPCHK(hipStreamSynchronize(s->stream));
   s->cur = start;
@@ -738,7 +765,7 @@ int shx_autotune(shx_sim* s, int reps, int chosen[3]) {
   rc = build_graphs(s);
   if (rc) return rc;
   if (chosen) {
-    if (s->flat2d) ens_tile_cells(bt, chosen[0], chosen[1]);
+    if (s->flat2d) ens_tile_cells(bt, s->rows_fit, chosen[0], chosen[1]);
     else fused_tile_cells(bt, chosen[0], chosen[1]);
     chosen[2] = s->zc;
   }

@@ -32,10 +32,12 @@ struct shx_ens {
   unsigned int* epoch = nullptr;
   int cur = 0;
   int tile = ENS_ROWS16;
+  int rows_fit = 16;              // the rows of ENS_ROWSFIT
   int grid = 512;
   bool rates_stale = true;
   EnsOps ops{};
-  hipGraphExec_t graph[2] = {nullptr, nullptr};
+  // [parity][1, 2 or 8 steps]: small grids' steps are shorter than a graph launch's host cost
+  hipGraphExec_t graph[2][3] = {{nullptr, nullptr, nullptr}, {nullptr, nullptr, nullptr}};
 };
 
 namespace {
@@ -57,19 +59,22 @@ void enqueue_step(shx_ens* e, int p) { enqueue_fused(e, p, e->tile); }
 
 void destroy_graphs(shx_ens* e) {
   for (int p = 0; p < 2; p++)
-    if (e->graph[p]) { (void)hipGraphExecDestroy(e->graph[p]); e->graph[p] = nullptr; }
+    for (int k = 0; k < 3; k++)
+      if (e->graph[p][k]) { (void)hipGraphExecDestroy(e->graph[p][k]); e->graph[p][k] = nullptr; }
 }
 
 int build_graphs(shx_ens* e) {
   destroy_graphs(e);
-  for (int p = 0; p < 2; p++) {
-    hipGraph_t g;
-    HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_step(e, p);
-    HIPCHK(hipStreamEndCapture(e->stream, &g));
-    HIPCHK(hipGraphInstantiate(&e->graph[p], g, nullptr, nullptr, 0));
-    HIPCHK(hipGraphDestroy(g));
-  }
+  for (int p = 0; p < 2; p++)
+    for (int k = 0; k < 3; k++) {
+      hipGraph_t g;
+      HIPCHK(hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal));
+      const int n = k == 0 ? 1 : (k == 1 ? 2 : 8);
+      for (int i = 0; i < n; i++) enqueue_step(e, (p + i) & 1);
+      HIPCHK(hipStreamEndCapture(e->stream, &g));
+      HIPCHK(hipGraphInstantiate(&e->graph[p][k], g, nullptr, nullptr, 0));
+      HIPCHK(hipGraphDestroy(g));
+    }
   return SHX_OK;
 }
 
@@ -79,7 +84,9 @@ int refresh_rates(shx_ens* e) {
   if (!e->rates_stale) return SHX_OK;
   // every instance's epochs restart at 0: its rate into its slot 0
   HIPCHK(hipMemsetAsync(e->slot, 0, block_bytes(e) - clock_slots_at(e->count, e->es), e->stream));
-  e->ops.rates(e->stream, e->inst, e->tiles[e->tile], e->ntiles[e->tile], e->tile, e->U1[e->cur], e->U2[e->cur],
+  int tx, ty;
+  ens_tile_cells(e->tile, e->rows_fit, tx, ty);
+  e->ops.rates(e->stream, e->inst, e->tiles[e->tile], e->ntiles[e->tile], tx, ty, e->U1[e->cur], e->U2[e->cur],
                e->slot, 3);
   HIPCHK(hipGetLastError());
   e->rates_stale = false;
@@ -167,23 +174,25 @@ int shx_ens_create(const shx_config* cfg, int count, const int* sizes, shx_ens**
   e->es = c.precision == 64 ? 8 : 4;
   e->count = count;
   e->ops = ops;
-  e->tile = e->es == 8 ? ENS_20x20 : ENS_ROWS16;
-  // a tile asked for by its cells (tile[0] x tile[1]); FP64 has the one
-  for (int k = 0; c.tile[0] > 0 && e->es == 4 && k < ENS_NTILES; k++) {
-    int tx, ty;
-    ens_tile_cells(k, tx, ty);
-    if (tx == c.tile[0] && ty == c.tile[1]) e->tile = k;
-  }
   for (int i = 0; i < count; i++) {
     e->nx.push_back(sizes[2 * i]);
     e->ny.push_back(sizes[2 * i + 1]);
     e->off.push_back((long long)e->ncell);
     e->ncell += (size_t)sizes[2 * i] * sizes[2 * i + 1];
   }
-  {
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device) != hipSuccess || cus < 1) cus = 256;
-    e->grid = 4 * cus;
+  int cus = 0;
+  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device) != hipSuccess || cus < 1) cus = 256;
+  e->grid = 4 * cus;
+  e->rows_fit = ens_fit_rows(e->nx.data(), e->ny.data(), count, 4 * cus);
+  // untuned: strips from about a million cells on, where they fill the chip, else 28 x 12 tiles
+  // (24 grids up to 512^2, 2.4 M cells: 61 against 76 us per step; 12 up to 200^2, 0.16 M: 23 against 16.5)
+  e->tile = e->es == 8 ? ENS_20x20 : (e->ncell >= 800000 ? ENS_ROWSFIT : ENS_32x16);
+  // a tile asked for by its cells (tile[0] x tile[1]); FP64 has the one
+  if (e->es == 4 && c.tile[0] == ENS_STRIP && c.tile[1] > 0) e->rows_fit = c.tile[1];
+  for (int k = ENS_NTILES - 1; c.tile[0] > 0 && e->es == 4 && k >= 0; k--) {
+    int tx, ty;
+    ens_tile_cells(k, e->rows_fit, tx, ty);
+    if (tx == c.tile[0] && ty == c.tile[1]) e->tile = k;
   }
   auto alloc = [&](void** p, size_t b) { return hipMalloc(p, b) == hipSuccess; };
   bool ok = hipStreamCreateWithFlags(&e->stream, hipStreamNonBlocking) == hipSuccess;
@@ -199,7 +208,7 @@ int shx_ens_create(const shx_config* cfg, int count, const int* sizes, shx_ens**
   std::vector<EnsTile> lists[ENS_NTILES];
   for (int k = 0; k < ENS_NTILES; k++) {
     int tx, ty;
-    ens_tile_cells(k, tx, ty);
+    ens_tile_cells(k, e->rows_fit, tx, ty);
     for (int i : order)
       for (int y0 = 0; y0 < e->ny[i]; y0 += ty)
         for (int x0 = 0; x0 < e->nx[i]; x0 += tx) lists[k].push_back(EnsTile{i, x0, y0, std::min(y0 + ty, e->ny[i])});
@@ -261,8 +270,10 @@ int shx_ens_step(shx_ens* e, int count) {
   if (!e || count < 0) return fail(SHX_EINVAL, "bad argument");
   int rc = refresh_rates(e);
   if (rc) return rc;
-  for (int n = 0; n < count; n++) {
-    HIPCHK(hipGraphLaunch(e->graph[e->cur], e->stream));
+  for (; count >= 8; count -= 8) HIPCHK(hipGraphLaunch(e->graph[e->cur][2], e->stream));
+  for (; count >= 2; count -= 2) HIPCHK(hipGraphLaunch(e->graph[e->cur][1], e->stream));
+  if (count == 1) {
+    HIPCHK(hipGraphLaunch(e->graph[e->cur][0], e->stream));
     e->cur = 1 - e->cur;
   }
   return SHX_OK;
@@ -337,7 +348,7 @@ int shx_ens_autotune(shx_ens* e, int reps, int chosen[2]) {
   HIPCHK(hipEventCreate(&e1));
   double best = 1e30;
   int bt = e->tile;
-  const int cands[] = {ENS_32x32, ENS_32x16, ENS_20x20, ENS_ROWS8, ENS_ROWS16, ENS_ROWS32};
+  const int cands[] = {ENS_32x32, ENS_32x16, ENS_20x20, ENS_ROWS8, ENS_ROWS16, ENS_ROWS32, ENS_ROWSFIT};
   for (int k : cands) {
     if (e->es == 8 && k != ENS_20x20) continue;
     rc = restore();
@@ -364,7 +375,7 @@ int shx_ens_autotune(shx_ens* e, int reps, int chosen[2]) {
   (void)hipFree(b1); (void)hipFree(b2); (void)hipFree(cs);
   rc = build_graphs(e);
   if (rc) return rc;
-  if (chosen) ens_tile_cells(bt, chosen[0], chosen[1]);
+  if (chosen) ens_tile_cells(bt, e->rows_fit, chosen[0], chosen[1]);
   return SHX_OK;
 }
 

@@ -2,6 +2,7 @@
 // table per (precision, limiter, Riemann solver, isentropic) combination.
 #pragma once
 #include <algorithm>
+#include <vector>
 #include "diag.hpp"
 #include "hydro.hpp"
 
@@ -14,8 +15,9 @@ struct Launch {
 };
 
 // Column tiles of the fused kernel: k_fused's (block BX x BY threads in raster order, tile
-// (BX - 4) x (BY - 4) cells) and k_fused_r's (threads by role, tiles of 32 x 16 or 32 x 8 cells).
-// FUSED_20x20 is a 16 x 16 cell tile: k_fused_r's in FP32, k_fused's (the only FP64 tile) in FP64.
+// (BX - 4) x (BY - 4) cells) and k_fused_r's (threads by role, tiles of 32 x 16, 32 x 8 or, as
+// FUSED_20x20, 16 x 16 cells: the only one in FP64). k_fused is slower on every grid measured; it
+// is run where a plane exceeds the 4 GiB that k_fused_r addresses, and on request.
 enum { FUSED_20x20 = 0, FUSED_32x16 = 1, FUSED_32x32 = 2, FUSED_R32x16 = 3, FUSED_R32x8 = 4, FUSED_NTILES = 5 };
 // cells per tile along x and y
 inline void fused_tile_cells(int tile, int& tx, int& ty) {
@@ -26,6 +28,46 @@ inline void fused_tile_cells(int tile, int& tx, int& ty) {
     case FUSED_R32x16: tx = 32; ty = 16; break;
     default: tx = 32; ty = 8; break;
   }
+}
+
+// A launch of the 3D march: tile and planes per chunk, and what it is expected to cost, in planes of
+// a 32 x 16 tile.
+struct FusedShape { int tile, zc; double cost; };
+
+// The shapes of k_fused_r for an nx x ny x nz grid on `cus` CUs, cheapest first. A workgroup marches
+// zc planes and about 2.5 planes' worth before and after; workgroups fill the chip's slots in turn,
+// so the step takes the work of the slot with the most. Per plane of a tile, with as many
+// workgroups on a CU as fit (two of 32 x 8 and 16 x 16; one of 32 x 16, and of 16 x 16 with
+// Koren's edges) and with one, against one 32 x 16: measured at 256^3 (MC 2.63 us a plane, Koren +
+// isentropic 5.05) and at 48^3 to 64^3. tile, zc > 0 (FP64: the tile is given): only those.
+inline std::vector<FusedShape> fused_shapes(int nx, int ny, int nz, int cus, bool fp64, bool koren, int tile, int zc) {
+  struct Cost { int tile, fit; double alone, full; };
+  const Cost sym[3] = {{FUSED_R32x16, 1, 1.0, 1.0}, {FUSED_R32x8, 2, 0.80, 1.09}, {FUSED_20x20, 2, 0.78, 1.09}};
+  const Cost asym[3] = {{FUSED_R32x16, 1, 1.0, 1.0}, {FUSED_R32x8, 2, 0.85, 1.5}, {FUSED_20x20, 1, 0.69, 0.69}};
+  std::vector<FusedShape> out;
+  for (int k = 0; k < 3; k++) {
+    Cost c = koren ? asym[k] : sym[k];
+    if (fp64) {
+      if (c.tile != FUSED_20x20) continue;
+      c.fit = 1;
+      c.full = c.alone;
+    }
+    if (tile >= 0 && c.tile != tile) continue;
+    int tx, ty, last = 0;
+    fused_tile_cells(c.tile, tx, ty);
+    const long long tiles = (long long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty);
+    for (int chunks = 1; chunks <= nz; chunks++) {
+      const int z = zc > 0 ? std::min(zc, nz) : (nz + chunks - 1) / chunks;
+      if (z == last) continue;
+      last = z;
+      const long long n = tiles * ((nz + z - 1) / z), slots = (long long)cus * c.fit;
+      const double each = n <= cus ? c.alone : c.full * (double)((n + slots - 1) / slots);
+      out.push_back(FusedShape{c.tile, z, each * (z + 2.5)});
+      if (zc > 0) break;
+    }
+  }
+  std::stable_sort(out.begin(), out.end(), [](const FusedShape& a, const FusedShape& b) { return a.cost < b.cost; });
+  return out;
 }
 
 // The clocks of a fused step (the step kernel takes its own clock pass, StepClock in

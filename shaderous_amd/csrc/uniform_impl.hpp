@@ -24,10 +24,26 @@
 namespace shx {
 
 // ---------------- reductions ----------------
-template <typename T>
-__device__ __forceinline__ T wave_max(T v) {
+// The largest of the wave's values (none negative), in every lane. In FP32 a prefix maximum by row
+// shifts and broadcasts in the lanes' own registers (a lane without a source reads 0), of which the
+// last active lane holds the whole (a workgroup's last wave may be part of one): a dozen VALU
+// instructions, where the butterfly of shuffles waits six times on the LDS unit.
+__device__ __forceinline__ double wave_max(double v) {
   for (int o = 32; o > 0; o >>= 1) v = tmax(v, __shfl_xor(v, o, 64));
   return v;
+}
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_zero(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, ROWS, 0xf, false));
+}
+__device__ __forceinline__ float wave_max(float v) {
+  v = raw_max(v, dpp_or_zero<0x111, 0xf>(v));   // row_shr 1, 2, 4, 8: within the rows of 16 lanes
+  v = raw_max(v, dpp_or_zero<0x112, 0xf>(v));
+  v = raw_max(v, dpp_or_zero<0x114, 0xf>(v));
+  v = raw_max(v, dpp_or_zero<0x118, 0xf>(v));
+  v = raw_max(v, dpp_or_zero<0x142, 0xa>(v));   // row_bcast 15 into rows 1 and 3
+  v = raw_max(v, dpp_or_zero<0x143, 0xc>(v));   // row_bcast 31 into rows 2 and 3
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63 - __builtin_clzll(__ballot(1))));
 }
 
 // atomicMax on a rate slot, which only grows during a launch (it is cleared before the launch

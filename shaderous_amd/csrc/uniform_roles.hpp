@@ -97,10 +97,9 @@ __device__ __forceinline__ void role_column(int t, int& cx, int& cy) {
 template <typename T> struct Vec2;
 template <> struct Vec2<float> { using type = float2; };
 template <> struct Vec2<double> { using type = double2; };
+// Columns' values in LDS as 4- and 2-vectors (structure of arrays over NT columns; offsets in T)
 template <typename T, int NT>
-struct PlaneLds {
-  static constexpr int QA = 0, QB = 4 * NT, QN = 6 * NT;      // + QN: the other plane
-  static constexpr int SX = 12 * NT, SY = 20 * NT, SK = 28 * NT, FX = 29 * NT, FY = 37 * NT, SIZE = 45 * NT;
+struct ColumnLds {
   using V4 = T4<T>;
   using V2 = typename Vec2<T>::type;
   // A column's byte offsets in the arrays of 4-, 2- and 1-vectors, each kept as a value of its own
@@ -127,12 +126,12 @@ struct PlaneLds {
   static __device__ __forceinline__ void put_prim(T* L, int q, const At& t, const Prim<T>& w) {
     V4 a; a.x = w.rho; a.y = w.vx; a.z = w.vy; a.w = w.vz;
     V2 b; b.x = w.p; b.y = w.s;
-    ref<V4>(L, q + QA, t.a) = a;
-    ref<V2>(L, q + QB, t.b) = b;
+    ref<V4>(L, q, t.a) = a;
+    ref<V2>(L, q + 4 * NT, t.b) = b;
   }
   static __device__ __forceinline__ Prim<T> prim(T* L, int q, const At& t) {
-    const V4 a = ref<V4>(L, q + QA, t.a);
-    const V2 b = ref<V2>(L, q + QB, t.b);
+    const V4 a = ref<V4>(L, q, t.a);
+    const V2 b = ref<V2>(L, q + 4 * NT, t.b);
     Prim<T> w;
     w.rho = a.x; w.vx = a.y; w.vy = a.z; w.vz = a.w; w.p = b.x; w.s = b.y; w.cs = T(0);
     return w;
@@ -143,12 +142,12 @@ struct PlaneLds {
     ref<V4>(L, s, t.a) = a;
     ref<V4>(L, s + 4 * NT, t.a) = b;
   }
-  static __device__ __forceinline__ void put_shock(T* L, const At& t, T shock) { ref<T>(L, SK, t.c) = shock; }
-  static __device__ __forceinline__ SideData<T> side(T* L, int s, const At& t) {
+  static __device__ __forceinline__ void put_shock(T* L, int k, const At& t, T shock) { ref<T>(L, k, t.c) = shock; }
+  static __device__ __forceinline__ SideData<T> side(T* L, int s, int k, const At& t) {
     const V4 a = ref<V4>(L, s, t.a), b = ref<V4>(L, s + 4 * NT, t.a);
     SideData<T> d;
     d.rho = a.x; d.vx = a.y; d.vy = a.z; d.vz = a.w; d.p = b.x; d.s = b.y; d.hrho = b.z; d.hp = b.w;
-    d.shock = ref<T>(L, SK, t.c);
+    d.shock = ref<T>(L, k, t.c);
     return d;
   }
   static __device__ __forceinline__ void put_flux(T* L, int f, const At& t, const Flux<T>& F) {
@@ -186,6 +185,13 @@ __device__ __forceinline__ void plane_store(T4<T>* base, unsigned int off, T4<T>
 #pragma unroll
   for (int i = 0; i < (int)(sizeof(T4<T>) / 16); i++) __builtin_amdgcn_raw_buffer_store_b128(k.w[i], r, off + 16 * i, 0, 0);
 }
+
+// k_fused_r's planes: primitives of two planes (QN apart), sides, shock flags, fluxes
+template <typename T, int NT>
+struct PlaneLds : ColumnLds<T, NT> {
+  static constexpr int QN = 6 * NT, SX = 12 * NT, SY = 20 * NT, SK = 28 * NT, FX = 29 * NT, FY = 37 * NT,
+                       SIZE = 45 * NT;
+};
 
 // The net inflow of a plane's x and y faces, and with the z faces' (lower lo, upper hi)
 template <typename T>
@@ -438,7 +444,7 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile
       }
       PL::put_side(L, PL::SX, t, side_of(P, h, e.xu, T(1)));
       PL::put_side(L, PL::SY, t, side_of(P, h, e.yu, T(1)));
-      PL::put_shock(L, t, h.shock);
+      PL::put_shock(L, PL::SK, t, h.shock);
       PL::put_prim(L, buf(c + 1), t, pp);
       cs = pp.cs;
       __builtin_amdgcn_sched_barrier(0);
@@ -451,10 +457,10 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile
       __builtin_amdgcn_sched_barrier(0);
       load(c + 2);
       __syncthreads();
-      const Flux<T> Fx = face_from_sides<T, RS>(P, PL::side(L, PL::SX, t.off(-1)), side_of(P, h, e.xd, T(-1)), 0);
+      const Flux<T> Fx = face_from_sides<T, RS>(P, PL::side(L, PL::SX, PL::SK, t.off(-1)), side_of(P, h, e.xd, T(-1)), 0);
       PL::put_flux(L, PL::FX, t, Fx);
       __builtin_amdgcn_sched_barrier(0);
-      const Flux<T> Fy = face_from_sides<T, RS>(P, PL::side(L, PL::SY, t.off(-BX)), side_of(P, h, e.yd, T(-1)), 1);
+      const Flux<T> Fy = face_from_sides<T, RS>(P, PL::side(L, PL::SY, PL::SK, t.off(-BX)), side_of(P, h, e.yd, T(-1)), 1);
       PL::put_flux(L, PL::FY, t, Fy);
       __syncthreads();
       const Flux<T> xh = PL::flux(L, PL::FX, t.off(1)), yh = PL::flux(L, PL::FY, t.off(BX));
@@ -503,7 +509,7 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile
         const Half<T> h = half_of(buf(c), buf(c - 1), cs, pp, e);
         PL::put_side(L, PL::SX, t, side_of(P, h, e.xu, T(1)));
         PL::put_side(L, PL::SY, t, side_of(P, h, e.yu, T(1)));
-        PL::put_shock(L, t, h.shock);
+        PL::put_shock(L, PL::SK, t, h.shock);
         const SideData<T> sxl = side_of(P, h, e.xd, T(-1)), syl = side_of(P, h, e.yd, T(-1));
         lo = ax ? sxl : syl;
       }
@@ -511,7 +517,7 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile
       cs = pp.cs;
       __syncthreads();
       if (face) {
-        const Flux<T> F = face_from_sides_rt<T, RS>(P, PL::side(L, ax ? PL::SX : PL::SY, t.off(ax ? -1 : -BX)), lo, ax ? 0 : 1);
+        const Flux<T> F = face_from_sides_rt<T, RS>(P, PL::side(L, ax ? PL::SX : PL::SY, PL::SK, t.off(ax ? -1 : -BX)), lo, ax ? 0 : 1);
         PL::put_flux(L, ax ? PL::FX : PL::FY, t, F);
       }
       __syncthreads();

@@ -1,0 +1,69 @@
+"""The launch shapes an untuned sim takes (by the grid's size, scheme and precision) and every
+strip height of the row march give the plain path's bits, on an MI355X: grids from two cells an
+axis to past a tile's edge, one and several chunks of planes, periodic and walled. Bit for bit, so
+there is no tolerance."""
+import numpy as np
+import pytest
+
+from shaderous_amd import problems
+from shaderous_amd.ensemble import Ensemble
+from shaderous_amd.sim import Sim, SimConfig, config_for
+
+pytestmark = pytest.mark.gpu
+
+
+def random_flow(n, bc, limiter, seed=1):
+    rng = np.random.default_rng(seed)
+    shape = n[::-1]
+    return problems.Problem(id="random", n=n, box=1.0, gamma=1.4, bc_lo=bc, bc_hi=bc, cfl=0.3, limiter=limiter,
+                            isentropic=limiter == "koren",
+                            prims={"rho": 1 + 0.3 * rng.random(shape), "vx": 0.5 * rng.normal(size=shape),
+                                   "vy": 0.5 * rng.normal(size=shape), "p": 1 + 0.5 * rng.random(shape),
+                                   "vz": 0.5 * rng.normal(size=shape) if n[2] > 1 else np.zeros(shape),
+                                   "s": rng.random(shape)})
+
+
+def runs_alike(pb, precision, steps=3, **fused):
+    out = []
+    for path, over in (("plain", {}), ("fused", fused)):
+        with Sim(config_for(pb, path=path, precision=precision, **over)) as sim:
+            sim.set_state(*pb.state(np.float64 if precision == 64 else np.float32))
+            sim.step(steps)
+            out.append((*sim.read_state(), sim.clock()))
+    return all(np.array_equal(a, b) for a, b in zip(*out))
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("limiter", ["mc", "koren"])
+@pytest.mark.parametrize("n,bc", [((2, 2, 2), (0, 0, 0)), ((3, 17, 2), (0, 0, 0)), ((33, 16, 5), (0, 0, 0)),
+                                  ((16, 33, 67), (2, 1, 1)), ((70, 15, 9), (1, 2, 0)), ((5, 4, 40), (2, 2, 2)),
+                                  ((64, 48, 30), (0, 0, 1)), ((2, 5, 1), (0, 0, 0)), ((17, 61, 1), (1, 2, 0)),
+                                  ((260, 130, 1), (2, 1, 0))])
+def test_untuned_shapes_give_the_plain_bits(n, bc, limiter, precision):
+    assert runs_alike(random_flow(n, bc, limiter), precision)
+
+
+@pytest.mark.parametrize("rows", [1, 5, 13, 64])
+@pytest.mark.parametrize("bc", [(0, 0, 0), (2, 1, 0)])
+def test_strips_of_any_height_give_the_plain_bits(rows, bc):
+    assert runs_alike(random_flow((130, 61, 1), bc, "koren"), 32, tile=(60, rows, 1))
+
+
+def test_runs_of_steps_of_an_ensemble_equal_single_steps():
+    """A run of steps in one call goes out eight, two and one to a graph: the single steps' bits."""
+    cfg = SimConfig(n=(64, 64, 1), ndim=2, dx=1.0 / 64, gamma=1.4, bc_lo=(1, 1, 0), bc_hi=(1, 1, 0), limiter="mc",
+                    isentropic=False, cfl=0.4)
+    out = []
+    for counts in ((19, 3), (1,) * 22):
+        ens = Ensemble(cfg, [(64, 64), (100, 37)])
+        for i, n in enumerate((64, 100)):
+            pb = problems.riemann_quadrants(n, 7 + i)
+            u1, u2 = pb.state()
+            cells = (64 * 64, 100 * 37)[i]
+            ens.set_state(i, u1[:cells], u2[:cells])
+        for c in counts:
+            ens.step(c)
+        out.append([ens.read_state(i) for i in range(2)])
+        ens.destroy()
+    for a, b in zip(*out):
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
