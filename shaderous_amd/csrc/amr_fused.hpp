@@ -26,10 +26,12 @@
 // ever hold a value: threads 0-255 the 16 x 16 cell columns, 256-319 the 64 face-ghost columns
 // of ring 1, 320-383 the 64 of ring 2 (x or y = -2 or 17, the other in range). The 16 remaining
 // columns (both x and y outside the cells) are edges or corners at every plane: zero, as in the
-// atlas. So the cell waves never diverge on ghost work. LDS holds the plane data in raster order
-// of the 20 x 20 columns, fluxes apart from sides (the role-tiled uniform kernel's layout, 73.6 KB
-// per block in FP32), so a plane needs two barriers: after the half steps, after the fluxes.
-// Two blocks share a 12-wave workgroup (one per CU at up to 168 VGPRs).
+// atlas. So the cell waves never diverge on ghost work, and each role runs its own loop over the
+// planes (the uniform march's form, uniform_roles.hpp, with its LDS layout: 72 KB per block in
+// FP32), with two barriers per plane: after the half steps, after the fluxes. The ghost planes
+// z = -1 and 16 concern the cell waves alone. Two blocks share a 12-wave workgroup (one per CU at
+// up to 168 VGPRs), whose waves go to the SIMDs in turn: two cell waves and one ghost or load wave
+// on each.
 #pragma once
 #include "amr_impl.hpp"
 
@@ -286,7 +288,11 @@ __global__ void k_amr_queue_start(int* qctl) {
 }
 
 // Launch bound: twelve waves per workgroup (two blocks), one workgroup per CU in FP32 (three
-// waves per SIMD: up to 168 VGPRs); six waves (one block) in FP64
+// waves per SIMD: up to 168 VGPRs); six waves (one block) in FP64.
+// Bound by VALU issue and, on a few hundred leaves, by how evenly the pairs divide among the CUs.
+// On the 3D blast (8^3 root blocks, two refinements, 1618 leaves, MC, HLLC): 462 us with one loop
+// for all roles, ghost cases chosen by lane in it; 342 us with a loop per role (-26%). The rate's
+// division is by the block (a quotient by one dx keeps the order, so its maximum has the same bits).
 template <typename T, int LIM, int RS, bool ISEN>
 __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) == 4 ? 3 : 1)) void k_amr_fused(
     Params<T> P, const int* __restrict__ tab, const int* __restrict__ list, int count,
@@ -296,25 +302,25 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     const T4<T>* __restrict__ U2, T4<T>* __restrict__ O1, T4<T>* __restrict__ O2, const T* __restrict__ clk,
     unsigned long long* next_slot) {
   constexpr int NT = AF_NT, BX = AF_SIDE, AF_PAIR = af_pair<T>();
-  using LY = RoleLayout<NT>;
-  __shared__ T LL[AF_PAIR * LY::SIZE];
+  using PL = PlaneLds<T, NT>;
+  __shared__ T4<T> LL[AF_PAIR * PL::SIZE / 4];
   __shared__ T red[AF_PAIR * AF_THREADS / 64];
   __shared__ int q_pair;
   const int epoch = qctl[AMR_Q_EPOCH];
-  // which of the workgroup's two blocks this thread marches, and its thread index there
-  const int half = threadIdx.x >= AF_THREADS;
+  // which of the workgroup's two blocks this wave marches (a scalar), and its thread index there
+  const int gwave = __builtin_amdgcn_readfirstlane(threadIdx.x) >> 6;
+  const int half = gwave >= AF_THREADS / 64;
   const int tid = threadIdx.x - AF_THREADS * half;
-  T* L = LL + half * LY::SIZE;
+  T* const L = reinterpret_cast<T*>(LL) + half * PL::SIZE;
   int x, y;
   af_column(tid, x, y);
-  const int t = (y + 2) * BX + (x + 2);                  // raster index of the column in LDS
+  const typename PL::At t = PL::at((y + 2) * BX + (x + 2));   // the column, in raster order
   // the columns no thread owns are edges at every plane: zero in both plane slots, for good
   for (int i = tid; i < 12 * NT; i += AF_THREADS) L[i] = T(0);
-  // roles by wave (uniform branches): waves 0-3 the cell columns, wave 4 the face ghosts of
-  // ring 1, wave 5 ring 2 (loads only)
-  const int wave = __builtin_amdgcn_readfirstlane(tid) >> 6;
-  const bool cells0 = wave < 4, ghosts0 = wave == 4;
-  // a face-ghost lane's side: 0 -x, 1 +x, 2 -y, 3 +y
+  // roles by wave: 0-3 the cell columns, 4 the face ghosts of ring 1, 5 ring 2 (loads only)
+  const int wave = gwave - (AF_THREADS / 64) * half;
+  const bool cells = wave < 4, ghosts = wave == 4;
+  // a ghost lane's side: 0 -x, 1 +x, 2 -y, 3 +y
   const int side = (tid >> 4) & 3;
   const T dt = clk[0];
   const T dx0 = P.dx;
@@ -324,7 +330,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     // the next pair from the queue (every thread has passed a barrier since it last read q_pair)
     if (threadIdx.x == 0) q_pair = atomicAdd(&qctl[AMR_Q_NEXT], 1);
     __syncthreads();
-    const int wp = q_pair;
+    const int wp = __builtin_amdgcn_readfirstlane(q_pair);
     __syncthreads();   // every thread has read q_pair before thread 0 takes the next ticket
     if (AF_PAIR * wp >= count) break;
     // -1 pads a queue part of odd length. With pairs it is always a pair's second entry (parts
@@ -333,7 +339,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     if (list[AF_PAIR * wp] < 0) continue;
     const int wi = AF_PAIR * wp + half;
     const bool act_blk = wi < count && list[wi] >= 0;
-    const int s = list[act_blk ? wi : AF_PAIR * wp];
+    const int s = __builtin_amdgcn_readfirstlane(list[act_blk ? wi : AF_PAIR * wp]);
     // a leaf with a refined neighbour: wait for the finer leaves across it (one lane each), then
     // form the means of their fluxes on its coarse-fine faces
     const int d0 = act_blk ? dep_off[s] : 0, nd = act_blk ? dep_off[s + 1] - d0 : 0;
@@ -374,181 +380,262 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     const T dx = dx0 * (T(1) / T(1 << bt(tab, s, BT_LEVEL)));
     P.dx = dx;
     const T dtdx = wave_uniform(dt / dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
-    const bool cells = cells0 && act_blk, ghosts = ghosts0 && act_blk;
-    // beside a coarser block (-1): its ghosts are predicted in place; elsewhere they are another
-    // block's cells, whose half steps come from the shell
-    const bool gk = ghosts && bt(tab, s, BT_NB + side) == -1;
-    const bool kz_lo = bt(tab, s, BT_NB + 4) == -1, kz_hi = bt(tab, s, BT_NB + 5) == -1;
-    // same-level leaves: across this ring lane's side, and across the two z faces
-    const int nbs = (!cells0 && act_blk) ? same_leaf(tab, s, side) : -1;
-    const int nbz_lo = same_leaf(tab, s, 4), nbz_hi = same_leaf(tab, s, 5);
+    // the faces' actions (boundary_face)
+    int fa[6];
+#pragma unroll
+    for (int k = 0; k < 6; k++) fa[k] = __builtin_amdgcn_readfirstlane(act[s * 6 + k]);
     __syncthreads();   // the previous block's last LDS reads are done
 
-    // texel (x, y, z) of this block: its own cells and a same-level leaf's from U, edges zero,
-    // other ghosts from the shell
-    auto texel = [&](int z) -> Prim<T> {
+    const size_t own = (size_t)s * AMR_CELLS;
+    // slopes and edge increments of this column in the plane whose primitives are at q (those of
+    // the plane below at m, of the plane above in pp), and the shock detector's terms
+    struct Edges { Inc<T> xu, xd, yu, yd, zu, zd; };
+    auto slopes = [&](int q, int m, Prim<T>& pc, T cs, const Prim<T>& pp, AxisSlope<T> sl[3], Edges& e, T& conv,
+                      T& jump) {
+      pc = PL::prim(L, q, t);
+      pc.cs = cs;
+      // (axis by axis, as k_fused_r)
+      {
+        const Prim<T> xm = PL::prim(L, q, t.off(-1)), xp = PL::prim(L, q, t.off(1));
+        sl[0] = axis_slope<T, LIM, ISEN>(P, xm, pc, xp, &e.xu, &e.xd);
+        conv = xp.vx - xm.vx;
+        jump = jump_over(P, xm.p, xp.p);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      {
+        const Prim<T> ym = PL::prim(L, q, t.off(-BX)), yp = PL::prim(L, q, t.off(BX));
+        sl[1] = axis_slope<T, LIM, ISEN>(P, ym, pc, yp, &e.yu, &e.yd);
+        conv = conv + (yp.vy - ym.vy);
+        jump = tmax(jump, jump_over(P, ym.p, yp.p));
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      const Prim<T> pm = PL::prim(L, m, t);
+      sl[2] = axis_slope<T, LIM, ISEN>(P, pm, pc, pp, &e.zu, &e.zd);
+      conv = conv + (pp.vz - pm.vz);
+      jump = tmax(jump, jump_over(P, pm.p, pp.p));
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto shell_half = [&](int h) {
+      const T4<T> a = sh[2 * (SH_TEXELS + h)], b = sh[2 * (SH_TEXELS + h) + 1];
+      Half<T> hc;
+      hc.rho = a.x; hc.vx = a.y; hc.vy = a.z; hc.vz = a.w;
+      hc.p = b.x; hc.s = b.y; hc.shock = b.z; hc.fo = b.w;
+      return hc;
+    };
+    auto shell_prim = [](T4<T> a, T4<T> b) {
       Prim<T> w;
-      w.rho = w.vx = w.vy = w.vz = w.p = w.s = w.cs = T(0);
-      const bool oz = z < 0 || z >= AMR_BS;
-      if (!act_blk || (!cells0 && oz)) return w;
-      int src = -1;
-      if (cells0) {
-        if (!oz) src = s;
-        else if ((z < 0 ? nbz_lo : nbz_hi) >= 0) src = z < 0 ? nbz_lo : nbz_hi;
-      } else {
-        src = nbs;
-      }
-      if (src >= 0) {
-        const int xs = x < 0 ? x + AMR_BS : (x >= AMR_BS ? x - AMR_BS : x);
-        const int ys = y < 0 ? y + AMR_BS : (y >= AMR_BS ? y - AMR_BS : y);
-        const int zs = z < 0 ? z + AMR_BS : (z >= AMR_BS ? z - AMR_BS : z);
-        const size_t o = (size_t)src * AMR_CELLS + cel(xs, ys, zs);
-        return prim_from_cons(P, U1[o], U2[o]);
-      }
-      const int g = oz ? ghost_plane_slot(z) * AF_NT + t : 4 * AF_NT + z * AF_RING + (tid - 256);
-      const T4<T> a = sh[2 * g], b = sh[2 * g + 1];
       w.rho = a.x; w.vx = a.y; w.vy = a.z; w.vz = a.w;
       w.p = b.x; w.s = b.y; w.cs = b.z;
       return w;
     };
-    lds_put_prim6<T, NT>(L + LY::Q0, t, texel(-2));
-    T cs_c;   // this column's sound speed in plane c
-    {
-      const Prim<T> q = texel(-1);
-      lds_put_prim6<T, NT>(L + LY::Q1, t, q);
-      cs_c = q.cs;
-    }
-    Prim<T> nxt = texel(0);
-    __syncthreads();
+    // the buffer of plane c's primitives
+    auto buf = [](int c) { return (c & 1) ? PL::QN : 0; };
 
-    SideData<T> zs_prev;
-    T hp_prev = T(0);
-    Flux<T> fz_lo = zero_flux<T>();
-    Flux<T> axy_prev = zero_flux<T>();
-
-    for (int c = -1; c <= AMR_BS; c++) {
-      const Prim<T> pp = nxt;             // plane c + 1
-      if (c + 2 <= AMR_BS + 1) nxt = texel(c + 2);
-      const bool odd = ((c + 1) & 1) != 0;
-      const T* Lq = L + (odd ? LY::Q0 : LY::Q1);
-      T* Lm = L + (odd ? LY::Q1 : LY::Q0);
-
-      // 2. the half step of texel (x, y, c) and its sides: every cell; a ghost plane's texels
-      //    (c = -1, 16) in the cell waves; the face ghosts of the cell planes in the ghost wave
-      const bool oz = c < 0 || c >= AMR_BS;
-      SideData<T> sxl, syl, szl, szu;
-      T hp = T(0);
-      if (cells || (ghosts && !oz)) {
-        Prim<T> pc = lds_prim<T, NT>(Lq, t);
-        pc.cs = cs_c;
-        const Prim<T> pm = lds_prim<T, NT>(Lm, t);
-        const Prim<T> xm = lds_prim<T, NT>(Lq, t - 1), xp = lds_prim<T, NT>(Lq, t + 1);
-        const Prim<T> ym = lds_prim<T, NT>(Lq, t - BX), yp = lds_prim<T, NT>(Lq, t + BX);
-        Inc<T> ixu, ixd, iyu, iyd, izu, izd;
-        AxisSlope<T> sl[3];
-        sl[0] = axis_slope<T, LIM, ISEN>(P, xm, pc, xp, &ixu, &ixd);
-        sl[1] = axis_slope<T, LIM, ISEN>(P, ym, pc, yp, &iyu, &iyd);
-        sl[2] = axis_slope<T, LIM, ISEN>(P, pm, pc, pp, &izu, &izd);
-        const bool ghost = ghosts || oz;
-        const bool in_place = ghosts ? gk : (oz && (c < 0 ? kz_lo : kz_hi));
-        // a same-level leaf's cell away from the face's rim: as at its source, in place
-        const bool exact = ghosts ? (nbs >= 0 && off_rim(side < 2 ? y : x, c))
-                                  : (oz && (c < 0 ? nbz_lo : nbz_hi) >= 0 && off_rim(x, y));
-        Half<T> hc;
-        if (!ghost || in_place || exact) {
-          if (ghost && !exact) {
-            // beside a coarser block: predicted in place, the slopes along the ghost's rim axes
-            // dropped where their neighbour is an unassembled edge texel (amr/predict.wgsl:183-221)
-            const bool ox = x < 0 || x >= AMR_BS, oy = y < 0 || y >= AMR_BS;
-            scale_inc(sl[0].s, (!ox && (x == 0 || x == AMR_BS - 1)) ? T(0) : T(1));
-            scale_inc(sl[1].s, (!oy && (y == 0 || y == AMR_BS - 1)) ? T(0) : T(1));
-            scale_inc(sl[2].s, (!oz && (c == 0 || c == AMR_BS - 1)) ? T(0) : T(1));
-          }
-          const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (pp.vz - pm.vz);
-          const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, pm.p, pp.p)));
-          hc = hancock<T, LIM>(P, pc, sl, conv, jump, hstep);
+    if (!act_blk) {
+      for (int k = 0; k < 2 + 2 * AMR_BS; k++) __syncthreads();
+    } else if (cells) {
+      const bool kz_lo = bt(tab, s, BT_NB + 4) == -1, kz_hi = bt(tab, s, BT_NB + 5) == -1;
+      const int nbz_lo = same_leaf(tab, s, 4), nbz_hi = same_leaf(tab, s, 5);
+      const unsigned int at = (unsigned int)(cel(x, y, 0)) * (unsigned int)sizeof(T4<T>);
+      T4<T> b1, b2;
+      // plane z's texel: this block's cells and a same-level leaf's from U, other ghosts from the
+      // shell (a scalar choice per plane)
+      auto load = [&](int z) {
+        const bool oz = z < 0 || z >= AMR_BS;
+        const int src = !oz ? s : (z < 0 ? nbz_lo : nbz_hi);
+        if (src >= 0) {
+          const size_t o = (size_t)src * AMR_CELLS + (z & (AMR_BS - 1)) * (AMR_BS * AMR_BS);
+          b1 = plane_load<T>(U1 + o, at);
+          b2 = plane_load<T>(U2 + o, at);
         } else {
-          // another block's cell (same level, refined, or this block's boundary image): its half
-          // step was formed in the shell pass
-          const int h = oz ? 64 * AMR_BS + (c < 0 ? 0 : AMR_BS * AMR_BS) + y * AMR_BS + x : (tid - 256) * AMR_BS + c;
-          const T4<T> a = sh[2 * (SH_TEXELS + h)], b = sh[2 * (SH_TEXELS + h) + 1];
-          hc.rho = a.x; hc.vx = a.y; hc.vy = a.z; hc.vz = a.w;
-          hc.p = b.x; hc.s = b.y; hc.shock = b.z; hc.fo = b.w;
+          const int g = ghost_plane_slot(z) * AF_NT + (y + 2) * BX + (x + 2);
+          b1 = sh[2 * g];
+          b2 = sh[2 * g + 1];
         }
-        hp = hc.p;
-        sxl = side_of(P, hc, ixd, T(-1));
-        syl = side_of(P, hc, iyd, T(-1));
-        szl = side_of(P, hc, izd, T(-1));
-        szu = side_of(P, hc, izu, T(1));
-        lds_put_side<T, NT>(L, LY::SX, t, side_of(P, hc, ixu, T(1)));
-        lds_put_side<T, NT>(L, LY::SY, t, side_of(P, hc, iyu, T(1)));
-      }
-      // plane c + 1 into the slot plane c - 1 leaves
-      lds_put_prim6<T, NT>(Lm, t, pp);
-      cs_c = pp.cs;
+      };
+      auto prim = [&](int z) {
+        const bool oz = z < 0 || z >= AMR_BS;
+        return !oz || (z < 0 ? nbz_lo : nbz_hi) >= 0 ? prim_from_cons(P, b1, b2) : shell_prim(b1, b2);
+      };
+      // a ghost plane's half step (c = -1, 16): in place beside a coarser block, with the slopes
+      // along the face dropped where their neighbour is an unassembled edge texel
+      // (amr/predict.wgsl:183-221), and where the texel is a same-level leaf's cell away from the
+      // face's rim, as at its source; else another block's cell, formed in the shell pass
+      auto ghost_plane_half = [&](int c, const Prim<T>& pp, T cs, Edges& e) {
+        AxisSlope<T> sl[3];
+        Prim<T> pc;
+        T conv, jump;
+        slopes(buf(c), buf(c - 1), pc, cs, pp, sl, e, conv, jump);
+        const bool coarse = c < 0 ? kz_lo : kz_hi;
+        if (coarse) {
+          scale_inc(sl[0].s, (x == 0 || x == AMR_BS - 1) ? T(0) : T(1));
+          scale_inc(sl[1].s, (y == 0 || y == AMR_BS - 1) ? T(0) : T(1));
+        }
+        Half<T> h = hancock<T, LIM>(P, pc, sl, conv, jump, hstep);
+        const bool exact = (c < 0 ? nbz_lo : nbz_hi) >= 0 && off_rim(x, y);
+        if (!coarse && !exact) h = shell_half(64 * AMR_BS + (c < 0 ? 0 : AMR_BS * AMR_BS) + y * AMR_BS + x);
+        return h;
+      };
+      load(-2);
+      PL::put_prim(L, buf(-2), t, prim(-2));
+      load(-1);
+      Prim<T> pp = prim(-1);
+      PL::put_prim(L, buf(-1), t, pp);
+      T cs = pp.cs;            // this column's sound speed in plane c
+      load(0);
       __syncthreads();
-
-      // 3. the x and y faces below this column (cells; the +x and +y ghosts' lower faces), and
-      //    the z face below plane c
-      const bool live = c >= 0 && c < AMR_BS;
-      Flux<T> Fx = zero_flux<T>(), Fy = zero_flux<T>(), fz = zero_flux<T>();
-      if (live && (cells || (ghosts && side == 1))) {
-        Fx = face_from_sides<T, RS>(P, lds_get_side<T, NT>(L, LY::SX, t - 1), sxl, 0);
-        if (x == 0) Fx = boundary_face<T>(act[s * 6 + 0], R, CF, c * 16 + y, Fx);
-        else if (x == AMR_BS) Fx = boundary_face<T>(act[s * 6 + 1], R, CF, c * 16 + y, Fx);
+      SideData<T> zs;          // the upper z side of the plane below, and its half-step pressure
+      T hp;
+      Flux<T> fz_lo, xy;       // the z face below and the x/y net inflow of that plane
+      T rate = T(0);           // the block's largest rate
+      auto update = [&](int c, T4<T> u1, T4<T> u2, const Flux<T>& fz) {
+        T4<T> o1, o2;
+        advance(P, u1, u2, net_z(xy, fz_lo, fz), hp, dtdx, o1, o2);
+        const size_t o = own + c * (AMR_BS * AMR_BS);
+        plane_store<T>(O1 + o, at, o1);
+        plane_store<T>(O2 + o, at, o2);
+        rate = tmax(rate, rate_of(P, prim_from_cons(P, o1, o2)));
+      };
+      {
+        pp = prim(0);
+        load(1);
+        Edges e;
+        const Half<T> h = ghost_plane_half(-1, pp, cs, e);
+        zs = side_of(P, h, e.zu, T(1));
+        PL::put_prim(L, buf(0), t, pp);
+        cs = pp.cs;
       }
-      if (live && (cells || (ghosts && side == 3))) {
-        Fy = face_from_sides<T, RS>(P, lds_get_side<T, NT>(L, LY::SY, t - BX), syl, 1);
-        if (y == 0) Fy = boundary_face<T>(act[s * 6 + 2], R, CF, x * 16 + c, Fy);
-        else if (y == AMR_BS) Fy = boundary_face<T>(act[s * 6 + 3], R, CF, x * 16 + c, Fy);
-      }
-      if (cells && c >= 0) {
-        fz = face_from_sides<T, RS>(P, zs_prev, szl, 2);
-        if (c == 0) fz = boundary_face<T>(act[s * 6 + 4], R, CF, y * 16 + x, fz);
-        else if (c == AMR_BS) fz = boundary_face<T>(act[s * 6 + 5], R, CF, y * 16 + x, fz);
-      }
-      // 4. the x/y fluxes into LDS
-      if (live && (cells || (ghosts && side == 1))) lds_put_flux<T, NT>(L, LY::FX, t, Fx);
-      if (live && (cells || (ghosts && side == 3))) lds_put_flux<T, NT>(L, LY::FY, t, Fy);
       __syncthreads();
-
-      // 5. this plane's x/y net inflow, and the update of plane c - 1
-      if (cells) {
-        Flux<T> axy = zero_flux<T>();
-        if (live) {
-          const Flux<T> xh = lds_get_flux<T, NT>(L, LY::FX, t + 1);
-          const Flux<T> yh = lds_get_flux<T, NT>(L, LY::FY, t + BX);
-          axy.m = (Fx.m - xh.m) + (Fy.m - yh.m);
-          axy.mx = (Fx.mx - xh.mx) + (Fy.mx - yh.mx);
-          axy.my = (Fx.my - xh.my) + (Fy.my - yh.my);
-          axy.mz = (Fx.mz - xh.mz) + (Fy.mz - yh.mz);
-          axy.e = (Fx.e - xh.e) + (Fy.e - yh.e);
-          axy.ei = (Fx.ei - xh.ei) + (Fy.ei - yh.ei);
-          axy.s = (Fx.s - xh.s) + (Fy.s - yh.s);
-          axy.vn = (Fx.vn - xh.vn) + (Fy.vn - yh.vn);
+      for (int c = 0; c < AMR_BS; c++) {
+        pp = prim(c + 1);
+        Edges e;
+        Half<T> h;
+        {
+          AxisSlope<T> sl[3];
+          Prim<T> pc;
+          T conv, jump;
+          slopes(buf(c), buf(c - 1), pc, cs, pp, sl, e, conv, jump);
+          h = hancock<T, LIM>(P, pc, sl, conv, jump, hstep);
         }
-        if (c - 1 >= 0 && c - 1 < AMR_BS) {
-          const size_t o = (size_t)s * AMR_CELLS + cel(x, y, c - 1);
-          Flux<T> net;
-          net.m = axy_prev.m + (fz_lo.m - fz.m);
-          net.mx = axy_prev.mx + (fz_lo.mx - fz.mx);
-          net.my = axy_prev.my + (fz_lo.my - fz.my);
-          net.mz = axy_prev.mz + (fz_lo.mz - fz.mz);
-          net.e = axy_prev.e + (fz_lo.e - fz.e);
-          net.ei = axy_prev.ei + (fz_lo.ei - fz.ei);
-          net.s = axy_prev.s + (fz_lo.s - fz.s);
-          net.vn = axy_prev.vn + (fz_lo.vn - fz.vn);
-          T4<T> o1, o2;
-          advance(P, U1[o], U2[o], net, hp_prev, dtdx, o1, o2);
-          O1[o] = o1;
-          O2[o] = o2;
-          // the next step's rate / dx (assemble's leaf-cell rate, amr/assemble.wgsl:77-154)
-          rate_max = tmax(rate_max, rate_of(P, prim_from_cons(P, o1, o2)) / dx);
+        __builtin_amdgcn_sched_barrier(0);
+        T4<T> u1, u2;
+        if (c > 0) {
+          const size_t o = own + (c - 1) * (AMR_BS * AMR_BS);
+          u1 = plane_load<T>(U1 + o, at);
+          u2 = plane_load<T>(U2 + o, at);
         }
-        zs_prev = szu;
-        hp_prev = hp;
+        PL::put_side(L, PL::SX, t, side_of(P, h, e.xu, T(1)));
+        PL::put_side(L, PL::SY, t, side_of(P, h, e.yu, T(1)));
+        PL::put_shock(L, PL::SK, t, h.shock);
+        PL::put_prim(L, buf(c + 1), t, pp);
+        cs = pp.cs;
+        __builtin_amdgcn_sched_barrier(0);
+        Flux<T> fz = face_from_sides<T, RS>(P, zs, side_of(P, h, e.zd, T(-1)), 2);
+        if (c == 0) fz = boundary_face<T>(fa[4], R, CF, y * 16 + x, fz);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c > 0) update(c - 1, u1, u2, fz);
         fz_lo = fz;
-        axy_prev = axy;
+        zs = side_of(P, h, e.zu, T(1));
+        hp = h.p;
+        __builtin_amdgcn_sched_barrier(0);
+        load(c + 2);
+        __syncthreads();
+        Flux<T> Fx = face_from_sides<T, RS>(P, PL::side(L, PL::SX, PL::SK, t.off(-1)), side_of(P, h, e.xd, T(-1)), 0);
+        if (fa[0] >= 0 && x == 0) Fx = boundary_face<T>(fa[0], R, CF, c * 16 + y, Fx);
+        PL::put_flux(L, PL::FX, t, Fx);
+        __builtin_amdgcn_sched_barrier(0);
+        Flux<T> Fy = face_from_sides<T, RS>(P, PL::side(L, PL::SY, PL::SK, t.off(-BX)), side_of(P, h, e.yd, T(-1)), 1);
+        if (fa[2] >= 0 && y == 0) Fy = boundary_face<T>(fa[2], R, CF, x * 16 + c, Fy);
+        PL::put_flux(L, PL::FY, t, Fy);
+        __syncthreads();
+        xy = net_xy(Fx, PL::flux(L, PL::FX, t.off(1)), Fy, PL::flux(L, PL::FY, t.off(BX)));
+      }
+      {
+        pp = prim(AMR_BS + 1);
+        const size_t o = own + (AMR_BS - 1) * (AMR_BS * AMR_BS);
+        const T4<T> u1 = plane_load<T>(U1 + o, at), u2 = plane_load<T>(U2 + o, at);
+        Edges e;
+        const Half<T> h = ghost_plane_half(AMR_BS, pp, cs, e);
+        Flux<T> fz = face_from_sides<T, RS>(P, zs, side_of(P, h, e.zd, T(-1)), 2);
+        fz = boundary_face<T>(fa[5], R, CF, y * 16 + x, fz);
+        update(AMR_BS - 1, u1, u2, fz);
+      }
+      // the next step's rate / dx (assemble's leaf-cell rate, amr/assemble.wgsl:77-154)
+      rate_max = tmax(rate_max, rate / dx);
+    } else {
+      // the ghost columns: a same-level leaf's cells from U, others from the shell; edges (the
+      // ghost planes' texels beside them) are zero
+      const int nbs = same_leaf(tab, s, side);
+      const int xs = (x + AMR_BS) & (AMR_BS - 1), ys = (y + AMR_BS) & (AMR_BS - 1);
+      const size_t o0 = nbs >= 0 ? (size_t)nbs * AMR_CELLS + cel(xs, ys, 0) : (size_t)0;
+      const T4<T>* s1 = nbs >= 0 ? U1 + o0 : sh + 2 * (4 * AF_NT + (tid - 256));
+      const T4<T>* s2 = nbs >= 0 ? U2 + o0 : s1 + 1;
+      const size_t step = nbs >= 0 ? AMR_BS * AMR_BS : 2 * AF_RING;
+      T4<T> b1, b2;
+      auto load = [&](int z) {
+        b1 = s1[z * step];
+        b2 = s2[z * step];
+      };
+      auto prim = [&] { return nbs >= 0 ? prim_from_cons(P, b1, b2) : shell_prim(b1, b2); };
+      Prim<T> none;
+      none.rho = none.vx = none.vy = none.vz = none.p = none.s = none.cs = T(0);
+      PL::put_prim(L, buf(-1), t, none);
+      load(0);
+      __syncthreads();
+      Prim<T> pp = prim();
+      load(1);
+      PL::put_prim(L, buf(0), t, pp);
+      T cs = pp.cs;
+      __syncthreads();
+      if (ghosts) {
+        // ring 1: beside a coarser block predicted in place; a same-level leaf's cell away from
+        // the face's rim as at its source; other half steps from the shell. The +x and +y ghosts'
+        // lower faces are the cells' upper ones: one solve along the lane's axis
+        const bool gk = bt(tab, s, BT_NB + side) == -1;
+        const bool upper = (side & 1) != 0, ax = side == 1;
+        const int fk = side == 1 ? fa[1] : fa[3];
+        for (int c = 0; c < AMR_BS; c++) {
+          if (c + 1 < AMR_BS) pp = prim(); else pp = none;
+          Edges e;
+          Half<T> h;
+          {
+            AxisSlope<T> sl[3];
+            Prim<T> pc;
+            T conv, jump;
+            slopes(buf(c), buf(c - 1), pc, cs, pp, sl, e, conv, jump);
+            if (gk) {
+              scale_inc(sl[0].s, (side >= 2 && (x == 0 || x == AMR_BS - 1)) ? T(0) : T(1));
+              scale_inc(sl[1].s, (side < 2 && (y == 0 || y == AMR_BS - 1)) ? T(0) : T(1));
+              scale_inc(sl[2].s, (c == 0 || c == AMR_BS - 1) ? T(0) : T(1));
+            }
+            h = hancock<T, LIM>(P, pc, sl, conv, jump, hstep);
+          }
+          const bool exact = nbs >= 0 && off_rim(side < 2 ? y : x, c);
+          if (!gk && !exact) h = shell_half((tid - 256) * AMR_BS + c);
+          if (c + 2 < AMR_BS) load(c + 2);
+          PL::put_side(L, PL::SX, t, side_of(P, h, e.xu, T(1)));
+          PL::put_side(L, PL::SY, t, side_of(P, h, e.yu, T(1)));
+          PL::put_shock(L, PL::SK, t, h.shock);
+          const SideData<T> sxl = side_of(P, h, e.xd, T(-1)), syl = side_of(P, h, e.yd, T(-1));
+          PL::put_prim(L, buf(c + 1), t, pp);
+          cs = pp.cs;
+          __syncthreads();
+          if (upper) {
+            Flux<T> F = face_from_sides_rt<T, RS>(P, PL::side(L, ax ? PL::SX : PL::SY, PL::SK, t.off(ax ? -1 : -BX)),
+                                                  ax ? sxl : syl, ax ? 0 : 1);
+            F = boundary_face<T>(fk, R, CF, ax ? c * 16 + y : x * 16 + c, F);
+            PL::put_flux(L, ax ? PL::FX : PL::FY, t, F);
+          }
+          __syncthreads();
+        }
+      } else {
+        // ring 2: loads only
+        for (int c = 0; c < AMR_BS; c++) {
+          if (c + 1 < AMR_BS) PL::put_prim(L, buf(c + 1), t, prim());
+          if (c + 2 < AMR_BS) load(c + 2);
+          __syncthreads();
+          __syncthreads();
+        }
       }
     }
     // a leaf on a coarser block: its register fluxes are written (the barrier waits for every
@@ -556,17 +643,15 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     // done flag
     __syncthreads();
     bool writes_reg = false;
-    for (int k = 0; k < 6; k++) {
-      const int a = act[s * 6 + k];
-      writes_reg = writes_reg || (a >= 0 && !(a & 1));
-    }
+#pragma unroll
+    for (int k = 0; k < 6; k++) writes_reg = writes_reg || (fa[k] >= 0 && !(fa[k] & 1));
     if (tid == 0 && act_blk && writes_reg) {
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       __hip_atomic_store(done + s, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
   // workgroup maximum of the next step's rate, one atomicMax
-  T v = wave_max(rate_max);
+  const T v = wave_max(rate_max);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0) {
