@@ -2,11 +2,11 @@
 // what the reference's assemble, predict and update passes compute (src/amr/assemble.wgsl,
 // predict.wgsl, update.wgsl), with no W, PA or PB atlas of the blocks' cells in HBM:
 //
-//  - k_amr_shell: per leaf, the ghost texels of its 20^3 region, formed from U (same-level
-//    neighbours, boundary images, prolongation from a coarser leaf, restriction of refined
-//    children: amr_texel), and the half steps of its first ghost layer where those are another
-//    block's cells ("at source", amr/predict.wgsl:183-221), all lanes busy; k_amr_rim, the half
-//    steps on the rims of faces beside same-level leaves, once per source cell;
+//  - k_amr_shell, twice: per leaf, the ghost texels of its 20^3 region, formed from U (boundary
+//    images, prolongation from a coarser leaf, restriction of refined children: amr_texel); then
+//    the half steps of its first ghost layer where those are another block's cells ("at source",
+//    amr/predict.wgsl:183-221): beside boundary images, and on the rims of faces beside same-level
+//    leaves, once per source cell;
 //  - k_amr_fused, one persistent kernel per launch: a workgroup owns one 16^3 block at a time
 //    and marches along z: its cells from U, its ghosts from the shell; the half step of every
 //    cell and of the ghosts beside a coarser block (masked transverse slopes), in LDS;
@@ -40,7 +40,7 @@ namespace shx {
 constexpr int AF_SIDE = AMR_PAD;              // 20 columns per side
 constexpr int AF_NT = AF_SIDE * AF_SIDE;      // 400 columns
 constexpr int AF_THREADS = 384;             // one block's march
-// blocks marched side by side per workgroup: two in FP32 (2 x 51 KB of LDS), one in FP64
+// blocks marched side by side per workgroup: two in FP32 (2 x 72 KB of LDS), one in FP64
 template <typename T>
 constexpr int af_pair() { return sizeof(T) == 4 ? 2 : 1; }
 constexpr int AF_RING = 128;                  // ghost columns with a value: 64 of ring 1, 64 of ring 2
@@ -56,46 +56,6 @@ __device__ __forceinline__ void af_column(int t, int& x, int& y) {
   const int lo = -ring, hi = AMR_BS - 1 + ring;
   x = side == 0 ? lo : (side == 1 ? hi : i);
   y = side == 2 ? lo : (side == 3 ? hi : i);
-}
-
-// Assembled primitives of a texel of block `slot` (zero for edges and corners, as the atlas).
-// LEAF: the caller knows `slot` is a leaf, whose cells are read directly (a parent's cells are
-// the means of its children's, u_at).
-template <typename T, int LIM, bool LEAF>
-__device__ __forceinline__ Prim<T> texel_of(const Params<T>& P, const int* __restrict__ tab,
-                                            const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, int slot,
-                                            int x, int y, int z) {
-  if (x >= 0 && x < AMR_BS && y >= 0 && y < AMR_BS && z >= 0 && z < AMR_BS && (LEAF || is_leaf(tab, slot))) {
-    const size_t o = (size_t)slot * AMR_CELLS + cel(x, y, z);
-    return prim_from_cons(P, U1[o], U2[o]);
-  }
-  Prim<T> w;
-  if (!amr_texel<T, LIM>(P, tab, U1, U2, slot, x, y, z, w)) {
-    w.rho = w.vx = w.vy = w.vz = w.p = w.s = w.cs = T(0);
-  }
-  return w;
-}
-
-// The half step of texel (x, y, z) of block `slot` from that block's texels formed directly
-// (predict_cell on the source block, amr/predict.wgsl:90-181); P carries the block's dx
-template <typename T, int LIM, bool ISEN>
-__device__ __forceinline__ Half<T> half_at_source(const Params<T>& P, const int* __restrict__ tab,
-                                               const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, int slot,
-                                               int x, int y, int z, T dt) {
-  const Prim<T> q = texel_of<T, LIM, false>(P, tab, U1, U2, slot, x, y, z);
-  const Prim<T> xm = texel_of<T, LIM, false>(P, tab, U1, U2, slot, x - 1, y, z);
-  const Prim<T> xp = texel_of<T, LIM, false>(P, tab, U1, U2, slot, x + 1, y, z);
-  const Prim<T> ym = texel_of<T, LIM, false>(P, tab, U1, U2, slot, x, y - 1, z);
-  const Prim<T> yp = texel_of<T, LIM, false>(P, tab, U1, U2, slot, x, y + 1, z);
-  const Prim<T> zm = texel_of<T, LIM, false>(P, tab, U1, U2, slot, x, y, z - 1);
-  const Prim<T> zp = texel_of<T, LIM, false>(P, tab, U1, U2, slot, x, y, z + 1);
-  AxisSlope<T> sl[3];
-  sl[0] = axis_slope<T, LIM, ISEN>(P, xm, q, xp, nullptr, nullptr);
-  sl[1] = axis_slope<T, LIM, ISEN>(P, ym, q, yp, nullptr, nullptr);
-  sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
-  const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
-  const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
-  return hancock<T, LIM>(P, q, sl, conv, jump, slope_step<T, LIM>(P, dt));
 }
 
 // Flux register: per coarse-fine face of a leaf, its 16 x 16 faces' fluxes (8 values each), in
@@ -211,71 +171,191 @@ __device__ __forceinline__ bool off_rim(int i, int j) {
   return i >= 1 && i <= AMR_BS - 2 && j >= 1 && j <= AMR_BS - 2;
 }
 
-// Work of the shell, one wave per item (shell index, slot, face k, chunk), listed on the host from
-// the static mesh: PART 0, the ghost texels of face k (two layers, 512 texels: chunks 0-7) where
-// its neighbour is not a same-level leaf; PART 1, the first layer's half steps (chunks 0-3)
-// beside a boundary image. Faces on a coarser block have no PART 1 work (the march predicts
-// those ghosts in place); beside a same-level leaf only the face's rim needs its half steps,
-// which k_amr_rim forms from the cells of the leaf across.
-template <int PART>
-constexpr int sh_part_waves() { return PART == 0 ? 6 : 3; }
+// a shell texel
+template <typename T>
+__device__ __forceinline__ Prim<T> shell_prim(T4<T> a, T4<T> b) {
+  Prim<T> w;
+  w.rho = a.x; w.vx = a.y; w.vy = a.z; w.vz = a.w;
+  w.p = b.x; w.s = b.y; w.cs = b.z;
+  return w;
+}
+// the item of ghost texel (x, y, z), out of the block along one axis
+__device__ __forceinline__ int shell_texel(int x, int y, int z) {
+  if (z < 0 || z >= AMR_BS) return ghost_plane_slot(z) * AF_NT + (y + 2) * AF_SIDE + (x + 2);
+  const bool ox = x < 0 || x >= AMR_BS;
+  const int c = ox ? x : y, i = ox ? y : x;
+  const int ring = c < 0 ? -1 - c : c - AMR_BS, side = (ox ? 0 : 2) + (c >= AMR_BS);
+  return 4 * AF_NT + z * AF_RING + ring * 64 + side * 16 + i;
+}
 
-template <typename T, int LIM, bool ISEN, int PART>
-__global__ __launch_bounds__(256, sh_part_waves<PART>()) void k_amr_shell(
-    Params<T> P, Levels<T> LV, const int* __restrict__ tab, const int4* __restrict__ work, int nwork,
-    const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, T4<T>* __restrict__ SH, const T* __restrict__ clk) {
+// The shell's texels, one wave per item (shell index, slot, face k, code), listed on the host from
+// the static mesh: the two layers (512 texels) beyond a face whose neighbour is not a same-level
+// leaf. Beside a coarser block (code 8) a lane takes one of the face's 64 coarse cells and forms
+// its eight fine texels from one set of slopes; else the wave takes 64 texels (code 0-7), images
+// and means. Bound by latency: a chain of table and cell reads.
+// On the 3D blast's 1618 leaves 43 us with a wave per 64 texels, slopes formed for each texel by
+// seven calls; 28 us as now.
+template <typename T, int LIM>
+__device__ __forceinline__ void shell_texels(const Params<T>& P, const int* __restrict__ tab,
+                                             const int4* __restrict__ work, int nwork, const T4<T>* __restrict__ U1,
+                                             const T4<T>* __restrict__ U2, T4<T>* __restrict__ SH) {
   const int wv = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (wv >= nwork) return;
   const int4 wk = work[wv];
-  const int li = wk.x, s = wk.y, k = wk.z, code = wk.w;
-  const int lane = threadIdx.x & 63;
-  int x, y, z, item;
-  if constexpr (PART == 0) {
-    const int e = code * 64 + lane, hi = e >> 8, rem = e & 255;
-    if (k < 4) {
-      // ring hi + 1 column k * 16 + i, plane rem / 16
-      const int col = hi * 64 + k * 16 + (rem & 15);
-      z = rem >> 4;
-      af_column(256 + col, x, y);
-      item = 4 * AF_NT + z * AF_RING + col;
-    } else {
-      // ghost plane (k == 4: z = -2, -1; k == 5: z = 16, 17), cell column rem
-      const int pl = (k == 4 ? 0 : 2) + hi;
-      x = rem & 15;
-      y = rem >> 4;
-      z = pl == 0 ? -2 : (pl == 1 ? -1 : (pl == 2 ? AMR_BS : AMR_BS + 1));
-      item = pl * AF_NT + (y + 2) * AF_SIDE + (x + 2);
-    }
-    const Prim<T> w = texel_of<T, LIM, true>(P, tab, U1, U2, s, x, y, z);
-    T4<T>* out = SH + ((size_t)li * SH_ITEMS + item) * 2;
+  // (the wave's own: the table reads of a face are scalar)
+  const int li = __builtin_amdgcn_readfirstlane(wk.x), s = __builtin_amdgcn_readfirstlane(wk.y);
+  const int k = __builtin_amdgcn_readfirstlane(wk.z), code = __builtin_amdgcn_readfirstlane(wk.w);
+  const int lane = threadIdx.x & 63, axis = k >> 1;
+  T4<T>* const sh = SH + (size_t)li * SH_ITEMS * 2;
+  auto put = [&](int x, int y, int z, const Prim<T>& w) {
+    T4<T>* out = sh + (size_t)shell_texel(x, y, z) * 2;
     out[0] = v4<T>(w.rho, w.vx, w.vy, w.vz);
     out[1] = v4<T>(w.p, w.s, w.cs, T(0));
+  };
+  if (code == 8) {
+    // the coarse cell's first fine texel: even along every axis
+    const int n = (k & 1) ? AMR_BS : -2, i = 2 * (lane & 7), j = 2 * (lane >> 3);
+    const int x = axis == 0 ? n : i, y = axis == 1 ? n : (axis == 0 ? i : j), z = axis == 2 ? n : j;
+    int par[3];
+    const Prolong<T> g = coarse_cell<T, LIM, 3>(P, tab, U1, U2, s, x, y, z, bt(tab, s, BT_COARSE + k), par);
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+      const Cons<T> u = g.child(c & 1, (c >> 1) & 1, c >> 2);
+      put(x + (c & 1), y + ((c >> 1) & 1), z + (c >> 2), prim_from_cons(P, u.a, u.b));
+    }
+    return;
+  }
+  const int e = code * 64 + lane, layer = e >> 8, i = e & 15, j = (e >> 4) & 15;
+  const int n = (k & 1) ? AMR_BS + layer : -1 - layer;
+  const int x = axis == 0 ? n : i, y = axis == 1 ? n : (axis == 0 ? i : j), z = axis == 2 ? n : j;
+  Prim<T> w;
+  if (amr_texel<T, LIM>(P, tab, U1, U2, s, x, y, z, w)) put(x, y, z, w);
+}
+
+// The half step of cell (x, y, z) of leaf `slot` (predict_cell on the source block,
+// amr/predict.wgsl:90-181): its texels from U where they are stored cells, else from the leaf's
+// own shell, all in one batch of loads; P carries the block's dx
+template <typename T, int LIM, bool ISEN>
+__device__ __forceinline__ Half<T> half_at_source(const Params<T>& P, const int* __restrict__ tab,
+                                                  const int* __restrict__ shell_of, const T4<T>* __restrict__ U1,
+                                                  const T4<T>* __restrict__ U2, const T4<T>* __restrict__ SH, int slot,
+                                                  int x, int y, int z, T dt) {
+  Spot sp[7];
+  spots(tab, slot, x, y, z, sp);
+  const T4<T>* sh = SH + (size_t)shell_of[slot] * SH_ITEMS * 2;
+  T4<T> a[7], b[7];
+#pragma unroll
+  for (int k = 0; k < 7; k++) {
+    int c[3];
+    stencil_at(k, x, y, z, c);
+    const T4<T>* g = sh + 2 * (k > 0 && !sp[k].ok ? shell_texel(c[0], c[1], c[2]) : 0);
+    a[k] = *(sp[k].ok ? U1 + sp[k].cell : g);
+    b[k] = *(sp[k].ok ? U2 + sp[k].cell : g + 1);
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  Prim<T> w[7];
+#pragma unroll
+  for (int k = 0; k < 7; k++) {
+    w[k] = prim_from_cons(P, a[k], b[k]);
+    if (!sp[k].ok) w[k] = shell_prim<T>(a[k], b[k]);
+  }
+  const Prim<T>&q = w[0], &xm = w[1], &xp = w[2], &ym = w[3], &yp = w[4], &zm = w[5], &zp = w[6];
+  AxisSlope<T> sl[3];
+  sl[0] = axis_slope<T, LIM, ISEN>(P, xm, q, xp, nullptr, nullptr);
+  sl[1] = axis_slope<T, LIM, ISEN>(P, ym, q, yp, nullptr, nullptr);
+  sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
+  const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
+  const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
+  return hancock<T, LIM>(P, q, sl, conv, jump, slope_step<T, LIM>(P, dt));
+}
+
+// The shell's half steps (after its texels). The first nrim lanes: the rims of faces beside
+// same-level leaves. A rim ghost's source is a cell on an edge of the leaf across the face, whose
+// transverse stencil reaches past the face (the march holds only the face itself). One lane per
+// source cell, from records listed on the host (source slot, cell x | y << 4 | z << 8, then up to
+// three (shell index, half-step item) destinations, -1 for none): an edge cell feeds the shells of
+// the leaves across both its faces, a corner cell three, so each is predicted once, and the lanes
+// of a wave take the edge cells of one block. A same-level face maps no velocity.
+// The other blocks: the first layer beside a boundary image, one wave per item (shell index, slot,
+// face k, chunk 0-3). Faces on a coarser block have no half steps here (the march predicts those
+// ghosts in place).
+// Bound by bandwidth: an edge cell's stencil along y and z touches a cache line per texel, nearly
+// the blocks' whole state in all (5.2 TB/s on the 3D blast: 81 us with the ghosts formed anew for
+// each stencil, 41 us read from the shell).
+template <typename T, int LIM, bool ISEN>
+__device__ __forceinline__ void shell_halves(const Params<T>& P, const int* __restrict__ tab,
+                                             const int* __restrict__ shell_of, const int4* __restrict__ rim, int nrim,
+                                             const int4* __restrict__ work, int nwork, const T4<T>* __restrict__ U1,
+                                             const T4<T>* __restrict__ U2, T4<T>* SH, const T* __restrict__ clk) {
+  const int rim_blocks = (nrim + 255) >> 8;
+  int slot, x, y, z;
+  int li[3], h[3];
+  GSrc g;
+  g.fx = g.fy = g.fz = 1;
+  g.sx = g.sy = g.sz = 0;
+  if ((int)blockIdx.x < rim_blocks) {
+    const int w = blockIdx.x * 256 + threadIdx.x;
+    if (w >= nrim) return;
+    const int4 a = rim[2 * w], b = rim[2 * w + 1];
+    slot = a.x;
+    x = a.y & 15;
+    y = (a.y >> 4) & 15;
+    z = (a.y >> 8) & 15;
+    li[0] = a.z; li[1] = b.x; li[2] = b.z;
+    h[0] = a.w; h[1] = b.y; h[2] = b.w;
   } else {
-    const int e = code * 64 + lane, i = e & 15, j = e >> 4;
-    int h;
+    const int wv = ((int)blockIdx.x - rim_blocks) * 4 + (threadIdx.x >> 6);
+    if (wv >= nwork) return;
+    const int4 wk = work[wv];
+    const int s = wk.y, k = wk.z, e = wk.w * 64 + (threadIdx.x & 63), i = e & 15, j = e >> 4;
     if (k < 4) {
       const int col = k * 16 + i;
       af_column(256 + col, x, y);
       z = j;
-      h = col * AMR_BS + z;
+      h[0] = col * AMR_BS + z;
     } else {
       x = i;
       y = j;
       z = k == 4 ? -1 : AMR_BS;
-      h = 64 * AMR_BS + (k == 4 ? 0 : AMR_BS * AMR_BS) + y * AMR_BS + x;
+      h[0] = 64 * AMR_BS + (k == 4 ? 0 : AMR_BS * AMR_BS) + y * AMR_BS + x;
     }
-    const GSrc g = ghost_src(tab, s, x, y, z);
-    if (g.kind != 0) return;   // beside a coarser block: predicted in place by the march
-    Params<T> Pl = P;
-    Pl.dx = level_dx(P, bt(tab, g.slot, BT_LEVEL));
-    Half<T> hc = half_at_source<T, LIM, ISEN>(Pl, tab, U1, U2, g.slot, g.x, g.y, g.z, clk[0]);
-    hc.vx = bc_vel(hc.vx, g.fx, g.sx);
-    hc.vy = bc_vel(hc.vy, g.fy, g.sy);
-    hc.vz = bc_vel(hc.vz, g.fz, g.sz);
-    T4<T>* out = SH + ((size_t)li * SH_ITEMS + SH_TEXELS + h) * 2;
-    out[0] = v4<T>(hc.rho, hc.vx, hc.vy, hc.vz);
-    out[1] = v4<T>(hc.p, hc.s, hc.shock, hc.fo);
+    li[0] = wk.x;
+    li[1] = li[2] = -1;
+    h[1] = h[2] = 0;
+    g = ghost_src(tab, s, x, y, z);
+    if (g.kind != 0) return;
+    slot = g.slot;
+    x = g.x;
+    y = g.y;
+    z = g.z;
   }
+  Params<T> Pl = P;
+  Pl.dx = level_dx(P, bt(tab, slot, BT_LEVEL));
+  Half<T> hc = half_at_source<T, LIM, ISEN>(Pl, tab, shell_of, U1, U2, SH, slot, x, y, z, clk[0]);
+  hc.vx = bc_vel(hc.vx, g.fx, g.sx);
+  hc.vy = bc_vel(hc.vy, g.fy, g.sy);
+  hc.vz = bc_vel(hc.vz, g.fz, g.sz);
+  const T4<T> v0 = v4<T>(hc.rho, hc.vx, hc.vy, hc.vz), v1 = v4<T>(hc.p, hc.s, hc.shock, hc.fo);
+#pragma unroll
+  for (int d = 0; d < 3; d++) {
+    if (li[d] < 0) continue;
+    T4<T>* out = SH + ((size_t)li[d] * SH_ITEMS + SH_TEXELS + h[d]) * 2;
+    out[0] = v0;
+    out[1] = v1;
+  }
+}
+
+// PART 0 the texels, PART 1 (a launch later: it reads them) the half steps
+template <typename T, int LIM, bool ISEN, int PART>
+__global__ __launch_bounds__(256, 4) void k_amr_shell(Params<T> P, const int* __restrict__ tab,
+                                                      const int* __restrict__ shell_of, const int4* __restrict__ rim,
+                                                      int nrim, const int4* __restrict__ work, int nwork,
+                                                      const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2,
+                                                      T4<T>* SH, const T* __restrict__ clk) {
+  if constexpr (PART == 0)
+    shell_texels<T, LIM>(P, tab, work, nwork, U1, U2, SH);
+  else
+    shell_halves<T, LIM, ISEN>(P, tab, shell_of, rim, nrim, work, nwork, U1, U2, SH, clk);
 }
 
 // ---------------- the march ----------------
@@ -422,12 +502,6 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
       hc.p = b.x; hc.s = b.y; hc.shock = b.z; hc.fo = b.w;
       return hc;
     };
-    auto shell_prim = [](T4<T> a, T4<T> b) {
-      Prim<T> w;
-      w.rho = a.x; w.vx = a.y; w.vy = a.z; w.vz = a.w;
-      w.p = b.x; w.s = b.y; w.cs = b.z;
-      return w;
-    };
     // the buffer of plane c's primitives
     auto buf = [](int c) { return (c & 1) ? PL::QN : 0; };
 
@@ -455,7 +529,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
       };
       auto prim = [&](int z) {
         const bool oz = z < 0 || z >= AMR_BS;
-        return !oz || (z < 0 ? nbz_lo : nbz_hi) >= 0 ? prim_from_cons(P, b1, b2) : shell_prim(b1, b2);
+        return !oz || (z < 0 ? nbz_lo : nbz_hi) >= 0 ? prim_from_cons(P, b1, b2) : shell_prim<T>(b1, b2);
       };
       // a ghost plane's half step (c = -1, 16): in place beside a coarser block, with the slopes
       // along the face dropped where their neighbour is an unassembled edge texel
@@ -576,7 +650,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
         b1 = s1[z * step];
         b2 = s2[z * step];
       };
-      auto prim = [&] { return nbs >= 0 ? prim_from_cons(P, b1, b2) : shell_prim(b1, b2); };
+      auto prim = [&] { return nbs >= 0 ? prim_from_cons(P, b1, b2) : shell_prim<T>(b1, b2); };
       Prim<T> none;
       none.rho = none.vx = none.vy = none.vz = none.p = none.s = none.cs = T(0);
       PL::put_prim(L, buf(-1), t, none);
@@ -661,52 +735,20 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
   }
 }
 
-// The half steps of the face-rim ghosts beside same-level leaves: a rim ghost's source is a cell
-// on an edge of the leaf across the face, whose transverse stencil reaches past the face (the
-// march holds only the face itself). One lane per source cell, from records listed on the host
-// (source slot, cell x | y << 4 | z << 8, then up to three (shell index, half-step item)
-// destinations, -1 for none): an edge cell feeds the shells of the leaves across both its faces,
-// a corner cell three, so each is predicted once, and the lanes of a wave take the edge cells of
-// one block. The value is the shell's own for that ghost (half_at_source at the source; a
-// same-level face maps no velocity).
-template <typename T, int LIM, bool ISEN>
-__global__ __launch_bounds__(256) void k_amr_rim(Params<T> P, const int* __restrict__ tab,
-                                                 const int4* __restrict__ work, int nwork,
-                                                 const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2,
-                                                 T4<T>* __restrict__ SH, const T* __restrict__ clk) {
-  const int w = blockIdx.x * 256 + threadIdx.x;
-  if (w >= nwork) return;
-  const int4 a = work[2 * w], b = work[2 * w + 1];
-  const int x = a.y & 15, y = (a.y >> 4) & 15, z = (a.y >> 8) & 15;
-  Params<T> Pl = P;
-  Pl.dx = level_dx(P, bt(tab, a.x, BT_LEVEL));
-  const Half<T> hc = half_at_source<T, LIM, ISEN>(Pl, tab, U1, U2, a.x, x, y, z, clk[0]);
-  const T4<T> v0 = v4<T>(hc.rho, hc.vx, hc.vy, hc.vz), v1 = v4<T>(hc.p, hc.s, hc.shock, hc.fo);
-  const int li[3] = {a.z, b.x, b.z}, h[3] = {a.w, b.y, b.w};
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    if (li[d] < 0) continue;
-    T4<T>* out = SH + ((size_t)li[d] * SH_ITEMS + SH_TEXELS + h[d]) * 2;
-    out[0] = v0;
-    out[1] = v1;
-  }
-}
-
 // (3D blocks only: the ops of a 2D grid leave the fused form out)
 template <typename T, int LIM, int RS, bool ISEN, int D>
-void AmrImpl<T, LIM, RS, ISEN, D>::shell(const AmrLaunch& L, const int* work0, int n0, const int* work1, int n1,
-                                         const int* work2, int n2, const void* u1, const void* u2, void* sh,
-                                         const void* clk) {
+void AmrImpl<T, LIM, RS, ISEN, D>::shell(const AmrLaunch& L, const int* shell_of, const int* work0, int n0,
+                                         const int* work1, int n1, const int* work2, int n2, const void* u1,
+                                         const void* u2, void* sh, const void* clk) {
   static_assert(D == 3, "the fused form steps 3D blocks");
-  if (n2 > 0)
-    hipLaunchKernelGGL((k_amr_rim<T, LIM, ISEN>), dim3((n2 + 255) / 256), dim3(256), 0, L.stream, P(L), L.tab,
-                       (const int4*)work2, n2, (const T4<T>*)u1, (const T4<T>*)u2, (T4<T>*)sh, (const T*)clk);
   if (n0 > 0)
-    hipLaunchKernelGGL((k_amr_shell<T, LIM, ISEN, 0>), dim3((n0 + 3) / 4), dim3(256), 0, L.stream, P(L), LV(L), L.tab,
-                       (const int4*)work0, n0, (const T4<T>*)u1, (const T4<T>*)u2, (T4<T>*)sh, (const T*)clk);
-  if (n1 > 0)
-    hipLaunchKernelGGL((k_amr_shell<T, LIM, ISEN, 1>), dim3((n1 + 3) / 4), dim3(256), 0, L.stream, P(L), LV(L), L.tab,
-                       (const int4*)work1, n1, (const T4<T>*)u1, (const T4<T>*)u2, (T4<T>*)sh, (const T*)clk);
+    hipLaunchKernelGGL((k_amr_shell<T, LIM, false, 0>), dim3((n0 + 3) / 4), dim3(256), 0, L.stream, P(L), L.tab,
+                       shell_of, nullptr, 0, (const int4*)work0, n0, (const T4<T>*)u1, (const T4<T>*)u2, (T4<T>*)sh,
+                       (const T*)clk);
+  if (n1 + n2 > 0)
+    hipLaunchKernelGGL((k_amr_shell<T, LIM, ISEN, 1>), dim3((n2 + 255) / 256 + (n1 + 3) / 4), dim3(256), 0, L.stream,
+                       P(L), L.tab, shell_of, (const int4*)work2, n2, (const int4*)work1, n1, (const T4<T>*)u1,
+                       (const T4<T>*)u2, (T4<T>*)sh, (const T*)clk);
 }
 
 template <typename T, int LIM, int RS, bool ISEN, int D>

@@ -157,6 +157,94 @@ __device__ __forceinline__ bool u_near(const int* __restrict__ tab, const T4<T>*
   return true;
 }
 
+// Cell (x, y, z) of block `slot`, up to two cells past one face, where it is stored as it is: in
+// the block itself or across that face in a same-level leaf. Else (boundary image, coarser or
+// refined neighbour, edge or corner) ok is false and `cell` is some cell of the block. No branch:
+// a stencil's table reads are in flight together, then its cells'.
+struct Spot {
+  size_t cell;
+  bool ok;
+};
+__device__ __forceinline__ void spots(const int* __restrict__ tab, int slot, int x, int y, int z, Spot sp[7]) {
+  // centre, -x, +x, -y, +y, -z, +z
+  constexpr int N = 6;
+  int nb[N], leaf[N], own = bt(tab, slot, BT_FLAGS);
+#pragma unroll
+  for (int f = 0; f < N; f++) nb[f] = bt(tab, slot, BT_NB + f);
+  const int at[3] = {x, y, z};
+  const bool in = ((x | y | z) & ~(AMR_BS - 1)) == 0;
+#pragma unroll
+  for (int f = 0; f < N; f++) {
+    const int c = at[f >> 1] + ((f & 1) ? 1 : -1);
+    const bool out = (c & ~(AMR_BS - 1)) != 0;
+    const int t = out ? nb[f] : slot;
+    nb[f] = t;
+    leaf[f] = bt(tab, t >= 0 ? t : slot, BT_FLAGS);
+  }
+  sp[0].ok = in && (own & 3) == 3;
+  sp[0].cell = (size_t)slot * AMR_CELLS + (in ? cel(x, y, z) : 0);
+#pragma unroll
+  for (int f = 0; f < N; f++) {
+    int c[3] = {x, y, z};
+    c[f >> 1] = (c[f >> 1] + ((f & 1) ? 1 : -1)) & (AMR_BS - 1);
+    sp[1 + f].ok = in && nb[f] >= 0 && (leaf[f] & 3) == 3;
+    sp[1 + f].cell = sp[1 + f].ok ? (size_t)nb[f] * AMR_CELLS + cel(c[0], c[1], c[2]) : sp[0].cell;
+  }
+}
+
+// texel k of that stencil
+__device__ __forceinline__ void stencil_at(int k, int x, int y, int z, int c[3]) {
+  const int d = (k & 1) ? -1 : 1;
+  c[0] = x + (k == 1 || k == 2 ? d : 0);
+  c[1] = y + (k == 3 || k == 4 ? d : 0);
+  c[2] = z + (k >= 5 ? d : 0);
+}
+
+// The 7-point stencil of a coarse leaf's cell in 3D, as u_near gives each: the cells stored
+// as they are in one batch of loads, u_near only for the others. A wave's chain of dependent
+// reads is three long for the batch, where seven calls made it three each: prolongation is bound
+// by that latency. (In 2D, five calls stay: two neighbours fewer, and the batch's registers cost
+// more waves than its latency saves, 29 -> 34 us for 4096 blocks' assembly.)
+template <typename T>
+__device__ __forceinline__ void near_cells(const int* __restrict__ tab, const T4<T>* __restrict__ U1,
+                                           const T4<T>* __restrict__ U2, int cs, int x, int y, int z, Cons<T> v[7],
+                                           bool ok[7]) {
+  constexpr int N = 7;
+  Spot sp[7];
+  spots(tab, cs, x, y, z, sp);
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    v[k].a = U1[sp[k].cell];
+    v[k].b = U2[sp[k].cell];
+    ok[k] = true;
+  }
+  __builtin_amdgcn_sched_barrier(0);
+  int rest = 0;
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const T zero = v[k].a.x * T(0);   // as u_near
+    v[k].a.y = v[k].a.y + zero;
+    v[k].a.z = v[k].a.z + zero;
+    v[k].a.w = v[k].a.w + zero;
+    rest |= sp[k].ok ? 0 : 1 << k;
+  }
+  // (one copy of the general form, in a loop over what is left)
+  while (rest) {
+    const int k = __ffs(rest) - 1;
+    rest &= rest - 1;
+    int c[3];
+    stencil_at(k, x, y, z, c);
+    Cons<T> u;
+    const bool got = u_near<T>(tab, U1, U2, cs, c[0], c[1], c[2], u);
+#pragma unroll
+    for (int j = 0; j < N; j++)
+      if (j == k) {
+        v[j] = u;
+        ok[j] = got;
+      }
+  }
+}
+
 // Per-block timesteps: whether block s starts a step on the substep (blk_active,
 // amr/bins_on.wgsl:14-17), and its own step (blk_dt, amr/blk_dt.wgsl)
 __device__ __forceinline__ bool bins_active(const AmrBins& B, int s) {
@@ -221,43 +309,55 @@ __device__ __forceinline__ Cons<T> slope_between(const Params<T>& P, const Cons<
 // prolong_slopes / prolong_child (amr/cons.wgsl:83-124): the fine child of parity (px, py, pz)
 // of a coarse cell, from the 7-cell stencil (centre, -x, +x, -y, +y, -z, +z); one common
 // scale-back keeps rho, E and e of every child at least half the coarse cell's
+template <typename T>
+struct Prolong {
+  Cons<T> c, sx, sy, sz;   // the coarse cell and its slopes along the axes
+  T fit;
+  __device__ __forceinline__ Cons<T> child(int px, int py, int pz) const {
+    const T ox = fit * (T(px) - T(0.5)) * T(0.5);
+    const T oy = fit * (T(py) - T(0.5)) * T(0.5);
+    const T oz = fit * (T(pz) - T(0.5)) * T(0.5);
+    Cons<T> o;
+#define SHX_PRO(F) o.F = ((c.F + ox * sx.F) + oy * sy.F) + oz * sz.F
+    SHX_PRO(a.x); SHX_PRO(a.y); SHX_PRO(a.z); SHX_PRO(a.w);
+    SHX_PRO(b.x); SHX_PRO(b.y); SHX_PRO(b.z); SHX_PRO(b.w);
+#undef SHX_PRO
+    return o;
+  }
+};
 template <typename T, int LIM>
-__device__ __forceinline__ Cons<T> prolong(const Params<T>& P, const Cons<T> v[7], const bool ok[7], int px, int py,
-                                           int pz) {
+__device__ __forceinline__ Prolong<T> prolong(const Params<T>& P, const Cons<T> v[7], const bool ok[7]) {
   const Cons<T> z{v4<T>(0, 0, 0, 0), v4<T>(0, 0, 0, 0)};
-  const Cons<T> sx = (ok[1] && ok[2]) ? slope_between<T, LIM>(P, v[0], v[1], v[2]) : z;
-  const Cons<T> sy = (ok[3] && ok[4]) ? slope_between<T, LIM>(P, v[0], v[3], v[4]) : z;
-  const Cons<T> sz = (ok[5] && ok[6]) ? slope_between<T, LIM>(P, v[0], v[5], v[6]) : z;
-  const Cons<T>& c = v[0];
+  Prolong<T> g;
+  g.c = v[0];
+  g.sx = (ok[1] && ok[2]) ? slope_between<T, LIM>(P, v[0], v[1], v[2]) : z;
+  g.sy = (ok[3] && ok[4]) ? slope_between<T, LIM>(P, v[0], v[3], v[4]) : z;
+  g.sz = (ok[5] && ok[6]) ? slope_between<T, LIM>(P, v[0], v[5], v[6]) : z;
   T fit = T(1);
   {
-    T d0 = ((T(0) + tabs(sx.a.x)) + tabs(sy.a.x)) + tabs(sz.a.x);
-    T d1 = ((T(0) + tabs(sx.b.x)) + tabs(sy.b.x)) + tabs(sz.b.x);
-    T d2 = ((T(0) + tabs(sx.b.y)) + tabs(sy.b.y)) + tabs(sz.b.y);
-    T r0 = T(0.5) * tmax(c.a.x, T(0)), r1 = T(0.5) * tmax(c.b.x, T(0)), r2 = T(0.5) * tmax(c.b.y, T(0));
+    T d0 = ((T(0) + tabs(g.sx.a.x)) + tabs(g.sy.a.x)) + tabs(g.sz.a.x);
+    T d1 = ((T(0) + tabs(g.sx.b.x)) + tabs(g.sy.b.x)) + tabs(g.sz.b.x);
+    T d2 = ((T(0) + tabs(g.sx.b.y)) + tabs(g.sy.b.y)) + tabs(g.sz.b.y);
+    T r0 = T(0.5) * tmax(g.c.a.x, T(0)), r1 = T(0.5) * tmax(g.c.b.x, T(0)), r2 = T(0.5) * tmax(g.c.b.y, T(0));
     fit = tmin(fit, tmin(T(1), tdiv(r0, tmax(T(0.25) * d0, T(1e-37)))));
     fit = tmin(fit, tmin(T(1), tdiv(r1, tmax(T(0.25) * d1, T(1e-37)))));
     fit = tmin(fit, tmin(T(1), tdiv(r2, tmax(T(0.25) * d2, T(1e-37)))));
   }
-  const T ox = fit * (T(px) - T(0.5)) * T(0.5);
-  const T oy = fit * (T(py) - T(0.5)) * T(0.5);
-  const T oz = fit * (T(pz) - T(0.5)) * T(0.5);
-  Cons<T> o;
-#define SHX_PRO(F) o.F = ((c.F + ox * sx.F) + oy * sy.F) + oz * sz.F
-  SHX_PRO(a.x); SHX_PRO(a.y); SHX_PRO(a.z); SHX_PRO(a.w);
-  SHX_PRO(b.x); SHX_PRO(b.y); SHX_PRO(b.z); SHX_PRO(b.w);
-#undef SHX_PRO
-  return o;
+  g.fit = fit;
+  return g;
 }
 
 // from_coarse (amr/assemble.wgsl:47-75): texel (x, y, z) of block `slot` interpolated from the
-// coarser leaf cs. n0 = level-0 cells per axis. In 2D the z neighbours are left unread (not ok).
+// coarser leaf cs: the slopes of its coarse cell, and the texel's parity there (the other fine
+// texels of that cell are the same slopes' other children). n0 = level-0 cells per axis. In 2D the
+// z neighbours are left unread (not ok).
 template <typename T, int LIM, int D = 3>
-__device__ __forceinline__ Cons<T> from_coarse(const Params<T>& P, const int* __restrict__ tab,
+__device__ __forceinline__ Prolong<T> coarse_cell(const Params<T>& P, const int* __restrict__ tab,
                                                const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, int slot,
-                                               int x, int y, int z, int cs, const AmrBins& B = AmrBins{}) {
+                                               int x, int y, int z, int cs, int par[3],
+                                               const AmrBins& B = AmrBins{}) {
   const int lc = bt(tab, cs, BT_LEVEL);
-  int c[3], par[3];
+  int c[3];
   const int l[3] = {x, y, z};
 #pragma unroll
   for (int a = 0; a < 3; a++) {
@@ -290,18 +390,26 @@ __device__ __forceinline__ Cons<T> from_coarse(const Params<T>& P, const int* __
       v[6] = mid_cons<T, D>(P, B, cs, c[0], c[1], c[2] + 1);
       ok[5] = ok[6] = true;
     }
-    return prolong<T, LIM>(P, v, ok, par[0], par[1], par[2]);
+    return prolong<T, LIM>(P, v, ok);
   }
-  ok[0] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1], c[2], v[0]);
-  ok[1] = u_near<T, D>(tab, U1, U2, cs, c[0] - 1, c[1], c[2], v[1]);
-  ok[2] = u_near<T, D>(tab, U1, U2, cs, c[0] + 1, c[1], c[2], v[2]);
-  ok[3] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1] - 1, c[2], v[3]);
-  ok[4] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1] + 1, c[2], v[4]);
   if constexpr (D == 3) {
-    ok[5] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1], c[2] - 1, v[5]);
-    ok[6] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1], c[2] + 1, v[6]);
+    near_cells<T>(tab, U1, U2, cs, c[0], c[1], c[2], v, ok);
+  } else {
+    ok[0] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1], c[2], v[0]);
+    ok[1] = u_near<T, D>(tab, U1, U2, cs, c[0] - 1, c[1], c[2], v[1]);
+    ok[2] = u_near<T, D>(tab, U1, U2, cs, c[0] + 1, c[1], c[2], v[2]);
+    ok[3] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1] - 1, c[2], v[3]);
+    ok[4] = u_near<T, D>(tab, U1, U2, cs, c[0], c[1] + 1, c[2], v[4]);
   }
-  return prolong<T, LIM>(P, v, ok, par[0], par[1], par[2]);
+  return prolong<T, LIM>(P, v, ok);
+}
+template <typename T, int LIM, int D = 3>
+__device__ __forceinline__ Cons<T> from_coarse(const Params<T>& P, const int* __restrict__ tab,
+                                               const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, int slot,
+                                               int x, int y, int z, int cs, const AmrBins& B = AmrBins{}) {
+  int par[3];
+  const Prolong<T> g = coarse_cell<T, LIM, D>(P, tab, U1, U2, slot, x, y, z, cs, par, B);
+  return g.child(par[0], par[1], par[2]);
 }
 
 // The assembled primitives of texel (x, y, z) of block `slot`; false for edges and corners.
@@ -878,11 +986,12 @@ __global__ __launch_bounds__(256) void k_amr_regrid(Params<T> P, const int* __re
         ok[k] = u_near<T, D>(told, U1, U2, m.z, at[0], at[1], at[2], v[k]);
       }
     }
-    u = prolong<T, LIM>(P, v, ok, x & 1, y & 1, z & 1);
+    const Prolong<T> gr = prolong<T, LIM>(P, v, ok);
+    u = gr.child(x & 1, y & 1, z & 1);
     T ke = T(0);
     for (int k = 0; k < (D == 3 ? 2 : 1); k++)
       for (int j = 0; j < 2; j++)
-        for (int i = 0; i < 2; i++) ke = ke + ke_of(P, prolong<T, LIM>(P, v, ok, i, j, k));
+        for (int i = 0; i < 2; i++) ke = ke + ke_of(P, gr.child(i, j, k));
     ke = ke * (D == 3 ? T(0.125) : T(0.25));
     u.b.x = ke_of(P, u) + u.b.y + ((v[0].b.x - v[0].b.y) - ke);
   }
@@ -998,8 +1107,8 @@ struct AmrImpl {
                          (const T4<T>*)u1, (const T4<T>*)u2, part);
     hipLaunchKernelGGL(k_diag_final<T>, dim3(1), dim3(32 * DIAG_CH), 0, L.stream, (const double*)part, count, out);
   }
-  static void shell(const AmrLaunch& L, const int* work0, int n0, const int* work1, int n1, const int* work2, int n2,
-                    const void* u1, const void* u2, void* sh, const void* clk);
+  static void shell(const AmrLaunch& L, const int* shell_of, const int* work0, int n0, const int* work1, int n1,
+                    const int* work2, int n2, const void* u1, const void* u2, void* sh, const void* clk);
   static void fused(const AmrLaunch& L, const AmrQueue& Q, const void* sh, const void* u1, const void* u2, void* o1,
                     void* o2, const void* clk, unsigned long long* slot);
   static void regrid(const AmrLaunch& Lold, const int* map, int count, const void* u1, const void* u2, void* n1a,

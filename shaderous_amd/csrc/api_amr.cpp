@@ -424,9 +424,9 @@ int enqueue_step(shx_amr* s, int p, int stage = -1) {
   if (s->lay.path == SHX_AMR_PATH_FUSED) {
     if (run(1)) { o.clock(L, s->clk, s->slot); n++; }
     if (run(2)) {
-      o.shell(L, s->d_shw[0], s->nshw[0], s->d_shw[1], s->nshw[1], s->d_shw[2], s->nshw[2], s->U1[p], s->U2[p],
+      o.shell(L, s->d_shell_of, s->d_shw[0], s->nshw[0], s->d_shw[1], s->nshw[1], s->d_shw[2], s->nshw[2], s->U1[p], s->U2[p],
               s->shell, s->clk);
-      n += (s->nshw[0] > 0) + (s->nshw[1] > 0) + (s->nshw[2] > 0);
+      n += (s->nshw[0] > 0) + (s->nshw[1] + s->nshw[2] > 0);
     }
     if (run(3) && s->queue.count > 0) {
       AmrQueue Q{lp(s, s->queue), s->queue.count, s->grid, s->d_shell_of, s->d_act, s->reg, s->cf, s->d_reg_of,
@@ -890,7 +890,10 @@ int shx_amr_create(const shx_config* cfg, const shx_amr_layout* layout, const in
           rim.push_back({nb, cell, i, h});
         }
       } else {
-        for (int c = 0; c < 8; c++) add(0, c);
+        // beside a coarser block one wave per face, a lane per coarse cell (8)
+        if (nb == -1) add(0, 8);
+        else
+          for (int c = 0; c < 8; c++) add(0, c);
         // half steps beside a boundary image only: beside a coarser block the march predicts
         // them in place, and beside a refined block the faces are the children's means (the
         // coarse-face buffer replaces what those half steps would give)
