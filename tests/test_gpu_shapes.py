@@ -5,7 +5,8 @@ there is no tolerance."""
 import numpy as np
 import pytest
 
-from shaderous_amd import problems
+from shaderous_amd import amr_tree, problems
+from shaderous_amd.amr import AmrSim
 from shaderous_amd.ensemble import Ensemble
 from shaderous_amd.sim import Sim, SimConfig, config_for
 
@@ -67,3 +68,34 @@ def test_runs_of_steps_of_an_ensemble_equal_single_steps():
         ens.destroy()
     for a, b in zip(*out):
         assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+@pytest.mark.parametrize("cells,levels,walls", [((3, 3, 3), 0, False), ((8, 8, 7), 0, False), ((8, 8, 8), 0, True),
+                                                ((4, 4, 4), 2, True), ((8, 8, 8), 2, False)])
+def test_march_queue_equals_passes_bitwise(cells, levels, walls, precision):
+    """The fused march's queue on meshes of one round and several, whose last round holds single
+    blocks or pairs, with leaves that wait for finer ones at two levels: the passes' bits."""
+    if levels:
+        blocks, dx0, prim = problems.amr_blast(seed=3, root=cells[0], max_level=levels)[:3]
+    else:
+        blocks = np.array([(0, x, y, z) for z in range(cells[2]) for y in range(cells[1]) for x in range(cells[0])],
+                          dtype=np.int32)
+        dx0, prim = problems.amr_blast(seed=3, root=4, max_level=0)[1:3]
+    u1, u2 = amr_tree.blocks_state(blocks, dx0, prim, 1.4, ndim=3)
+    bc = (2, 1, 0) if walls else (0, 0, 0)
+    cfg = SimConfig(n=tuple(16 * c for c in cells), dx=dx0, gamma=1.4, cfl=0.4, bc_lo=bc, bc_hi=bc, limiter="mc",
+                    isentropic=False, precision=precision)
+    t = np.float64 if precision == 64 else np.float32
+    out = []
+    for path in ("passes", "fused"):
+        sim = AmrSim(cfg, blocks, cells, path=path)
+        sim.set_state(u1.astype(t), u2.astype(t))
+        sim.step(3)
+        out.append((*sim.read_state(), sim.clock()))
+        sim.destroy()
+    leaves = np.repeat(amr_tree.leaf_mask(blocks), 4096)
+    assert np.all(np.isfinite(out[0][0]))
+    for a, b in zip(out[0][:2], out[1][:2]):
+        assert np.array_equal(a.reshape(-1, 4)[leaves], b.reshape(-1, 4)[leaves])
+    assert np.array_equal(out[0][2], out[1][2])
