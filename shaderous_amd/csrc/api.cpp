@@ -8,12 +8,14 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
 #include <string>
 #include <vector>
 
 #include "../../include/shx.h"
 #include "common.hpp"
 #include "ens_impl.hpp"
+#include "state_reader.hpp"
 #include "uniform.hpp"
 
 using namespace shx;
@@ -33,6 +35,7 @@ int fail(int code, const char* fmt, ...) {
 
 struct shx_sim {
   shx_config cfg;
+  std::unique_ptr<StateReader> rb{new StateReader};
   int es;                    // element size: 4 or 8
   size_t ncell;
   hipStream_t stream = nullptr;
@@ -200,9 +203,7 @@ int read_state_t(shx_sim* s, T* u1, T* u2) {
   if (!s) return fail(SHX_EINVAL, "null sim");
   if ((int)sizeof(T) != s->es) return fail(SHX_EINVAL, "state precision mismatch");
   size_t bytes = s->ncell * 4 * sizeof(T);
-  HIPCHK(hipMemcpyAsync(u1, s->U1[s->cur], bytes, hipMemcpyDeviceToHost, s->stream));
-  HIPCHK(hipMemcpyAsync(u2, s->U2[s->cur], bytes, hipMemcpyDeviceToHost, s->stream));
-  HIPCHK(hipStreamSynchronize(s->stream));
+  HIPCHK(s->rb->read(s->stream, s->cfg.device, u1, s->U1[s->cur], u2, s->U2[s->cur], bytes));
   return SHX_OK;
 }
 
@@ -493,6 +494,7 @@ int shx_create(const shx_config* cfg, shx_sim** out) {
   }
   int rc = build_graphs(s);
   if (rc) { shx_destroy(s); return rc; }
+  s->rb->fit(2 * bytes);
   *out = s;
   return SHX_OK;
 }

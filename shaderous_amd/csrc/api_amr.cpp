@@ -8,6 +8,7 @@
 
 #include <algorithm>
 #include <array>
+#include <memory>
 #include <string>
 #include <unordered_map>
 #include <unordered_set>
@@ -15,6 +16,7 @@
 
 #include "amr.hpp"
 #include "common.hpp"
+#include "state_reader.hpp"
 
 using namespace shx;
 
@@ -28,6 +30,7 @@ struct Range {
 
 struct shx_amr {
   shx_config cfg;
+  std::unique_ptr<StateReader> rb{new StateReader};
   shx_amr_layout lay;
   int ndim = 3;
   int cells = AMR_CELLS;     // per block: 16^ndim cells, 20^ndim atlas texels
@@ -596,9 +599,7 @@ int read_state_t(shx_amr* s, T* u1, T* u2) {
   if (!s) return fail(SHX_EINVAL, "null sim");
   if ((int)sizeof(T) != s->es) return fail(SHX_EINVAL, "state precision mismatch");
   const size_t bytes = s->ncell * 4 * sizeof(T);
-  HIPCHK(hipMemcpyAsync(u1, s->U1[s->cur], bytes, hipMemcpyDeviceToHost, s->stream));
-  HIPCHK(hipMemcpyAsync(u2, s->U2[s->cur], bytes, hipMemcpyDeviceToHost, s->stream));
-  HIPCHK(hipStreamSynchronize(s->stream));
+  HIPCHK(s->rb->read(s->stream, s->cfg.device, u1, s->U1[s->cur], u2, s->U2[s->cur], bytes));
   return check_queue(s);
 }
 
@@ -793,8 +794,8 @@ int run_cycle(shx_amr* s) {
 
 extern "C" {
 
-int shx_amr_create(const shx_config* cfg, const shx_amr_layout* layout, const int* blocks, int nblocks,
-                   shx_amr** out) {
+// (all but the slots of its reads)
+static int create(const shx_config* cfg, const shx_amr_layout* layout, const int* blocks, int nblocks, shx_amr** out) {
   if (!cfg || !layout || !blocks || !out || nblocks < 1) return fail(SHX_EINVAL, "null argument or no blocks");
   *out = nullptr;
   const shx_config& c = *cfg;
@@ -1002,6 +1003,13 @@ int shx_amr_create(const shx_config* cfg, const shx_amr_layout* layout, const in
   if (rc) { shx_amr_destroy(s); return rc; }
   *out = s;
   return SHX_OK;
+}
+
+int shx_amr_create(const shx_config* cfg, const shx_amr_layout* layout, const int* blocks, int nblocks,
+                   shx_amr** out) {
+  const int rc = create(cfg, layout, blocks, nblocks, out);
+  if (rc == SHX_OK) (*out)->rb->fit(2 * (*out)->ncell * 4 * (*out)->es);
+  return rc;
 }
 
 int shx_amr_destroy(shx_amr* s) {
@@ -1244,7 +1252,7 @@ int shx_amr_regrid(shx_amr* s, const int* blocks, int nblocks) {
   if (rc != SHX_OK) return rc;
   // the new tree's sim (validates the tree and allocates its memory), then the state moved over
   shx_amr* ns = nullptr;
-  rc = shx_amr_create(&s->cfg, &s->lay, blocks, nblocks, &ns);
+  rc = create(&s->cfg, &s->lay, blocks, nblocks, &ns);
   if (rc != SHX_OK) return rc;
   int* d_map = nullptr;
   const int count = (int)(map.size() / 4);
@@ -1273,6 +1281,8 @@ int shx_amr_regrid(shx_amr* s, const int* blocks, int nblocks) {
     }
   }
   std::swap(*s, *ns);
+  std::swap(s->rb, ns->rb);   // its slots stay; more of them if the state has outgrown them
+  s->rb->fit(2 * s->ncell * 4 * s->es);
   shx_amr_destroy(ns);
   return SHX_OK;
 }

@@ -5,15 +5,18 @@
 #include <string.h>
 
 #include <algorithm>
+#include <memory>
 #include <vector>
 
 #include "common.hpp"
 #include "ens_impl.hpp"
+#include "state_reader.hpp"
 
 using namespace shx;
 
 struct shx_ens {
   shx_config cfg;
+  std::unique_ptr<StateReader> rb{new StateReader};
   int es = 4;
   int count = 0;
   std::vector<int> nx, ny;
@@ -118,9 +121,8 @@ int read_state_t(shx_ens* e, int i, T* u1, T* u2) {
   if (!e || i < 0 || i >= e->count) return fail(SHX_EINVAL, "bad instance");
   if ((int)sizeof(T) != e->es) return fail(SHX_EINVAL, "state precision mismatch");
   const size_t n = (size_t)e->nx[i] * e->ny[i];
-  HIPCHK(hipMemcpyAsync(u1, (char*)e->U1[e->cur] + e->off[i] * 4 * sizeof(T), n * 4 * sizeof(T), hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(hipMemcpyAsync(u2, (char*)e->U2[e->cur] + e->off[i] * 4 * sizeof(T), n * 4 * sizeof(T), hipMemcpyDeviceToHost, e->stream));
-  HIPCHK(hipStreamSynchronize(e->stream));
+  const size_t at = e->off[i] * 4 * sizeof(T);
+  HIPCHK(e->rb->read(e->stream, e->cfg.device, u1, (char*)e->U1[e->cur] + at, u2, (char*)e->U2[e->cur] + at, n * 4 * sizeof(T)));
   return SHX_OK;
 }
 
@@ -241,6 +243,9 @@ int shx_ens_create(const shx_config* cfg, int count, const int* sizes, shx_ens**
   }
   int rc = build_graphs(e);
   if (rc) { shx_ens_destroy(e); return rc; }
+  size_t largest = 0;
+  for (int i = 0; i < count; i++) largest = std::max(largest, (size_t)e->nx[i] * e->ny[i]);
+  e->rb->fit(2 * largest * 4 * e->es);
   *out = e;
   return SHX_OK;
 }
