@@ -101,6 +101,15 @@ struct AmrOps {
                 const int* work2, int n2, const void* u1, const void* u2, void* sh, const void* clk);
   void (*fused)(const AmrLaunch&, const AmrQueue& Q, const void* sh, const void* u1, const void* u2, void* o1, void* o2,
                 const void* clk, unsigned long long* slot);
+  // 2D blocks in FP32: the listed leaves' ghosts (into w1, w2 and the corners of pa, pb) and rate;
+  // then the rest of the step of the listed leaves, the first nfull of them; of the others only the
+  // fluxes of their faces on a coarser block. match: the leaves have refined neighbours, whose
+  // fluxes an earlier launch left in the register
+  void (*flat_ghosts)(const AmrLaunch&, const int* list, int count, const void* u1, const void* u2, void* w1, void* w2,
+                      void* pa, void* pb, unsigned long long* slot);
+  void (*flat)(const AmrLaunch&, const int* list, int nfull, int count, bool match, bool compensated,
+               const int* reg_of, void* reg, const void* u1, const void* u2, const void* w1, const void* w2,
+               const void* pa, const void* pb, void* o1, void* o2, const void* clk);
   // re-meshing: `count` new leaves listed as int4 (new slot, kind 1 copy / 2 prolong / 3
   // restrict, old slot, child octant), from the old tree (L: its table, params, stream) and
   // state into both buffers of the new state

@@ -1,7 +1,7 @@
-// FP32 block-AMR kernels for 2D grids (quadtrees of 16^2-cell blocks), the passes forms (plain
-// per level and batched): PLM with MC, van Leer or minmod (HLLC or HLL) and the reference
+// FP32 block-AMR kernels for 2D grids (quadtrees of 16^2-cell blocks), the passes plain per
+// level, and the batched step in one kernel: PLM with MC, van Leer or minmod (HLLC or HLL) and the reference
 // defaults (Koren with HLLC or HLL, with or without the density reconstruction along the adiabat).
-#include "amr_impl.hpp"
+#include "amr2d.hpp"
 namespace shx {
 AmrOps amr2d_ops_f32(int lim, int rs, int isen) {
   const bool c = rs == RS_HLLC;

@@ -459,7 +459,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
     // this block's cell size (P is the kernel's own copy: its dx is the block's from here on)
     const T dx = dx0 * (T(1) / T(1 << bt(tab, s, BT_LEVEL)));
     P.dx = dx;
-    const T dtdx = wave_uniform(dt / dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
+    const T dtdx = wave_uniform(tratio(dt, dx)), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
     // the faces' actions (boundary_face)
     int fa[6];
 #pragma unroll

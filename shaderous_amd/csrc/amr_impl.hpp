@@ -910,7 +910,7 @@ __global__ __launch_bounds__(UpdTile<D>::NT) void k_amr_update(
   Pl.dx = dx;
   const T dt = B.k ? clk[0] * T(1 << gbin) : clk[0];
   T4<T> o1, o2;
-  advance(Pl, U1[o], U2[o], net, PB[(size_t)s * AmrGeo<D>::TEXELS + texd<D>(x, y, z)].x, dt / dx, o1, o2);
+  advance(Pl, U1[o], U2[o], net, PB[(size_t)s * AmrGeo<D>::TEXELS + texd<D>(x, y, z)].x, tratio(dt, dx), o1, o2);
   O1[o] = o1;
   O2[o] = o2;
 }
@@ -1111,6 +1111,11 @@ struct AmrImpl {
                     const int* work2, int n2, const void* u1, const void* u2, void* sh, const void* clk);
   static void fused(const AmrLaunch& L, const AmrQueue& Q, const void* sh, const void* u1, const void* u2, void* o1,
                     void* o2, const void* clk, unsigned long long* slot);
+  static void flat_ghosts(const AmrLaunch& L, const int* list, int count, const void* u1, const void* u2, void* w1,
+                          void* w2, void* pa, void* pb, unsigned long long* slot);
+  static void flat(const AmrLaunch& L, const int* list, int nfull, int count, bool match, bool compensated,
+                   const int* reg_of, void* reg, const void* u1, const void* u2, const void* w1, const void* w2,
+                   const void* pa, const void* pb, void* o1, void* o2, const void* clk);
   static void regrid(const AmrLaunch& Lold, const int* map, int count, const void* u1, const void* u2, void* n1a,
                      void* n2a, void* n1b, void* n2b) {
     if (count <= 0) return;
@@ -1155,6 +1160,12 @@ struct AmrImpl {
     } else {
       o.shell = nullptr;
       o.fused = nullptr;
+    }
+    o.flat = nullptr;
+    o.flat_ghosts = nullptr;
+    if constexpr (D == 2 && sizeof(T) == 4) {
+      o.flat = flat;
+      o.flat_ghosts = flat_ghosts;
     }
     o.assemble = assemble;
     o.clock = clock;

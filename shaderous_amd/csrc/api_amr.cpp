@@ -48,6 +48,7 @@ struct shx_amr {
   // same split per level
   Range all, leaf, plain, match;
   Range queue;   // the fused march's queue (-1 pads)
+  Range supply;  // the flat step's first launch: the plain leaves, then the matched ones with a coarser neighbour
   Range all_lv[AMR_MAXLEV], leaf_lv[AMR_MAXLEV], plain_lv[AMR_MAXLEV], match_lv[AMR_MAXLEV];
   void* U1[2] = {nullptr, nullptr};
   void* U2[2] = {nullptr, nullptr};
@@ -388,6 +389,13 @@ int build_lists(shx_amr* s, std::vector<int>& lists) {
   add(s->leaf, [&](int i) { return is_leaf(i); });
   add(s->plain, [&](int i) { return is_leaf(i) && !has_fine(i); });
   add(s->match, [&](int i) { return is_leaf(i) && has_fine(i); });
+  add(s->supply, [&](int i) { return is_leaf(i) && !has_fine(i); });
+  for (int i : order) {
+    bool has_coarse = false;
+    for (int f = 0; f < 6; f++) has_coarse = has_coarse || s->tab[(size_t)i * AMR_BT + BT_NB + f] == -1;
+    if (is_leaf(i) && has_fine(i) && has_coarse) lists.push_back(i);
+  }
+  s->supply.count = (int)lists.size() - s->supply.off;
   // the fused march's queue. A leaf beside a refined block (has_fine) waits for the finer leaves
   // across it, so the levels' leaves with a coarse-fine face come level by level from the finest:
   // first those that only supply (has_coarse alone), then the waiting ones. A workgroup that takes
@@ -471,6 +479,23 @@ int enqueue_step(shx_amr* s, int p, int stage = -1) {
       o.fused(L, Q, s->shell, s->U1[p], s->U2[p], s->U1[1 - p], s->U2[1 - p], s->clk, s->slot);
       n += 2;
     }
+    return n;
+  }
+  if (o.flat && !levels && s->kbins == 0) {
+    // 2D in FP32: ghosts and rate, clock, then the leaves in two launches of the rest
+    if (run(0)) {
+      o.flat_ghosts(L, lp(s, s->leaf), s->leaf.count, s->U1[p], s->U2[p], s->W1, s->W2, s->PA, s->PB, s->slot);
+      n++;
+    }
+    if (run(1)) { o.clock(L, s->clk, s->slot); n++; }
+    auto part = [&](const Range& r, int nfull, bool match) {
+      if (!r.count) return;
+      o.flat(L, lp(s, r), nfull, r.count, match, comp, s->d_reg_of, s->reg, s->U1[p], s->U2[p], s->W1, s->W2, s->PA,
+             s->PB, s->U1[1 - p], s->U2[1 - p], s->clk);
+      n++;
+    };
+    if (run(2)) part(s->supply, s->plain.count, false);
+    if (run(3)) part(s->match, s->match.count, true);
     return n;
   }
   if (run(0)) {

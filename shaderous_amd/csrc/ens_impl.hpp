@@ -100,7 +100,7 @@ __global__ __launch_bounds__(BX* BY, (ens_minw<T, LIM, BX * BY, SINGLE>())) void
     const size_t o = off + (size_t)my.i * nx + mx.i;
     const T4<T> u1 = U1[o], u2 = U2[o];
     const T dt = step_dt(P, C, w.inst);
-    const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
+    const T dtdx = wave_uniform(tratio(dt, P.dx)), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
     const bool real_x = x >= 0 && x < nx, real_y = y >= 0 && y < ny;
     const bool cell = tx >= 2 && tx <= BX - 3 && ty >= 2 && ty <= BY - 3 && real_x && real_y;
     const bool xface = tx >= 2 && tx <= BX - 2 && ty >= 2 && ty <= BY - 3 && x <= nx && real_y;
@@ -247,7 +247,7 @@ __global__ __launch_bounds__(64) void k_ens_rows(const EnsInst<float>* __restric
   const long long off = inst[w.inst].off;
   const int nx = P.n[0], ny = P.n[1];
   const T dt = step_dt(P, C, w.inst);
-  const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
+  const T dtdx = wave_uniform(tratio(dt, P.dx)), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
   const int lane = threadIdx.x;
   if (blockIdx.x == 0)
     for (int i = lane; i < ninst; i += 64) step_clock_advance(inst[i].P, C, i);

@@ -81,6 +81,14 @@ __device__ __forceinline__ float trcp(float b) { return __builtin_amdgcn_rcpf(b)
 __device__ __forceinline__ double trcp(double b) { return 1.0 / b; }
 __device__ __forceinline__ float tdiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 __device__ __forceinline__ double tdiv(double a, double b) { return a / b; }
+// A quotient that several kernels form for themselves and that has to be the same in each (a step
+// over a cell size): spelled out, as the compiler lowers a plain a / b to a correctly rounded or an
+// approximate form by what stands around it. To half an ulp and a little.
+__device__ __forceinline__ float tratio(float a, float b) {
+  const float r = __builtin_amdgcn_rcpf(b), q = a * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
+}
+__device__ __forceinline__ double tratio(double a, double b) { return a / b; }
 __device__ __forceinline__ float tsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ double tsqrt(double x) { return __builtin_sqrt(x); }
 // Single-precision pow as WGSL defines it, exp2(b log2 a) (every base here is positive), by the
@@ -357,7 +365,7 @@ __device__ __forceinline__ AxisSlope<T> axis_slope(const Params<T>& P, const Pri
 // What the half step multiplies an axis's slope by: half a step's dt / dx for a whole slope
 template <typename T, int LIM>
 __device__ __forceinline__ T slope_step(const Params<T>& P, T dt) {
-  return lim_symmetric<LIM>() ? dt / P.dx : T(0.5) * dt / P.dx;
+  return lim_symmetric<LIM>() ? tratio(dt, P.dx) : tratio(T(0.5) * dt, P.dx);
 }
 
 // Shock detector (predictor.wgsl:114-134): converging flow and a relative pressure jump across

@@ -351,7 +351,7 @@ __global__ __launch_bounds__(WX* WY* WZ) void k_update(Params<T> P, const T4<T>*
     return;
   }
   Flux<T> net = net_of(xl, xh, yl, yh, zl, zh);
-  T dtdx = clk[0] / P.dx;
+  T dtdx = tratio(clk[0], P.dx);
   T4<T> o1, o2;
   advance(P, U1[o], U2[o], net, PB[o].x, dtdx, o1, o2);
   O1[o] = o1;
@@ -473,7 +473,7 @@ __global__ __launch_bounds__(BX* BY, (sizeof(T) == 4 ? 4 : 1)) void k_fused(
   const int z0 = blockIdx.z * zc;
   const int z1 = min(z0 + zc, nz);
   const T dt = step_dt(P, C, 0);
-  const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
+  const T dtdx = wave_uniform(tratio(dt, P.dx)), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
   if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && t == 0) step_clock_advance(P, C, 0);
 
   // this column's source through the x/y boundaries (clamped in range for the ragged rim,

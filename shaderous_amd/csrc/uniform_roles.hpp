@@ -273,7 +273,7 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile
   const int z0 = bz * zc;
   const int z1 = min(z0 + zc, nz);
   const T dt = step_dt(P, C, 0);
-  const T dtdx = wave_uniform(dt / P.dx), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
+  const T dtdx = wave_uniform(tratio(dt, P.dx)), hstep = wave_uniform(slope_step<T, LIM>(P, dt));
   if (blockIdx.x == 0 && blockIdx.y == 0 && blockIdx.z == 0 && tid == 0) step_clock_advance(P, C, 0);
 
   const size_t plane = (size_t)nx * ny;

@@ -81,7 +81,8 @@ def test_march_queue_equals_passes_bitwise(cells, levels, walls, precision):
     else:
         blocks = np.array([(0, x, y, z) for z in range(cells[2]) for y in range(cells[1]) for x in range(cells[0])],
                           dtype=np.int32)
-        dx0, prim = problems.amr_blast(seed=3, root=4, max_level=0)[1:3]
+        prim = problems.amr_blast(seed=3, root=4, max_level=0)[2]
+        dx0 = 1 / (16 * cells[0])
     u1, u2 = amr_tree.blocks_state(blocks, dx0, prim, 1.4, ndim=3)
     bc = (2, 1, 0) if walls else (0, 0, 0)
     cfg = SimConfig(n=tuple(16 * c for c in cells), dx=dx0, gamma=1.4, cfl=0.4, bc_lo=bc, bc_hi=bc, limiter="mc",
@@ -96,6 +97,45 @@ def test_march_queue_equals_passes_bitwise(cells, levels, walls, precision):
         sim.destroy()
     leaves = np.repeat(amr_tree.leaf_mask(blocks), 4096)
     assert np.all(np.isfinite(out[0][0]))
+    for a, b in zip(out[0][:2], out[1][:2]):
+        assert np.array_equal(a.reshape(-1, 4)[leaves], b.reshape(-1, 4)[leaves])
+    assert np.array_equal(out[0][2], out[1][2])
+
+
+@pytest.mark.parametrize("scheme", [("mc", False, "hllc"), ("koren", True, "hllc"), ("vanleer", False, "hll"),
+                                    ("koren", False, "hll")])
+@pytest.mark.parametrize("root,levels,bc,compensated", [((4, 4, 1), 2, (0, 0, 0), True), ((4, 4, 1), 2, (2, 2, 0), False),
+                                                        ((8, 8, 1), 3, (0, 1, 0), True), ((8, 8, 1), 1, (1, 2, 0), True),
+                                                        ((1, 1, 1), 0, (0, 0, 0), True), ((3, 2, 1), 0, (1, 3, 0), True),
+                                                        ((5, 5, 1), 2, (0, 0, 0), True)])
+def test_flat_blocks_step_equals_the_passes_bitwise(root, levels, bc, compensated, scheme):
+    """The batched step of 2D blocks (ghosts, then the rest in one kernel) against the passes run
+    level by level: periodic, walled and outflow, faces on coarser and refined leaves."""
+    if levels:
+        blocks, dx0 = problems.kh_adaptive(root=root[0], max_level=levels)[:2]
+    else:
+        blocks = np.array([(0, x, y, 0) for y in range(root[1]) for x in range(root[0])], dtype=np.int32)
+        dx0 = 1 / (16 * root[0])
+    blocks = np.asarray(blocks, np.int32)
+    rng = np.random.default_rng(5)
+
+    def prims(x, y, z):
+        return {"rho": 1 + 0.4 * np.sin(7 * x + 3 * y) + 0.1 * rng.random(x.shape), "vx": 0.5 * np.cos(5 * y) + 0 * x,
+                "vy": 0.4 * np.sin(6 * x) + 0.05 * rng.random(x.shape), "vz": 0.1 * np.sin(4 * x) + 0 * y,
+                "p": 1 + 0.5 * rng.random(x.shape), "s": rng.random(x.shape)}
+    u1, u2 = amr_tree.blocks_state(blocks, dx0, prims, 1.4, ndim=2)
+    limiter, isen, riemann = scheme
+    cfg = SimConfig(n=(16 * root[0], 16 * root[1], 1), ndim=2, dx=dx0, gamma=1.4, cfl=0.4, bc_lo=bc, bc_hi=bc,
+                    limiter=limiter, isentropic=isen, riemann=riemann)
+    out = []
+    for path in ("levels", "passes"):
+        sim = AmrSim(cfg, blocks, root, path=path, compensated=compensated)
+        sim.set_state(u1, u2)
+        sim.step(4)
+        out.append((*sim.read_state(), sim.clock()))
+        sim.destroy()
+    leaves = np.repeat(amr_tree.leaf_mask(blocks), 256)
+    assert np.all(np.isfinite(out[0][0].reshape(-1, 4)[leaves]))
     for a, b in zip(out[0][:2], out[1][:2]):
         assert np.array_equal(a.reshape(-1, 4)[leaves], b.reshape(-1, 4)[leaves])
     assert np.array_equal(out[0][2], out[1][2])
