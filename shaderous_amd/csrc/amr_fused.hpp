@@ -229,7 +229,7 @@ __device__ __forceinline__ void shell_texels(const Params<T>& P, const int* __re
   const int n = (k & 1) ? AMR_BS + layer : -1 - layer;
   const int x = axis == 0 ? n : i, y = axis == 1 ? n : (axis == 0 ? i : j), z = axis == 2 ? n : j;
   Prim<T> w;
-  if (amr_texel<T, LIM>(P, tab, U1, U2, s, x, y, z, w)) put(x, y, z, w);
+  if (amr_texel<T, LIM, 3, false>(P, tab, U1, U2, s, x, y, z, w)) put(x, y, z, w);
 }
 
 // The half step of cell (x, y, z) of leaf `slot` (predict_cell on the source block,
