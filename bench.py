@@ -42,30 +42,32 @@ HBM_PEAK = 8.0e12          # MI355X HBM3E, bytes/s
 BYTES_PER_UPDATE = 64      # read 8 FP32 conserved values, write 8
 # HBM bytes per launch of the dominant kernel, measured with rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE (scaled by the counters' reading of a 512 MiB device copy: 2.0 and 1.0), for the
-# configuration they were measured on: profiles/k_fused_turbulence_256.md
+# configuration they were measured on: profiles/hydro_step_kernels.md
 TRAFFIC_MEASURED = {
-    ("k_fused_r", 256, (32, 8, 128)): (2 * 501524 + 524304) * 1024,
-    ("k_fused_r", 256, (16, 16, 128)): (2 * 505142 + 524306) * 1024,
-    ("k_fused_r", 256, (32, 16, 128)): (2 * 544123 + 524296) * 1024,
+    ("k_fused_r", 256, (32, 8, 64)): (2 * 515283 + 524289) * 1024,
+    ("k_fused_r", 256, (32, 8, 128)): (2 * 512333 + 524289) * 1024,
+    ("k_fused_r", 256, (16, 16, 64)): (2 * 533872 + 524289) * 1024,
+    ("k_fused_r", 256, (16, 16, 128)): (2 * 544001 + 524289) * 1024,
+    ("k_fused_r", 256, (32, 16, 128)): (2 * 394139 + 524288) * 1024,
 }
 
 
-TRAFFIC_SOURCE = "profiles/k_fused_turbulence_256.md"
+TRAFFIC_SOURCE = "profiles/hydro_step_kernels.md"
 # HBM bytes per step of the AMR blast's fused path (the ghost shell pass and the march), from
 # rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE summed over a step's kernels, scaled as above
-AMR_TRAFFIC_MEASURED = {"blast": (int((0.45 + 0.05 + 0.79 + 0.05 + 2.00 + 0.64) * 1e9),
-                                   "profiles/k_amr_fused_blast.md: k_amr_shell texels + k_amr_rim + k_amr_fused, "
+AMR_TRAFFIC_MEASURED = {"blast": ((2 * (141534 + 266171 + 922070) + 54968 + 44625 + 639282) * 1024,
+                                   "profiles/hydro_step_kernels.md: k_amr_shell texels + half steps + k_amr_fused, "
                                    "HBM read + write per step")}
 
 
 # VALU instructions (wave64) per launch of the dominant kernel, measured with rocprofv3 --pmc
-# SQ_INSTS_VALU for the configuration they were measured on (profiles/k_fused_turbulence_256.md)
+# SQ_INSTS_VALU for the configuration they were measured on (profiles/hydro_step_kernels.md)
 VALU_MEASURED = {
-    ("k_fused_r", 256, (32, 8, 64)): 286394543,
-    ("k_fused_r", 256, (32, 8, 128)): 282960418,
-    ("k_fused_r", 256, (16, 16, 64)): 265036818,
-    ("k_fused_r", 256, (16, 16, 128)): 261889406,
-    ("k_fused_r", 256, (32, 16, 128)): 253433258,
+    ("k_fused_r", 256, (32, 8, 64)): 185860728,
+    ("k_fused_r", 256, (32, 8, 128)): 184353152,
+    ("k_fused_r", 256, (16, 16, 64)): 169880688,
+    ("k_fused_r", 256, (16, 16, 128)): 168466020,
+    ("k_fused_r", 256, (32, 16, 128)): 166664508,
 }
 # MI355X VALU issue peak for FP32 without packed math: 256 CUs x 4 SIMDs x 16 lanes x 2.4 GHz
 VALU_LANE_PEAK = 256 * 4 * 16 * 2.4e9

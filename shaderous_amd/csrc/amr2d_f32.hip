@@ -1,5 +1,5 @@
-// FP32 block-AMR kernels for 2D grids (quadtrees of 16^2-cell blocks), the passes plain per
-// level, and the batched step in one kernel: PLM with MC, van Leer or minmod (HLLC or HLL) and the reference
+// FP32 block-AMR kernels for 2D grids (quadtrees of 16^2-cell blocks), the passes level by level
+// and the batched step (amr2d.hpp): PLM with MC, van Leer or minmod (HLLC or HLL) and the reference
 // defaults (Koren with HLLC or HLL, with or without the density reconstruction along the adiabat).
 #include "amr2d.hpp"
 namespace shx {

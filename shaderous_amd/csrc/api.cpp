@@ -96,7 +96,7 @@ const void* current_clock(const shx_sim* s) {
 }
 
 // The fused path's one-pass step from parity p into 1 - p (its clock pass included; after the
-// boundary planes' half steps): the 2D kernels on a flat FP32 grid, else the 3D march with tile
+// boundary planes' half steps): the 2D kernels on a flat grid, else the 3D march with tile
 // `tile`.
 void enqueue_fused(shx_sim* s, int p, int tile, int zc, bool debug) {
   if (s->flat2d && !debug) {

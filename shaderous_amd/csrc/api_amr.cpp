@@ -404,9 +404,8 @@ int build_lists(shx_amr* s, std::vector<int>& lists) {
   // and the next level's first waiting leaf go a round's worth of leaves (one for each block
   // that can march at once) that wait for nothing, as far as there are any. The rest of those
   // come last. Each level's part is padded to an even length, so a workgroup's pair never holds a
-  // leaf and a finer leaf it waits for. On the 3D blast's
-  // 1618 leaves (two levels, 3.2 rounds) the march takes 290 us so, 340 us with each level's leaves
-  // right behind the finer level's.
+  // leaf and a finer leaf it waits for. On the 3D blast's 1618 leaves (two levels, 3.2 rounds) the
+  // march takes 290 us so, 340 us with each level's leaves right behind the finer level's.
   auto has_coarse = [&](int i) {
     for (int f = 0; f < 6; f++)
       if (s->tab[(size_t)i * AMR_BT + BT_NB + f] == -1) return true;

@@ -6,7 +6,8 @@
 //   k_ens_fused   per tile (BX x BY columns, (BX - 4) x (BY - 4) cells), one plane: primitives
 //                 into LDS, the Hancock half step of the cells and the one-column ring, each face
 //                 once, the conservative update, and the next step's rate of the instance
-//                 (4 barriers per tile)
+//   k_ens_rows    per strip (60 columns x as many rows as fill the chip), one wave marching up the
+//                 rows, no LDS
 // The arithmetic is the uniform grid's, in the order of its plain 2D passes (a flat grid's z
 // neighbours are the cell itself: its half step leaves the zero z slope out, half_flat, as the
 // plain predictor does on a flat grid), so an instance gives the values of a single 2D run of

@@ -8,7 +8,8 @@
 //   k_update  hydro/update.wgsl:189-405 with the face tile (hydro/tile.wgsl:166-213): every
 //             face of the block's box computed once into LDS, then each cell's update
 //
-// FUSED path, one kernel per step (k_fused): a block owns a column tile of (BX - 4) x (BY - 4)
+// FUSED path, one kernel per step: k_fused_r (uniform_roles.hpp), threads by role, or the raster
+// form k_fused (below: planes beyond 4 GiB, and tiles asked for by their cells): a block owns a column tile of (BX - 4) x (BY - 4)
 // cells plus a two-cell halo ring and marches along z through a chunk of planes. Each plane's
 // primitives are converted once, staged in LDS for the x/y neighbours and kept in registers for
 // the z neighbours; each cell's half step and edge increments are computed once; each face is

@@ -49,20 +49,6 @@ struct RoleTile {
   }
 };
 
-// The block march's LDS (k_amr_fused), per column: primitives of two planes (rho, v, p, s: the
-// centre's sound speed stays in a register), x and y sides, x and y fluxes: 46 values
-template <int NT>
-struct RoleLayout {
-  static constexpr int Q0 = 0, Q1 = 6 * NT, SX = 12 * NT, SY = 21 * NT, FX = 30 * NT, FY = 38 * NT;
-  static constexpr int SIZE = 46 * NT;
-};
-
-template <typename T, int NT>
-__device__ __forceinline__ void lds_put_prim6(T* L, int t, const Prim<T>& q) {
-  L[0 * NT + t] = q.rho; L[1 * NT + t] = q.vx; L[2 * NT + t] = q.vy; L[3 * NT + t] = q.vz;
-  L[4 * NT + t] = q.p; L[5 * NT + t] = q.s;
-}
-
 // thread -> column (cx, cy) in cell-tile coordinates, [-2, TX + 2) x [-2, TY + 2)
 template <int TX, int TY>
 __device__ __forceinline__ void role_column(int t, int& cx, int& cy) {
