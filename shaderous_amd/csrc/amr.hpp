@@ -37,8 +37,10 @@ struct Levels {
 // Per-block timesteps (src/amr/bins_on.wgsl): the cycle's bin of every slot and the substep
 // being taken; a leaf whose step has not started on this substep is part way through a longer
 // one, seen through its half-step prediction, which the persistent PA/PB atlases hold from the
-// start of its step (amr/mid_on.wgsl). k null: every block steps every step (bins_off.wgsl).
+// start of its step (amr/mid_on.wgsl). k null: every block steps every step (bins_off.wgsl). on:
+// the pass belongs to a cycle of per-block timesteps (whose first assembly has no bins yet).
 struct AmrBins {
+  bool on = false;
   const int* k = nullptr;
   int sub = 0;
   const void* pa = nullptr;

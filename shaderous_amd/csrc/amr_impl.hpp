@@ -16,6 +16,7 @@
 // face).
 #pragma once
 #include "amr.hpp"
+#include "hydro_ref.hpp"
 #include "uniform_impl.hpp"
 
 namespace shx {
@@ -434,6 +435,14 @@ __device__ __forceinline__ bool amr_texel(const Params<T>& P, const int* __restr
 }
 
 // ---------------- assemble ----------------
+// The passes take BINS for a grid with per-block timesteps: its bins B, and the reference's
+// arrangement of the arithmetic (hydro_ref.hpp)
+template <typename T, bool BINS>
+__device__ __forceinline__ T leaf_rate(const Params<T>& P, const Prim<T>& w) {
+  if constexpr (BINS) return ref::rate_of(P, w);
+  else return rate_of(P, w);
+}
+
 // Workgroups of 256 per 3D block: 16 of cells, then two per face, a layer each (the edges and
 // corners are never assembled). Beside a coarser block the first wave of the first takes the whole
 // face, a lane per coarse cell and its eight texels from one set of slopes.
@@ -441,12 +450,12 @@ __device__ __forceinline__ bool amr_texel(const Params<T>& P, const int* __restr
 // at least: 47 us).
 constexpr int ASM_CELLS = AMR_CELLS / 256, ASM_CHUNKS = ASM_CELLS + 12;
 
-template <typename T, int LIM, int D = 3>
-__global__ __launch_bounds__(256, D == 3 && sizeof(T) == 4 ? 4 : 1) void k_amr_assemble(Params<T> P, Levels<T> LV, const int* __restrict__ tab,
-                                                      const int* __restrict__ list, const T4<T>* __restrict__ U1,
-                                                      const T4<T>* __restrict__ U2, T4<T>* __restrict__ W1,
-                                                      T4<T>* __restrict__ W2, unsigned long long* slot, AmrBins B,
-                                                      int count) {
+template <typename T, int LIM, int D, bool BINS>
+__global__ __launch_bounds__(256, D == 3 && sizeof(T) == 4 ? 4 : 1) void k_amr_assemble(
+    Params<T> P, Levels<T> LV, const int* __restrict__ tab, const int* __restrict__ list,
+    const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, T4<T>* __restrict__ W1, T4<T>* __restrict__ W2,
+    unsigned long long* slot, AmrBins B, int count) {
+  if constexpr (!BINS) B = AmrBins{};
   int b, t;
   if constexpr (D == 3) {
     b = blockIdx.x / ASM_CHUNKS;
@@ -518,7 +527,7 @@ __global__ __launch_bounds__(256, D == 3 && sizeof(T) == 4 ? 4 : 1) void k_amr_a
       W1[o] = v4<T>(w.rho, w.vx, w.vy, w.vz);
       W2[o] = v4<T>(w.p, w.cs, w.s, T(0));
       const bool inside = x >= 0 && y >= 0 && z >= 0 && x < AMR_BS && y < AMR_BS && z < AmrGeo<D>::ZC;
-      if (inside && is_leaf(tab, s)) r = rate_of(P, w) / level_dx(P, bt(tab, s, BT_LEVEL));
+      if (inside && is_leaf(tab, s)) r = leaf_rate<T, BINS>(P, w) / level_dx(P, bt(tab, s, BT_LEVEL));
     }
   }
   block_max_to(r, slot);
@@ -551,7 +560,7 @@ __global__ __launch_bounds__(256) void k_amr_block_rates(Params<T> P, const int*
   T r = T(0);
   for (int c = threadIdx.x; c < AmrGeo<D>::CELLS; c += 256) {
     const size_t o = (size_t)s * AmrGeo<D>::CELLS + c;
-    r = tmax(r, rate_of(P, prim_from_cons(P, U1[o], U2[o])) / dx);
+    r = tmax(r, leaf_rate<T, true>(P, prim_from_cons(P, U1[o], U2[o])) / dx);
   }
   r = wave_max(r);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = r;
@@ -622,7 +631,7 @@ __device__ __forceinline__ Prim<T> load_w(const T4<T>* __restrict__ W1, const T4
 // predict_cell (amr/predict.wgsl:90-181) on the atlas of block `slot` at texel (x, y, z); a zero
 // in mask drops that axis's slopes (ghosts next to a coarser block whose transverse neighbour
 // is an unassembled edge texel). In 2D the cell stands for its own z neighbours (:103-108).
-template <typename T, int LIM, bool ISEN, int D = 3>
+template <typename T, int LIM, bool ISEN, int D, bool BINS>
 __device__ __forceinline__ Half<T> predict_texel(const Params<T>& P, const T4<T>* __restrict__ W1,
                                                  const T4<T>* __restrict__ W2, int slot, int x, int y, int z, T mx,
                                                  T my, T mz, T dt) {
@@ -634,9 +643,15 @@ __device__ __forceinline__ Half<T> predict_texel(const Params<T>& P, const T4<T>
   const Prim<T> zm = D == 3 ? load_w<T>(W1, W2, base + c - AMR_PAD * AMR_PAD) : q;
   const Prim<T> zp = D == 3 ? load_w<T>(W1, W2, base + c + AMR_PAD * AMR_PAD) : q;
   AxisSlope<T> sl[3];
-  sl[0] = axis_slope<T, LIM, ISEN>(P, xm, q, xp, nullptr, nullptr);
-  sl[1] = axis_slope<T, LIM, ISEN>(P, ym, q, yp, nullptr, nullptr);
-  sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
+  if constexpr (BINS) {
+    sl[0] = ref::axis_slope<T, LIM, ISEN>(P, xm, q, xp);
+    sl[1] = ref::axis_slope<T, LIM, ISEN>(P, ym, q, yp);
+    sl[2] = ref::axis_slope<T, LIM, ISEN>(P, zm, q, zp);
+  } else {
+    sl[0] = axis_slope<T, LIM, ISEN>(P, xm, q, xp, nullptr, nullptr);
+    sl[1] = axis_slope<T, LIM, ISEN>(P, ym, q, yp, nullptr, nullptr);
+    sl[2] = axis_slope<T, LIM, ISEN>(P, zm, q, zp, nullptr, nullptr);
+  }
   const T mk[3] = {mx, my, mz};
 #pragma unroll
   for (int a = 0; a < 3; a++) {
@@ -644,16 +659,22 @@ __device__ __forceinline__ Half<T> predict_texel(const Params<T>& P, const T4<T>
     s.rho *= mk[a]; s.vx *= mk[a]; s.vy *= mk[a]; s.vz *= mk[a]; s.p *= mk[a]; s.s *= mk[a];
   }
   const T conv = (xp.vx - xm.vx) + (yp.vy - ym.vy) + (zp.vz - zm.vz);
-  const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
-  return hancock<T, LIM>(P, q, sl, conv, jump, slope_step<T, LIM>(P, dt));
+  if constexpr (BINS) {
+    const T jump = tmax(ref::jump_of(xm.p, xp.p), tmax(ref::jump_of(ym.p, yp.p), ref::jump_of(zm.p, zp.p)));
+    return ref::hancock(P, q, sl, conv, jump, dt);
+  } else {
+    const T jump = tmax(jump_over(P, xm.p, xp.p), tmax(jump_over(P, ym.p, yp.p), jump_over(P, zm.p, zp.p)));
+    return hancock<T, LIM>(P, q, sl, conv, jump, slope_step<T, LIM>(P, dt));
+  }
 }
 
-template <typename T, int LIM, bool ISEN, int D = 3>
+template <typename T, int LIM, bool ISEN, int D, bool BINS>
 __global__ __launch_bounds__(256) void k_amr_predict(Params<T> P, Levels<T> LV, const int* __restrict__ tab,
                                                      const int* __restrict__ list, const T4<T>* __restrict__ W1,
                                                      const T4<T>* __restrict__ W2, T4<T>* __restrict__ PA,
                                                      T4<T>* __restrict__ PB, const T* __restrict__ clk, AmrBins B,
                                                      int count) {
+  if constexpr (!BINS) B = AmrBins{};
   constexpr int NCH = pred_chunks<D>();
   int b, t;
   if constexpr (D == 3) {
@@ -708,8 +729,8 @@ __global__ __launch_bounds__(256) void k_amr_predict(Params<T> P, Levels<T> LV, 
   const T mx = (!at && (x == 0 || x == AMR_BS - 1)) ? T(0) : T(1);
   const T my = (!at && (y == 0 || y == AMR_BS - 1)) ? T(0) : T(1);
   const T mz = (!at && (z == 0 || z == AMR_BS - 1)) ? T(0) : T(1);
-  Half<T> h = at ? predict_texel<T, LIM, ISEN, D>(Pl, W1, W2, src, g.x, g.y, g.z, T(1), T(1), T(1), dt)
-                 : predict_texel<T, LIM, ISEN, D>(Pl, W1, W2, src, x, y, z, mx, my, mz, dt);
+  Half<T> h = at ? predict_texel<T, LIM, ISEN, D, BINS>(Pl, W1, W2, src, g.x, g.y, g.z, T(1), T(1), T(1), dt)
+                 : predict_texel<T, LIM, ISEN, D, BINS>(Pl, W1, W2, src, x, y, z, mx, my, mz, dt);
   if (at) {
     h.vx = bc_vel(h.vx, g.fx, g.sx);
     h.vy = bc_vel(h.vy, g.fy, g.sy);
@@ -732,7 +753,7 @@ __device__ __forceinline__ Half<T> load_half_at(const T4<T>* __restrict__ PA, co
 
 // flux_between on block s's atlas (hydro/flux.wgsl:254-347 with stored ghosts, amr/update.wgsl:
 // 50-58): the face between texel (x, y, z) and the next one along axis
-template <typename T, int LIM, int RS, bool ISEN, int D = 3>
+template <typename T, int LIM, int RS, bool ISEN, int D, bool BINS>
 __device__ __forceinline__ Flux<T> amr_flux(const Params<T>& P, const T4<T>* __restrict__ W1,
                                             const T4<T>* __restrict__ W2, const T4<T>* __restrict__ PA,
                                             const T4<T>* __restrict__ PB, int s, int x, int y, int z, int axis) {
@@ -741,9 +762,15 @@ __device__ __forceinline__ Flux<T> amr_flux(const Params<T>& P, const T4<T>* __r
   const Prim<T> wll = load_w<T>(W1, W2, o - e), wl = load_w<T>(W1, W2, o);
   const Prim<T> wr = load_w<T>(W1, W2, o + e), wrr = load_w<T>(W1, W2, o + 2 * e);
   const Half<T> hl = load_half_at<T>(PA, PB, o), hr = load_half_at<T>(PA, PB, o + e);
-  const Inc<T> il = edge<T, LIM, ISEN, true>(P, wll, wl, wr);
-  const Inc<T> ir = edge<T, LIM, ISEN, false>(P, wl, wr, wrr);
-  return face_flux<T, RS>(P, hl, il, hr, ir, axis);
+  if constexpr (BINS) {
+    const Inc<T> il = ref::edge<T, LIM, ISEN, true>(P, wll, wl, wr);
+    const Inc<T> ir = ref::edge<T, LIM, ISEN, false>(P, wl, wr, wrr);
+    return ref::face_flux<T, RS>(P, hl, il, hr, ir, axis);
+  } else {
+    const Inc<T> il = edge<T, LIM, ISEN, true>(P, wll, wl, wr);
+    const Inc<T> ir = edge<T, LIM, ISEN, false>(P, wl, wr, wrr);
+    return face_flux<T, RS>(P, hl, il, hr, ir, axis);
+  }
 }
 
 // TwoSum: s + e = a + b exactly (Knuth)
@@ -760,7 +787,7 @@ __device__ __forceinline__ void two_sum(T a, T b, T& s, T& e) {
 // across it is refined: the mean of the four fine fluxes through it (match_faces,
 // amr/update.wgsl:207-290; two in 2D, whose faces are edges: :246-251), summed in a fixed order,
 // with TwoSum when COMP.
-template <typename T, int LIM, int RS, bool ISEN, bool COMP, int D = 3>
+template <typename T, int LIM, int RS, bool ISEN, bool COMP, int D, bool BINS>
 __device__ __forceinline__ Flux<T> fine_face(const Params<T>& P, const int* __restrict__ tab,
                                              const T4<T>* __restrict__ W1, const T4<T>* __restrict__ W2,
                                              const T4<T>* __restrict__ PA, const T4<T>* __restrict__ PB, int np, int k,
@@ -786,7 +813,7 @@ __device__ __forceinline__ Flux<T> fine_face(const Params<T>& P, const int* __re
       const int fx = ax + (t1 == 0 ? i : 0) + (t2 == 0 ? j : 0);
       const int fy = ay + (t1 == 1 ? i : 0) + (t2 == 1 ? j : 0);
       const int fz = az + (t1 == 2 ? i : 0) + (t2 == 2 ? j : 0);
-      const Flux<T> f = amr_flux<T, LIM, RS, ISEN, D>(P, W1, W2, PA, PB, ch, fx, fy, fz, axis);
+      const Flux<T> f = amr_flux<T, LIM, RS, ISEN, D, BINS>(P, W1, W2, PA, PB, ch, fx, fy, fz, axis);
       const T fv[8] = {f.m, f.mx, f.my, f.mz, f.e, f.ei, f.s, f.vn};
 #pragma unroll
       for (int q = 0; q < 8; q++) {
@@ -822,12 +849,13 @@ struct UpdTile {
 
 // DEBUG (DEBUG_FLUX, amr/update.wgsl:324): instead of the update, each cell writes the mass
 // flux of its six faces, (x lo, x hi, y lo, y hi) to O1 and (z lo, z hi, 0, 0) to O2.
-template <typename T, int LIM, int RS, bool ISEN, bool MATCH, bool COMP, bool DEBUG = false, int D = 3>
+template <typename T, int LIM, int RS, bool ISEN, bool MATCH, bool COMP, bool DEBUG, int D, bool BINS>
 __global__ __launch_bounds__(UpdTile<D>::NT) void k_amr_update(
     Params<T> P, Levels<T> LV, const int* __restrict__ tab, const int* __restrict__ list,
     const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, const T4<T>* __restrict__ W1,
     const T4<T>* __restrict__ W2, const T4<T>* __restrict__ PA, const T4<T>* __restrict__ PB, T4<T>* __restrict__ O1,
     T4<T>* __restrict__ O2, const T* __restrict__ clk, AmrBins B) {
+  if constexpr (!BINS) B = AmrBins{};
   using UT = UpdTile<D>;
   constexpr int WX = UT::WX, WY = UT::WY, WZ = UT::WZ;
   constexpr int NFX = UT::NFX, NFY = UT::NFY;
@@ -854,7 +882,7 @@ __global__ __launch_bounds__(UpdTile<D>::NT) void k_amr_update(
       const int g = f - NFX - NFY;
       axis = 2; fx = g % WX; fy = (g / WX) % WY; fz = g / (WX * WY);
     }
-    const Flux<T> F = amr_flux<T, LIM, RS, ISEN, D>(P, W1, W2, PA, PB, s, x0 + fx - (axis == 0),
+    const Flux<T> F = amr_flux<T, LIM, RS, ISEN, D, BINS>(P, W1, W2, PA, PB, s, x0 + fx - (axis == 0),
                                                     y0 + fy - (axis == 1), z0 + fz - (axis == 2), axis);
     put_flux(tf, NF, f, F);
   }
@@ -897,7 +925,7 @@ __global__ __launch_bounds__(UpdTile<D>::NT) void k_amr_update(
         if (part == T(0)) {
           F = zero_flux<T>();
         } else {
-          F = fine_face<T, LIM, RS, ISEN, COMP, D>(P, tab, W1, W2, PA, PB, np, k, x, y, z);
+          F = fine_face<T, LIM, RS, ISEN, COMP, D, BINS>(P, tab, W1, W2, PA, PB, np, k, x, y, z);
           if (B.k) {
             F.m = F.m * part; F.mx = F.mx * part; F.my = F.my * part; F.mz = F.mz * part;
             F.e = F.e * part; F.ei = F.ei * part; F.s = F.s * part; F.vn = F.vn * part;
@@ -907,7 +935,7 @@ __global__ __launch_bounds__(UpdTile<D>::NT) void k_amr_update(
       } else if (B.k && np != s && bins_bin(B, np) < gbin) {
         // a faster leaf of the same level: half of its flux through the face, as it computes it
         const int an = hi ? -1 : AMR_BS - 1;
-        F = amr_flux<T, LIM, RS, ISEN, D>(P, W1, W2, PA, PB, np, axis == 0 ? an : x, axis == 1 ? an : y,
+        F = amr_flux<T, LIM, RS, ISEN, D, BINS>(P, W1, W2, PA, PB, np, axis == 0 ? an : x, axis == 1 ? an : y,
                                           axis == 2 ? an : z, axis);
         F.m = F.m * T(0.5); F.mx = F.mx * T(0.5); F.my = F.my * T(0.5); F.mz = F.mz * T(0.5);
         F.e = F.e * T(0.5); F.ei = F.ei * T(0.5); F.s = F.s * T(0.5); F.vn = F.vn * T(0.5);
@@ -943,8 +971,9 @@ __global__ __launch_bounds__(UpdTile<D>::NT) void k_amr_update(
   Params<T> Pl = P;
   Pl.dx = dx;
   const T dt = B.k ? clk[0] * T(1 << gbin) : clk[0];
+  const T dtdx = BINS ? dt / dx : tratio(dt, dx);
   T4<T> o1, o2;
-  advance(Pl, U1[o], U2[o], net, PB[(size_t)s * AmrGeo<D>::TEXELS + texd<D>(x, y, z)].x, tratio(dt, dx), o1, o2);
+  advance(Pl, U1[o], U2[o], net, PB[(size_t)s * AmrGeo<D>::TEXELS + texd<D>(x, y, z)].x, dtdx, o1, o2);
   O1[o] = o1;
   O2[o] = o2;
 }
@@ -1093,8 +1122,9 @@ struct AmrImpl {
                        void* w2, unsigned long long* slot) {
     if (count <= 0) return;
     const int grid = D == 3 ? count * ASM_CHUNKS : count + (count + 1) / 2;
-    hipLaunchKernelGGL((k_amr_assemble<T, LIM, D>), dim3(grid), dim3(256), 0, L.stream, P(L), LV(L), L.tab, list,
-                       (const T4<T>*)u1, (const T4<T>*)u2, (T4<T>*)w1, (T4<T>*)w2, slot, L.bins, count);
+    auto* kernel = L.bins.on ? k_amr_assemble<T, LIM, D, true> : k_amr_assemble<T, LIM, D, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, L.stream, P(L), LV(L), L.tab, list, (const T4<T>*)u1,
+                       (const T4<T>*)u2, (T4<T>*)w1, (T4<T>*)w2, slot, L.bins, count);
   }
   static void clock(const AmrLaunch& L, void* clk, unsigned long long* slot) {
     Params<T> P1 = P(L);
@@ -1105,26 +1135,31 @@ struct AmrImpl {
                       void* pb, const void* clk) {
     if (count <= 0) return;
     const int grid = D == 3 ? count * pred_chunks<D>() : count + (count + 3) / 4;
-    hipLaunchKernelGGL((k_amr_predict<T, LIM, ISEN, D>), dim3(grid), dim3(256), 0, L.stream, P(L), LV(L), L.tab, list,
-                       (const T4<T>*)w1, (const T4<T>*)w2, (T4<T>*)pa, (T4<T>*)pb, (const T*)clk, L.bins, count);
+    auto* kernel = L.bins.on ? k_amr_predict<T, LIM, ISEN, D, true> : k_amr_predict<T, LIM, ISEN, D, false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, L.stream, P(L), LV(L), L.tab, list, (const T4<T>*)w1,
+                       (const T4<T>*)w2, (T4<T>*)pa, (T4<T>*)pb, (const T*)clk, L.bins, count);
   }
   static void update(const AmrLaunch& L, const int* list, int count, bool match, bool comp, const void* u1,
                      const void* u2, const void* w1, const void* w2, const void* pa, const void* pb, void* o1, void* o2,
                      const void* clk, bool debug) {
     if (count <= 0) return;
-#define SHX_UPD(M, C, DB)                                                                                              \
-  hipLaunchKernelGGL((k_amr_update<T, LIM, RS, ISEN, M, C, DB, D>), dim3(count * UpdTile<D>::TILES),                   \
+#define SHX_UPD(M, C, DB, BN)                                                                                          \
+  hipLaunchKernelGGL((k_amr_update<T, LIM, RS, ISEN, M, C, DB, D, BN>), dim3(count * UpdTile<D>::TILES),               \
                      dim3(UpdTile<D>::NT), 0, L.stream, P(L), LV(L), L.tab, list, (const T4<T>*)u1, (const T4<T>*)u2,  \
                      (const T4<T>*)w1, (const T4<T>*)w2, (const T4<T>*)pa, (const T4<T>*)pb, (T4<T>*)o1, (T4<T>*)o2,   \
                      (const T*)clk, L.bins)
-    if (debug) {
-      if (!match) SHX_UPD(false, false, true);
-      else if (comp) SHX_UPD(true, true, true);
-      else SHX_UPD(true, false, true);
+    if (L.bins.on) {
+      // (a substep's leaves may all have faster neighbours: always the matching form)
+      if (comp) SHX_UPD(true, true, false, true);
+      else SHX_UPD(true, false, false, true);
+    } else if (debug) {
+      if (!match) SHX_UPD(false, false, true, false);
+      else if (comp) SHX_UPD(true, true, true, false);
+      else SHX_UPD(true, false, true, false);
     } else {
-      if (!match) SHX_UPD(false, false, false);
-      else if (comp) SHX_UPD(true, true, false);
-      else SHX_UPD(true, false, false);
+      if (!match) SHX_UPD(false, false, false, false);
+      else if (comp) SHX_UPD(true, true, false, false);
+      else SHX_UPD(true, false, false, false);
     }
 #undef SHX_UPD
   }

@@ -765,7 +765,8 @@ bool faster_neighbor(const shx_amr* s, const std::vector<int>& k, int b) {
 int run_cycle(shx_amr* s) {
   const int n = 1 << s->kbins;
   const int p = s->cur, q = 1 - p;
-  const AmrLaunch L = launch_of(s);
+  AmrLaunch L = launch_of(s);
+  L.bins.on = true;
   const AmrOps& o = s->ops;
   o.bank(L, s->clk);
   o.assemble(L, lp(s, s->all), s->all.count, s->U1[p], s->U2[p], s->W1, s->W2, s->slot);
