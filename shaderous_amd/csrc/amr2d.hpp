@@ -132,11 +132,11 @@ __global__ __launch_bounds__(256) void k_amr_flat_ghosts(Params<T> P, const int*
 }
 
 // The rest of the step. Bound by VALU issue with the barriers between its three phases; three
-// workgroups per CU. The adaptive shear layer's 3136 leaves (Koren, HLLC; 2176 plain, 896 of the
+// workgroups per CU (at most 96 VGPRs; at 100, two, shear 4096 takes 5% longer). The adaptive shear layer's 3136 leaves (Koren, HLLC; 2176 plain, 896 of the
 // others with a coarser neighbour): 106 us per step in passes (29 assembly, 30 half steps, 41
 // updates, clock), 75 so (21 ghosts, 34 and 16 the two launches, clock); 352 leaves (MC) 38 -> 28 us.
 template <typename T, int LIM, int RS, bool ISEN, bool MATCH, bool COMP>
-__global__ __launch_bounds__(AF_THREADS, 4) void k_amr_flat(
+__global__ __launch_bounds__(AF_THREADS, 5) void k_amr_flat(
     Params<T> G, const int* __restrict__ tab, const int* __restrict__ list, int nfull, const int* __restrict__ reg_of,
     T* __restrict__ R, const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, const T4<T>* __restrict__ W1,
     const T4<T>* __restrict__ W2, const T4<T>* __restrict__ PA, const T4<T>* __restrict__ PB, T4<T>* __restrict__ O1,
@@ -238,14 +238,17 @@ __global__ __launch_bounds__(AF_THREADS, 4) void k_amr_flat(
   }
   __syncthreads();
 
+  // the first launch writes the register, for every leaf with a coarser neighbour; the second only
+  // reads it (a store there, though of the same flux, would race with the coarser leaf's read)
   auto face = [&](int k, Flux<T> F) {
-    const int r = reg_of[s * 6 + k];
-    if (r >= 0) {
-      T4<T>* p = reinterpret_cast<T4<T>*>(R + ((size_t)r * AMR_BS + (k < 2 ? y : x)) * 8);
-      p[0] = v4<T>(F.m, F.mx, F.my, F.mz);
-      p[1] = v4<T>(F.e, F.ei, F.s, F.vn);
-    }
-    if constexpr (MATCH) {
+    if constexpr (!MATCH) {
+      const int r = reg_of[s * 6 + k];
+      if (r >= 0) {
+        T4<T>* p = reinterpret_cast<T4<T>*>(R + ((size_t)r * AMR_BS + (k < 2 ? y : x)) * 8);
+        p[0] = v4<T>(F.m, F.mx, F.my, F.mz);
+        p[1] = v4<T>(F.e, F.ei, F.s, F.vn);
+      }
+    } else {
       const int np = bt(tab, s, BT_NB + k);
       if (np >= 0 && !is_leaf(tab, np))
         return reg_mean_flat<T, COMP>(tab, reg_of, R, np, k, min(max(x, 0), AMR_BS - 1), min(max(y, 0), AMR_BS - 1), F);

@@ -1,0 +1,57 @@
+"""What the built kernels' code holds, read from the code objects of the last build (CPU only; the
+tools are the ROCm toolchain's)."""
+import os
+import re
+import subprocess
+
+import pytest
+
+from shaderous_amd import build
+
+LLVM = "/opt/rocm/llvm/bin"
+
+
+@pytest.fixture(scope="module")
+def code_objects(tmp_path_factory):
+    """The gfx950 code object of each translation unit, by its source's name."""
+    out = {}
+    folder = tmp_path_factory.mktemp("code")
+    for src in build.sources():
+        obj = os.path.join(build.BUILD, src + ".o")
+        if not src.endswith(".hip") or not os.path.exists(obj):
+            continue
+        fat, co = str(folder / (src + ".fat")), str(folder / (src + ".co"))
+        subprocess.run([f"{LLVM}/llvm-objcopy", "--dump-section", f".hip_fatbin={fat}", obj, os.devnull], check=True)
+        subprocess.run([f"{LLVM}/clang-offload-bundler", "--unbundle", "--type=o", f"--input={fat}",
+                        "--targets=hipv4-amdgcn-amd-amdhsa--gfx950", f"--output={co}"], check=True)
+        out[src] = co
+    if not out:
+        pytest.skip("no objects: build first (python -m shaderous_amd.build)")
+    return out
+
+
+def kernels(co):
+    """{kernel: bytes of code} of a code object."""
+    text = subprocess.run([f"{LLVM}/llvm-readelf", "-sW", co], check=True, capture_output=True, text=True).stdout
+    rows = [line.split() for line in text.splitlines() if " FUNC " in line]
+    return {r[-1]: int(r[2], 0) for r in rows}
+
+
+def test_second_flat_launch_stores_the_state_alone(code_objects):
+    """k_amr_flat with MATCH reads the flux register that the launch before it wrote: its only stores
+    are the leaf's two state vectors."""
+    co = code_objects["amr2d_f32.hip"]
+    found = [k for k in kernels(co) if re.match(r"_ZN3shx10k_amr_flatIfLi\dELi\dELb\dELb1E", k)]
+    assert len(found) == 20   # ten schemes, means compensated or not
+    text = subprocess.run([f"{LLVM}/llvm-objdump", "-d", "--no-show-raw-insn",
+                           "--disassemble-symbols=" + ",".join(found), co], check=True, capture_output=True,
+                          text=True).stdout
+    stores, name = {k: [] for k in found}, None
+    for line in text.splitlines():
+        head = re.match(r"[0-9a-f]+ <(\S+)>:", line)
+        if head:
+            name = head.group(1)
+        elif re.search(r"\b(global|buffer|flat)_(store|atomic)", line):
+            stores[name].append(line.split()[0])
+    bad = {k: v for k, v in stores.items() if v != ["global_store_dwordx4"] * 2}
+    assert not bad, bad
