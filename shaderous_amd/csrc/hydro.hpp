@@ -95,10 +95,11 @@ __device__ __forceinline__ double tsqrt(double x) { return __builtin_sqrt(x); }
 // hardware's log2 and exp2 (v_log_f32, v_exp_f32): the library powf's exact-case handling costs
 // ~40 instructions a call, and the isentropic reconstruction makes six calls per axis.
 __device__ __forceinline__ float tpow(float a, float b) { return __builtin_amdgcn_exp2f(b * __builtin_amdgcn_logf(a)); }
-// Double precision: the library's, as a call. Inlined at each of the twelve uses of a plane (and in
-// every role's loop) it made kernels of up to 347 KB, several times the instruction cache; one
-// that large (isentropic reconstruction beside reflecting faces) also came out of the compiler
-// wrong. Turbulence 96^3 in FP64, Koren + isentropic: 0.78 -> 0.50 ms per step.
+// Double precision: the library's, as a call. Inlined at its 24 uses of a plane it made kernels of up
+// to 348 KB, several times the instruction cache; the largest (k_fused_r, isentropic reconstruction
+// beside walls) gave wrong values, where the same source with the call gives the plain path's. What
+// in that build was wrong is not known, so the kernels' sizes are bounded by a test. Turbulence 96^3 in
+// FP64, Koren + isentropic: 0.78 -> 0.50 ms per step with the call.
 __device__ __attribute__((noinline)) inline double tpow(double a, double b) { return pow(a, b); }
 // WGSL mix(x, y, a) = x (1 - a) + y a
 template <typename T> __device__ __forceinline__ T tmix(T x, T y, T a) { return x * (T(1) - a) + y * a; }

@@ -55,3 +55,17 @@ def test_second_flat_launch_stores_the_state_alone(code_objects):
             stores[name].append(line.split()[0])
     bad = {k: v for k, v in stores.items() if v != ["global_store_dwordx4"] * 2}
     assert not bad, bad
+
+
+def test_kernels_stay_small(code_objects):
+    """A role kernel of 348 KB (FP64, Koren with the density reconstruction along the adiabat, walls;
+    pow inlined at its 24 uses, 1452 B of scratch per lane) computed wrong values where the same source
+    with pow as a call computed the plain path's. So pow stays a call, the uniform kernels stay
+    within a branch's reach (2^15 words, 128 KiB: no branch through a register), and
+    no kernel grows past the sizes that the GPU tests have covered."""
+    found = {src: kernels(co) for src, co in code_objects.items()}
+    assert "_ZN3shx4tpowEdd" in found["uniform_f64.hip"]
+    for src, sizes in found.items():
+        most = 128 << 10 if src.startswith(("uniform", "ens")) else 160 << 10
+        big = {k: v for k, v in sizes.items() if v >= most}
+        assert not big, (src, big)
