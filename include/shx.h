@@ -66,8 +66,11 @@ typedef struct {
   double t_end;        /* 1e30 (or +inf) for none */
   double fluff[3];     /* SimConfig.fluff: (rho below which the limits apply, max e, max v); rho 0 = off */
   int tile[3];         /* fused kernel's column tile (x, y) and z chunk; 0 = chosen by the grid's size
-                        * and the scheme. A flat FP32 grid takes the 2D tiles (16,16), (28,12),
-                        * (28,28) and strips (60, any number of rows) */
+                        * and the scheme. 3D: (32,16), (32,8) and (16,16), threads by role, (28,12)
+                        * and (28,28), threads in raster order; in FP64 (16,16) cells, in raster order
+                        * where a raster tile is asked for. Planes of 4 GiB or more are always in
+                        * raster order. A flat FP32 grid takes the 2D tiles (16,16), (28,12), (28,28)
+                        * and strips (60, any number of rows) */
   double org[3];       /* the domain's lower corner (domainLo, src/domain.ts:17-26; Params.org):
                         * cell (i, j, k) is centred at (i + 1/2) dx + org. Read by the
                         * diagnostics' centre of mass. Default -n[0] dx / 2 on every axis */

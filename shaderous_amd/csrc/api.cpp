@@ -424,12 +424,7 @@ int shx_create(const shx_config* cfg, shx_sim** out) {
   int cus = 0;
   if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c.device) != hipSuccess || cus < 1) cus = 256;
   // the 3D march's tile and chunk: as asked for, the rest by what it is expected to cost
-  int asked = -1;
-  for (int k = 0; c.tile[0] > 0 && s->es == 4 && k < FUSED_NTILES; k++) {
-    int tx, ty;
-    fused_tile_cells(k, tx, ty);
-    if (tx == c.tile[0] && ty == c.tile[1]) asked = k;
-  }
+  const int asked = fused_asked(c.n[0], c.n[1], s->es, c.tile[0], c.tile[1]);
   const auto shapes = shapes_of(c, cus, asked, c.tile[2]);
   s->tile = shapes.empty() ? asked : shapes[0].tile;
   s->zc = shapes.empty() ? std::min(c.tile[2] > 0 ? c.tile[2] : 32, c.n[2]) : shapes[0].zc;
@@ -666,9 +661,8 @@ int shx_profile(shx_sim* s, int steps, double ms[5]) {
 
 int shx_kernel_name(shx_sim* s, char* buf, size_t len) {
   if (!s || !buf || len == 0) return fail(SHX_EINVAL, "bad argument");
-  // threads by role: tiles of 32 x 16, 32 x 8 and 16 x 16
-  const bool roles = s->tile == FUSED_R32x16 || s->tile == FUSED_R32x8 || s->tile == FUSED_20x20;
-  const char* fused = s->flat2d ? (ens_is_rows(s->etile) ? "k_ens_rows" : "k_ens_fused") : (roles ? "k_fused_r" : "k_fused");
+  const char* march = fused_is_raster(s->tile) ? "k_fused" : "k_fused_r";
+  const char* fused = s->flat2d ? (ens_is_rows(s->etile) ? "k_ens_rows" : "k_ens_fused") : march;
   snprintf(buf, len, "%s", !s->fused ? "k_update" : fused);
   return SHX_OK;
 }
@@ -699,11 +693,16 @@ int shx_autotune(shx_sim* s, int reps, int chosen[3]) {
     HIPCHK(hipMemcpyAsync(s->clk, clk_saved.data(), clk_saved.size(), hipMemcpyHostToDevice, s->stream));
     return SHX_OK;
   };
-  // candidates: the 2D shapes, or the three likeliest chunks of each 3D tile
+  // candidates: the 2D shapes, the raster tiles on wide planes, or the three likeliest chunks of each
+  // 3D tile
   std::vector<FusedShape> cands;
   if (s->flat2d) {
     for (int k : {ENS_32x32, ENS_32x16, ENS_20x20, ENS_ROWS8, ENS_ROWS16, ENS_ROWS32, ENS_ROWSFIT})
       cands.push_back(FusedShape{k, 1, 0});
+  } else if (fused_wide(s->cfg.n[0], s->cfg.n[1], s->es)) {
+    for (int k : {FUSED_32x32, FUSED_32x16})
+      for (int z : {16, 32, 64, 128})
+        if (z == 16 || z <= s->cfg.n[2]) cands.push_back(FusedShape{k, z, 0});
   } else {
     int cus = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, s->cfg.device) != hipSuccess || cus < 1) cus = 256;

@@ -14,20 +14,40 @@ struct Launch {
   size_t ncell;
 };
 
-// Column tiles of the fused kernel: k_fused's (block BX x BY threads in raster order, tile
-// (BX - 4) x (BY - 4) cells) and k_fused_r's (threads by role, tiles of 32 x 16, 32 x 8 or, as
-// FUSED_20x20, 16 x 16 cells: the only one in FP64). k_fused is slower on every grid measured; it
-// is run where a plane exceeds the 4 GiB that k_fused_r addresses, and on request.
-enum { FUSED_20x20 = 0, FUSED_32x16 = 1, FUSED_32x32 = 2, FUSED_R32x16 = 3, FUSED_R32x8 = 4, FUSED_NTILES = 5 };
+// Column tiles of the fused kernel: k_fused_r's (threads by role, tiles of 32 x 16, 32 x 8 or, as
+// FUSED_20x20, 16 x 16 cells: the only one in FP64) and k_fused's (block BX x BY threads in raster
+// order, tile (BX - 4) x (BY - 4) cells; FUSED_RASTER20 in FP64 alone, the others in FP32 alone).
+// k_fused is slower on every grid measured: it is run on wide planes and on request.
+enum { FUSED_20x20 = 0, FUSED_32x16 = 1, FUSED_32x32 = 2, FUSED_R32x16 = 3, FUSED_R32x8 = 4, FUSED_RASTER20 = 5,
+       FUSED_NTILES = 6 };
+inline bool fused_is_raster(int tile) { return tile == FUSED_32x16 || tile == FUSED_32x32 || tile == FUSED_RASTER20; }
+// A plane of 4 GiB or more: k_fused_r addresses a plane with 32 bits
+inline bool fused_wide(int nx, int ny, int elem) { return (size_t)nx * ny * 4 * elem >= (size_t)1 << 32; }
 // cells per tile along x and y
 inline void fused_tile_cells(int tile, int& tx, int& ty) {
   switch (tile) {
-    case FUSED_20x20: tx = 16; ty = 16; break;
+    case FUSED_20x20:
+    case FUSED_RASTER20: tx = 16; ty = 16; break;
     case FUSED_32x16: tx = 28; ty = 12; break;
     case FUSED_32x32: tx = 28; ty = 28; break;
     case FUSED_R32x16: tx = 32; ty = 16; break;
     default: tx = 32; ty = 8; break;
   }
+}
+
+// The k_fused_r or k_fused tile a grid is stepped by where the configuration or the plane's size
+// decides it, else -1. FP64 has one tile, 16 x 16 cells, in raster order where a raster tile is
+// asked for.
+inline int fused_asked(int nx, int ny, int elem, int tx, int ty) {
+  int asked = -1;
+  for (int k = 0; tx > 0 && k < FUSED_RASTER20; k++) {
+    int x, y;
+    fused_tile_cells(k, x, y);
+    if (x == tx && y == ty) asked = k;
+  }
+  if (elem == 8) asked = asked >= 0 && fused_is_raster(asked) ? FUSED_RASTER20 : -1;
+  if (fused_wide(nx, ny, elem) && !(asked >= 0 && fused_is_raster(asked))) asked = elem == 8 ? FUSED_RASTER20 : FUSED_32x16;
+  return asked;
 }
 
 // A launch of the 3D march: tile and planes per chunk, and what it is expected to cost, in planes of

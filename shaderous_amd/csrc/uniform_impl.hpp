@@ -749,20 +749,16 @@ struct UniformImpl {
   // za, zb: the half steps of planes 0 and nz - 1 for a non-periodic z face (null: z periodic)
   static void fused(const Launch& L, int tile, const void* u1, const void* u2, void* o1, void* o2, const ClockRefs& ck,
                     const void* za, const void* zb, int zc, bool debug) {
-    // the role kernel addresses a plane with 32 bits: beyond 4 GiB a plane, the raster tiles
-    const Params<T>& P = *static_cast<const Params<T>*>(L.params);
-    const bool wide = (size_t)P.n[0] * P.n[1] * sizeof(T4<T>) >= (size_t)1 << 32;
+    // (wide planes come with a raster tile: fused_asked)
     if constexpr (sizeof(T) == 8) {
-      if (wide) fused_tile<20, 20>(L, u1, u2, o1, o2, ck, za, zb, zc, debug);
+      if (tile == FUSED_RASTER20) fused_tile<20, 20>(L, u1, u2, o1, o2, ck, za, zb, zc, debug);
       else fused_roles<16, 16>(L, u1, u2, o1, o2, ck, za, zb, zc, debug);
     } else {
-      if (wide) tile = FUSED_32x16;
       switch (tile) {
         case FUSED_R32x16: fused_roles<32, 16>(L, u1, u2, o1, o2, ck, za, zb, zc, debug); break;
         case FUSED_R32x8: fused_roles<32, 8>(L, u1, u2, o1, o2, ck, za, zb, zc, debug); break;
         case FUSED_32x32: fused_tile<32, 32>(L, u1, u2, o1, o2, ck, za, zb, zc, debug); break;
         case FUSED_32x16: fused_tile<32, 16>(L, u1, u2, o1, o2, ck, za, zb, zc, debug); break;
-        // 16 x 16 cells: threads by role in FP32
         default: fused_roles<16, 16>(L, u1, u2, o1, o2, ck, za, zb, zc, debug); break;
       }
     }
