@@ -126,7 +126,7 @@ __global__ __launch_bounds__(256) void k_amr_flat_ghosts(Params<T> P, const int*
   for (int b = wg - ghosts - ends; b < count; b += gridDim.x - ghosts - ends) {
     const int s = list[b];
     const size_t o = (size_t)s * AmrGeo<2>::CELLS + tid;
-    r = tmax(r, rate_of(P, prim_from_cons(P, U1[o], U2[o])) / level_dx(P, bt(tab, s, BT_LEVEL)));
+    r = tmax(r, tquot(rate_of(P, prim_from_cons(P, U1[o], U2[o])), level_dx(P, bt(tab, s, BT_LEVEL))));
   }
   block_max_to(r, slot);
 }

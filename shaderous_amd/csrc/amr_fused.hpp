@@ -372,7 +372,7 @@ __global__ void k_amr_queue_start(int* qctl) {
 // Bound by VALU issue and, on a few hundred leaves, by how evenly the pairs divide among the CUs.
 // On the 3D blast (8^3 root blocks, two refinements, 1618 leaves, MC, HLLC): 462 us with one loop
 // for all roles, ghost cases chosen by lane in it; 342 us with a loop per role (-26%). The rate's
-// division is by the block (a quotient by one dx keeps the order, so its maximum has the same bits).
+// division is by the block (tquot by one dx keeps the order, so the maximum has the same bits).
 template <typename T, int LIM, int RS, bool ISEN>
 __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) == 4 ? 3 : 1)) void k_amr_fused(
     Params<T> P, const int* __restrict__ tab, const int* __restrict__ list, int count,
@@ -635,7 +635,7 @@ __global__ __launch_bounds__((sizeof(T) == 4 ? 2 : 1) * AF_THREADS, (sizeof(T) =
         update(AMR_BS - 1, u1, u2, fz);
       }
       // the next step's rate / dx (assemble's leaf-cell rate, amr/assemble.wgsl:77-154)
-      rate_max = tmax(rate_max, rate / dx);
+      rate_max = tmax(rate_max, tquot(rate, dx));
     } else {
       // the ghost columns: a same-level leaf's cells from U, others from the shell; edges (the
       // ghost planes' texels beside them) are zero

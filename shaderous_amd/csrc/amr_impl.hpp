@@ -527,7 +527,7 @@ __global__ __launch_bounds__(256, D == 3 && sizeof(T) == 4 ? 4 : 1) void k_amr_a
       W1[o] = v4<T>(w.rho, w.vx, w.vy, w.vz);
       W2[o] = v4<T>(w.p, w.cs, w.s, T(0));
       const bool inside = x >= 0 && y >= 0 && z >= 0 && x < AMR_BS && y < AMR_BS && z < AmrGeo<D>::ZC;
-      if (inside && is_leaf(tab, s)) r = leaf_rate<T, BINS>(P, w) / level_dx(P, bt(tab, s, BT_LEVEL));
+      if (inside && is_leaf(tab, s)) r = tquot(leaf_rate<T, BINS>(P, w), level_dx(P, bt(tab, s, BT_LEVEL)));
     }
   }
   block_max_to(r, slot);
@@ -543,7 +543,7 @@ __global__ __launch_bounds__(256) void k_amr_rates(Params<T> P, Levels<T> LV, co
   T r = T(0);
   for (int c = threadIdx.x; c < AmrGeo<D>::CELLS; c += 256) {
     const size_t o = (size_t)s * AmrGeo<D>::CELLS + c;
-    r = tmax(r, rate_of(P, prim_from_cons(P, U1[o], U2[o])) / dx);
+    r = tmax(r, tquot(rate_of(P, prim_from_cons(P, U1[o], U2[o])), dx));
   }
   block_max_to(r, slot);
 }
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(256) void k_amr_block_rates(Params<T> P, const int*
   T r = T(0);
   for (int c = threadIdx.x; c < AmrGeo<D>::CELLS; c += 256) {
     const size_t o = (size_t)s * AmrGeo<D>::CELLS + c;
-    r = tmax(r, leaf_rate<T, true>(P, prim_from_cons(P, U1[o], U2[o])) / dx);
+    r = tmax(r, tquot(leaf_rate<T, true>(P, prim_from_cons(P, U1[o], U2[o])), dx));
   }
   r = wave_max(r);
   if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = r;
@@ -587,7 +587,7 @@ __global__ void k_amr_bank(T* clk) {
 template <typename T>
 __global__ void k_amr_clock_cycle(Params<T> P, T* clk, unsigned long long* slot, T cycle) {
   const T rate = from_bits<T>(*slot);
-  T dt = P.cfl * T(1) / tmax(rate, T(1e-30));
+  T dt = tquot(P.cfl, tmax(rate, T(1e-30)));
   dt = tmin(dt, P.dt_max);
   const T remaining = P.t_end - clk[1];
   if (remaining <= T(1e-6) * tabs(P.t_end)) dt = T(0);

@@ -89,6 +89,15 @@ __device__ __forceinline__ float tratio(float a, float b) {
   return __builtin_fmaf(__builtin_fmaf(-q, b, a), r, q);
 }
 __device__ __forceinline__ double tratio(double a, double b) { return a / b; }
+// The quotients that decide the step, a rate over a cell size and cfl dx over the largest rate: formed
+// in several kernels, with the same need. Spelled out in the form the compiler gives a plain a / b
+// in them today (mantissas by the approximate reciprocal, exponents apart; about an ulp), which never
+// falls as a rises, so that a quotient of the largest rate is the largest quotient.
+__device__ __forceinline__ float tquot(float a, float b) {
+  return __builtin_ldexpf(__builtin_amdgcn_frexp_mantf(a) * __builtin_amdgcn_rcpf(__builtin_amdgcn_frexp_mantf(b)),
+                          __builtin_amdgcn_frexp_expf(a) - __builtin_amdgcn_frexp_expf(b));
+}
+__device__ __forceinline__ double tquot(double a, double b) { return a / b; }
 __device__ __forceinline__ float tsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ double tsqrt(double x) { return __builtin_sqrt(x); }
 // Single-precision pow as WGSL defines it, exp2(b log2 a) (every base here is positive), by the
@@ -714,7 +723,7 @@ __device__ __forceinline__ void clock_pass(const Params<T>& P, T* clk, T max_rat
     clk[1] = t;
     clk[3] = clk[3] + T(1);
   }
-  T dt = P.cfl * P.dx / tmax(max_rate, T(1e-30));
+  T dt = tquot(P.cfl * P.dx, tmax(max_rate, T(1e-30)));
   dt = tmin(dt, P.dt_max);
   T remaining = P.t_end - clk[1];
   if (remaining <= T(1e-6) * tabs(P.t_end)) dt = T(0);
