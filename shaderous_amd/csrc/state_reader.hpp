@@ -18,7 +18,6 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
-#include <system_error>
 #include <thread>
 
 namespace shx {
@@ -92,8 +91,8 @@ class StateReader {
     for (int w = 1; w < n; w++) {
       try {
         others[w] = std::thread(work, w);
-      } catch (const std::system_error&) {
-        break;   // fewer threads do it too
+      } catch (...) {
+        break;   // no thread, or no memory for one: fewer do it too
       }
     }
     work(0);
