@@ -489,7 +489,7 @@ int shx_create(const shx_config* cfg, shx_sim** out) {
   }
   int rc = build_graphs(s);
   if (rc) { shx_destroy(s); return rc; }
-  s->rb->fit(2 * bytes);
+  s->rb->fit(2 * bytes, 2 * bytes);
   *out = s;
   return SHX_OK;
 }

@@ -1058,7 +1058,8 @@ int shx_amr_create(const shx_config* cfg, const shx_amr_layout* layout, const in
     *out = nullptr;
     return rc;
   }
-  (*out)->rb->fit(2 * (*out)->ncell * 4 * (*out)->es);
+  const size_t state = (*out)->ncell * 8 * (*out)->es;
+  (*out)->rb->fit(state, state);
   return SHX_OK;
 }
 
@@ -1334,7 +1335,8 @@ int shx_amr_regrid(shx_amr* s, const int* blocks, int nblocks) {
   }
   std::swap(*s, *ns);
   std::swap(s->rb, ns->rb);   // its slots stay; more of them if the state has outgrown them
-  s->rb->fit(2 * s->ncell * 4 * s->es);
+  const size_t state = s->ncell * 8 * s->es;
+  s->rb->fit(state, state);
   shx_amr_destroy(ns);
   return SHX_OK;
 }

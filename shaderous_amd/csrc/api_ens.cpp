@@ -243,9 +243,12 @@ int shx_ens_create(const shx_config* cfg, int count, const int* sizes, shx_ens**
   }
   int rc = build_graphs(e);
   if (rc) { shx_ens_destroy(e); return rc; }
-  size_t largest = 0;
-  for (int i = 0; i < count; i++) largest = std::max(largest, (size_t)e->nx[i] * e->ny[i]);
-  e->rb->fit(2 * largest * 4 * e->es);
+  size_t least = (size_t)-1, most = 0;
+  for (int i = 0; i < count; i++) {
+    least = std::min(least, (size_t)e->nx[i] * e->ny[i] * 8 * e->es);
+    most = std::max(most, (size_t)e->nx[i] * e->ny[i] * 8 * e->es);
+  }
+  e->rb->fit(least, most);
   *out = e;
   return SHX_OK;
 }

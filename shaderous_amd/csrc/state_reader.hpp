@@ -25,18 +25,22 @@ namespace shx {
 class StateReader {
  public:
   static constexpr int SLOTS = 8;
-  static constexpr size_t LEAST = (size_t)512 << 10, MOST = (size_t)4 << 20;   // bytes per slot
-  static constexpr size_t LARGE = (size_t)8 << 20;   // states read by several threads
+  static constexpr size_t LEAST = (size_t)512 << 10;   // states read through one slot
+  static constexpr size_t MOST = (size_t)4 << 20;      // bytes per slot
+  static constexpr size_t LARGE = (size_t)8 << 20;     // states read by several threads
 
   ~StateReader() { drop(); }
 
-  // Slots for states of up to `bytes`: 8 (at most half the host's threads) of 1 to 4 MiB for large
-  // ones, else one. Without memory for them reads are plain copies.
-  void fit(size_t bytes) {
+  // Slots for states of `least` to `most` bytes: 8 (at most half the host's threads) of 1 to 4 MiB
+  // where there are large ones, else one for the small ones if there are any. (Pinned memory takes
+  // 0.05 ms of the 0.2 in which a small sim is made, whatever its size: one read through it saves as
+  // much.) Without memory for them reads are plain copies.
+  void fit(size_t least, size_t most) {
+    if (least > LEAST && most < LARGE) return;
     const unsigned int hw = std::thread::hardware_concurrency();
-    const int n = bytes < LARGE ? 1 : std::max(1, std::min(SLOTS, (int)(hw / 2)));
-    const size_t per = bytes < LARGE ? LEAST : std::min(MOST, bytes / SLOTS);
-    if (n <= count_ && per <= 2 * chunk_) return;
+    const int n = most < LARGE ? 1 : std::max(1, std::min(SLOTS, (int)(hw / 2)));
+    const size_t per = most < LARGE ? std::min(LEAST, (most + 4095) & ~(size_t)4095) : std::min(MOST, most / SLOTS);
+    if (n <= count_ && per <= (n == 1 ? room() : 2 * chunk_)) return;
     drop();
     if (hipHostMalloc((void**)&pinned_, n * per, hipHostMallocDefault) != hipSuccess) {
       (void)hipGetLastError();
@@ -54,7 +58,7 @@ class StateReader {
   // Two arrays of `bytes` each, in stream order; returns when both are there. Reads of one sim take
   // their turns.
   hipError_t read(hipStream_t stream, int device, void* d0, const void* s0, void* d1, const void* s1, size_t bytes) {
-    const bool small = 2 * bytes <= LEAST;
+    const bool small = 2 * bytes <= std::min(LEAST, room());
     if (count_ == 0 || (!small && (count_ == 1 || 2 * bytes < LARGE)) || !pageable(d0) || !pageable(d1)) {
       hipError_t e = hipMemcpyAsync(d0, s0, bytes, hipMemcpyDeviceToHost, stream);
       if (e == hipSuccess) e = hipMemcpyAsync(d1, s1, bytes, hipMemcpyDeviceToHost, stream);
@@ -112,6 +116,7 @@ class StateReader {
     }
     return a.type == hipMemoryTypeUnregistered;
   }
+  size_t room() const { return count_ * chunk_; }
   void drop() {
     for (; count_ > 0; count_--) (void)hipEventDestroy(done_[count_ - 1]);
     if (pinned_) (void)hipHostFree(pinned_);

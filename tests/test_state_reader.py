@@ -1,5 +1,6 @@
-"""StateReader (csrc/state_reader.hpp) on the CPU, against a stub of the HIP calls it makes: a large
-state arrives whole also where some of its threads cannot be started, for want of memory (the
+"""StateReader (csrc/state_reader.hpp) on the CPU, against a stub of the HIP calls it makes: states of
+every size arrive whole whatever size its slots were made for, and pinned memory is taken for those
+that go through it alone; a large state arrives whole also where some of its threads cannot be started, for want of memory (the
 thread's own record) as for want of threads."""
 import shutil
 import subprocess
@@ -19,7 +20,8 @@ typedef int hipError_t;
 enum { hipSuccess = 0, hipHostMallocDefault = 0, hipEventDisableTiming = 2, hipMemcpyDeviceToHost = 2 };
 enum { hipMemoryTypeUnregistered = 0 };
 struct hipPointerAttribute_t { int type; };
-inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { *p = malloc(n); return *p ? 0 : 2; }
+static size_t pinned = 0;
+inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { pinned = n; *p = malloc(n); return *p ? 0 : 2; }
 inline hipError_t hipHostFree(void* p) { free(p); return 0; }
 inline hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = nullptr; return 0; }
 inline hipError_t hipEventDestroy(hipEvent_t) { return 0; }
@@ -52,7 +54,7 @@ int main() {
   std::vector<char> a(n), b(n), x(n), y(n);
   for (size_t i = 0; i < n; i++) { a[i] = (char)(i * 7 + i / 4099); b[i] = (char)(i * 5 + 1); }
   shx::StateReader r;
-  r.fit(2 * n);
+  r.fit(2 * n, 2 * n);
   for (int fail = -1; fail < 6; fail++) {
     std::fill(x.begin(), x.end(), 0);
     std::fill(y.begin(), y.end(), 0);
@@ -62,6 +64,23 @@ int main() {
     counting = false;
     if (rc != 0 || x != a || y != b) return 1;
     printf("allocation %d failed: read whole\n", fail);
+  }
+  // readers made for states of one size, or of a range as an ensemble's, read any other
+  const size_t K = 1024, M = K * K;
+  const size_t fits[][3] = {{3000, 3000, 4096}, {512 * K, 512 * K, 512 * K}, {512 * K + 16, 512 * K + 16, 0},
+                            {8 * M - 16, 8 * M - 16, 0}, {128 * K, 2 * M, 512 * K}, {4 * K, 96 * K, 96 * K}};
+  for (auto& f : fits) {
+    pinned = 0;
+    shx::StateReader s;
+    s.fit(f[0], f[1]);
+    if (pinned != f[2]) return 2;
+    for (size_t each : {(size_t)16, 64 * K, 256 * K, 256 * K + 16, M, 4 * M, 9 * M + 16}) {
+      std::fill(x.begin(), x.end(), 0);
+      std::fill(y.begin(), y.end(), 0);
+      if (s.read(nullptr, 0, x.data(), a.data(), y.data(), b.data(), each) != 0) return 3;
+      if (memcmp(x.data(), a.data(), each) || memcmp(y.data(), b.data(), each) || x[each] || y[each]) return 4;
+      s.fit(2 * each, 2 * each);   // as after a re-mesh
+    }
   }
   return 0;
 }
