@@ -737,18 +737,28 @@ int shx_autotune(shx_sim* s, int reps, int chosen[3]) {
     *ms = t / n;
     return SHX_OK;
   };
-  // (the first series only wakes the device and tells how many steps of a small grid to time)
+  // every candidate over `reps` steps (the first series only wakes the device), then on a small grid,
+  // whose steps are short against the events' resolution, those within 30% of the fastest over a
+  // third of a millisecond
   double ms;
   int rc = timed(bt, bz, reps, &ms);
   if (rc) return rc;
   const int n = std::max(reps, (int)std::min(32.0, 0.3 / std::max(ms, 1e-3)));
+  std::vector<double> took(cands.size(), 1e30);
+  double least = 1e30;
   for (size_t i = 0; i < cands.size(); i++) {
-    const int ti = cands[i].tile, z = cands[i].zc;
-    if (i > 0 && ti == cands[0].tile && z == cands[0].zc) continue;
-    rc = timed(ti, z, n, &ms);
+    if (i > 0 && cands[i].tile == cands[0].tile && cands[i].zc == cands[0].zc) continue;
+    rc = timed(cands[i].tile, cands[i].zc, reps, &took[i]);
     if (rc) return rc;
-    if (ms < best) { best = i == 0 ? 0.97 * ms : ms; bt = ti; bz = z; }
+    least = std::min(least, took[i]);
   }
+  for (size_t i = 0; n > reps && i < cands.size(); i++) {
+    if (took[i] > 1.3 * least) { took[i] = 1e30; continue; }
+    rc = timed(cands[i].tile, cands[i].zc, n, &took[i]);
+    if (rc) return rc;
+  }
+  for (size_t i = 0; i < cands.size(); i++)
+    if (took[i] < best) { best = i == 0 ? 0.97 * took[i] : took[i]; bt = cands[i].tile; bz = cands[i].zc; }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (s->flat2d) {
