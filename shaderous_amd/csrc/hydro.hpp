@@ -549,8 +549,9 @@ __device__ __forceinline__ Flux<T> riemann(const Params<T>& P, const Side<T>& l,
   o.ei = o.m * ((left ? l.pr : r.pr) * P.igm1);
   o.s = o.m * (left ? l.s : r.s);
   o.vn = u;
-  // The HLL state between the waves: the flux itself where the star densities are not positive
-  // (and for HLL) and where the face is flagged.
+  // The HLL state between the waves: the flux itself where the star densities are not positive (a
+  // sound speed of zero, or below the rounding of the velocity: else ql < 0 < qr), for HLL, and
+  // where the face is flagged.
   const bool star = ql < T(0) && qr > T(0);
   if (!super && (RS == RS_HLL || !star || w_hll != T(0))) {
     const SideFlux<T> a = side_flux(P, l);
