@@ -31,15 +31,19 @@ class StateReader {
 
   ~StateReader() { drop(); }
 
-  // Slots for states of `least` to `most` bytes: 8 (at most half the host's threads) of 1 to 4 MiB
-  // where there are large ones, else one for the small ones if there are any. (Pinned memory takes
-  // 0.05 ms of the 0.2 in which a small sim is made, whatever its size: one read through it saves as
-  // much.) Without memory for them reads are plain copies.
+  // Slots for states of `least` to `most` bytes: 8 (at most half the host's threads) of a 16th of the
+  // largest, 1 to 4 MiB, where there are large ones, else one for the small ones if there are any.
+  // Pinned memory costs: 0.05 ms for the least of it, a quarter of the time in which a small sim is made
+  // (one read through it saves as much), and the first touch of its pages, on the first read. States of
+  // 16 and 32 MiB take 2.2 and 3.0 ms on their first read with slots twice as large, 1.0 and 1.8 with
+  // these; 0.53 and 0.89 against 0.59 and 0.92 on later ones. Without memory for them reads are plain
+  // copies.
   void fit(size_t least, size_t most) {
     if (least > LEAST && most < LARGE) return;
     const unsigned int hw = std::thread::hardware_concurrency();
     const int n = most < LARGE ? 1 : std::max(1, std::min(SLOTS, (int)(hw / 2)));
-    const size_t per = most < LARGE ? std::min(LEAST, (most + 4095) & ~(size_t)4095) : std::min(MOST, most / SLOTS);
+    const size_t per = most < LARGE ? std::min(LEAST, (most + 4095) & ~(size_t)4095)
+                                    : std::min(MOST, std::max((size_t)1 << 20, most / 16));
     if (n <= count_ && per <= (n == 1 ? room() : 2 * chunk_)) return;
     drop();
     if (hipHostMalloc((void**)&pinned_, n * per, hipHostMallocDefault) != hipSuccess) {
