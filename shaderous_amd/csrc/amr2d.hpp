@@ -3,14 +3,15 @@
 // faces and updates, where the passes (amr_impl.hpp) carry the cells' texels (W) and half steps
 // (PA, PB) through HBM, ten times the state's own bytes. The ghosts stay apart: their chain of table
 // and cell reads needs more waves in flight than a workgroup with a leaf in LDS leaves room for
-// (formed inside, the two launches for 3136 leaves took 72 and 34 us against 21 + 34 and 16). The values are the passes':
+// (formed inside, the two launches for 3136 leaves took 72 and 34 us against 21 + 34 and 16). The
+// values are the passes':
 //  - threads 0-255 the cells, 256-319 the first layer of face ghosts, 320-383 the second
 //    (af_column);
 //  - a ghost's half step "at source" (amr/predict.wgsl:183-221): beside a same-level leaf the
 //    texels here are the ones that leaf's own predictor reads, but for a ghost at a face's end,
 //    whose stencil reaches past the face: that texel, as the leaf across assembles it, is formed
-//    besides (two per face, kept in PA's and PB's corners, which nothing else uses); beside a coarser block in place with masked slopes; a boundary image's
-//    from the cell it images;
+//    besides (two per face, kept in PA's and PB's corners, which nothing else uses); beside a
+//    coarser block in place with masked slopes; a boundary image's from the cell it images;
 //  - coarse-fine faces through a flux register, as the fused 3D march's: a leaf writes the fluxes
 //    of its faces on a coarser block, and the leaves with a refined neighbour, in a second launch,
 //    take the means of the two fine fluxes (match_faces). The first launch steps the other leaves,
@@ -132,8 +133,9 @@ __global__ __launch_bounds__(256) void k_amr_flat_ghosts(Params<T> P, const int*
 }
 
 // The rest of the step. Bound by VALU issue with the barriers between its three phases; three
-// workgroups per CU (at most 96 VGPRs; at 100, two, shear 4096 takes 5% longer). The adaptive shear layer's 3136 leaves (Koren, HLLC; 2176 plain, 896 of the
-// others with a coarser neighbour): 106 us per step in passes (29 assembly, 30 half steps, 41
+// workgroups per CU (at most 96 VGPRs; at 100, two, the step below takes 5% longer). The adaptive
+// shear layer's 3136 leaves (Koren, HLLC; 2176 plain, 896 of the others with a coarser neighbour):
+// 106 us per step in passes (29 assembly, 30 half steps, 41
 // updates, clock), 75 so (21 ghosts, 34 and 16 the two launches, clock); 352 leaves (MC) 38 -> 28 us.
 template <typename T, int LIM, int RS, bool ISEN, bool MATCH, bool COMP>
 __global__ __launch_bounds__(AF_THREADS, 5) void k_amr_flat(

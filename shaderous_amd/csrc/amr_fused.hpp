@@ -15,9 +15,10 @@
 //    coarser block (as it computed them), and the coarser leaf reads the four fine fluxes of
 //    each of its faces there and takes their mean (TwoSum-compensated when asked), which is
 //    what match_faces (amr/update.wgsl:207-290) recomputes from the finer block's atlas.
-//  - one launch for all leaves: workgroups take pairs from a device queue (leaves with no
-//    refined neighbour first, then the others level by level from the finest); a leaf with a
-//    refined neighbour first waits for the finer leaves across it (a done flag per slot, set
+//  - one launch for all leaves: workgroups take pairs from a device queue (level by level from the
+//    finest the leaves with a coarse-fine face, those that only supply a coarser leaf before those
+//    that wait for finer ones, with leaves that do neither between and at the end: build_lists in
+//    api_amr.cpp); a leaf with a refined neighbour first waits for the finer leaves across it (a done flag per slot, set
 //    with release order after their march). The queue hands out pairs in order and a leaf only
 //    waits for leaves earlier in it, all of which are held by running workgroups, so the waits
 //    end; each is bounded besides, and a wait that runs out sets an error flag the host reports.
@@ -152,7 +153,6 @@ __device__ __forceinline__ void scale_inc(Inc<T>& q, T m) {
 constexpr int SH_TEXELS = 4 * AF_NT + AF_RING * AMR_BS;                     // 1600 + 128 * 16 = 3648
 constexpr int SH_HALVES = 64 * AMR_BS + 2 * AMR_BS * AMR_BS;                 // 1024 + 512 = 1536
 constexpr int SH_ITEMS = SH_TEXELS + SH_HALVES;                               // 5184
-constexpr int SH_CHUNKS = (SH_ITEMS + 255) / 256;
 
 __device__ __forceinline__ int ghost_plane_slot(int z) { return z == -2 ? 0 : (z == -1 ? 1 : (z == AMR_BS ? 2 : 3)); }
 

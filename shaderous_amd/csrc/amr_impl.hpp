@@ -446,8 +446,8 @@ __device__ __forceinline__ T leaf_rate(const Params<T>& P, const Prim<T>& w) {
 // Workgroups of 256 per 3D block: 16 of cells, then two per face, a layer each (the edges and
 // corners are never assembled). Beside a coarser block the first wave of the first takes the whole
 // face, a lane per coarse cell and its eight texels from one set of slopes.
-// All of the 3D blast's 624 blocks (root 4): 131 us with every texel by itself in raster order, 88 us so (240 MB
-// at least: 47 us).
+// All of the 3D blast's 624 blocks (root 4): 131 us with every texel by itself in raster order, 88 us
+// so (240 MB at least: 47 us).
 constexpr int ASM_CELLS = AMR_CELLS / 256, ASM_CHUNKS = ASM_CELLS + 12;
 
 template <typename T, int LIM, int D, bool BINS>

@@ -208,9 +208,9 @@ __device__ __forceinline__ T koren_weight(T below, T above, T k) {
   const T e = T(1.5) - b * b;
   return tclamp(e - a * a, T(0), T(1));
 }
-// Koren's increment toward the face `near` lies on (least: the minmod of the two), blended by w from the limited value to the
-// plain one (w = 1 gives the plain one exactly: the limited value is no larger). The early return
-// of koren.wgsl gives the blend's value per channel, so each channel is formed on its own.
+// Koren's increment toward the face `near` lies on (least: the minmod of the two), blended by w from
+// the limited value to the plain one (w = 1 gives the plain one exactly: the limited value is no
+// larger). The early return of koren.wgsl gives the blend's value per channel, so each channel is formed on its own.
 template <typename T>
 __device__ __forceinline__ T koren_edge(T far, T near, T least, T w) {
   const T fr = (far + T(2) * near) * T(1.0 / 6.0);
@@ -387,8 +387,8 @@ __device__ __forceinline__ T jump_over(const Params<T>& P, T pm, T pp) {
 }
 
 // The Hancock half step from the cell, the three axis slopes, and for the shock detector the
-// convergence and the largest jump_over; h: slope_step. gamma p is the rho c_s^2 of predictor.wgsl, without the
-// sound speed's root.
+// convergence and the largest jump_over; h: slope_step. gamma p is the rho c_s^2 of
+// predictor.wgsl, without the sound speed's root.
 template <typename T, int LIM>
 __device__ __forceinline__ Half<T> hancock(const Params<T>& P, const Prim<T>& q, const AxisSlope<T> sl[3],
                                            T conv, T jump, T h) {

@@ -46,7 +46,8 @@ inline int fused_asked(int nx, int ny, int elem, int tx, int ty) {
     if (x == tx && y == ty) asked = k;
   }
   if (elem == 8) asked = asked >= 0 && fused_is_raster(asked) ? FUSED_RASTER20 : -1;
-  if (fused_wide(nx, ny, elem) && !(asked >= 0 && fused_is_raster(asked))) asked = elem == 8 ? FUSED_RASTER20 : FUSED_32x16;
+  if (fused_wide(nx, ny, elem) && !(asked >= 0 && fused_is_raster(asked)))
+    asked = elem == 8 ? FUSED_RASTER20 : FUSED_32x16;
   return asked;
 }
 

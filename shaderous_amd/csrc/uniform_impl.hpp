@@ -9,8 +9,9 @@
 //             face of the block's box computed once into LDS, then each cell's update
 //
 // FUSED path, one kernel per step: k_fused_r (uniform_roles.hpp), threads by role, or the raster
-// form k_fused (below: planes beyond 4 GiB, and tiles asked for by their cells): a block owns a column tile of (BX - 4) x (BY - 4)
-// cells plus a two-cell halo ring and marches along z through a chunk of planes. Each plane's
+// form k_fused (below: planes of 4 GiB and more, and tiles asked for by their cells): a block owns a
+// column tile of (BX - 4) x (BY - 4) cells plus a two-cell halo ring and marches along z through a
+// chunk of planes. Each plane's
 // primitives are converted once, staged in LDS for the x/y neighbours and kept in registers for
 // the z neighbours; each cell's half step and edge increments are computed once; each face is
 // solved once; the conservative update of the plane behind is written, and the next step's
@@ -739,8 +740,9 @@ struct UniformImpl {
     bool mapbc = za != nullptr;
     for (int a = 0; a < 2; a++) mapbc |= P.bc_lo[a] != BC_PERIODIC || P.bc_hi[a] != BC_PERIODIC;
 #define SHX_FUSED_R(D, M)                                                                                            \
-  hipLaunchKernelGGL((k_fused_r<T, LIM, RS, ISEN, TX, TY, D, M>), g, dim3(RoleTile<TX, TY>::template launch<T>()), 0, L.stream, P,     \
-                     (const T4<T>*)u1, (const T4<T>*)u2, (T4<T>*)o1, (T4<T>*)o2, step_clock<T>(ck), (const T4<T>*)za, \
+  hipLaunchKernelGGL((k_fused_r<T, LIM, RS, ISEN, TX, TY, D, M>), g,                                                 \
+                     dim3(RoleTile<TX, TY>::template launch<T>()), 0, L.stream, P, (const T4<T>*)u1,                  \
+                     (const T4<T>*)u2, (T4<T>*)o1, (T4<T>*)o2, step_clock<T>(ck), (const T4<T>*)za,                   \
                      (const T4<T>*)zb, zc)
     if (debug) { if (mapbc) SHX_FUSED_R(true, true); else SHX_FUSED_R(true, false); }
     else { if (mapbc) SHX_FUSED_R(false, true); else SHX_FUSED_R(false, false); }

@@ -219,7 +219,8 @@ __device__ __forceinline__ Flux<T> net_z(const Flux<T>& xy, const Flux<T>& lo, c
 // A plane's byte offsets fit 32 bits (the launcher's rule), so a load is a scalar base and one
 // vector offset.
 template <typename T, int LIM, int RS, bool ISEN, int TX, int TY, bool DEBUG, bool MAPBC>
-__global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile<TX, TY>::template minw<T, LIM>())) void k_fused_r(
+__global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()),
+                             (RoleTile<TX, TY>::template minw<T, LIM>())) void k_fused_r(
     Params<T> P, const T4<T>* __restrict__ U1, const T4<T>* __restrict__ U2, T4<T>* __restrict__ O1,
     T4<T>* __restrict__ O2, StepClock<T> C, const T4<T>* __restrict__ ZA, const T4<T>* __restrict__ ZB, int zc) {
   using RT = RoleTile<TX, TY>;
@@ -503,7 +504,8 @@ __global__ __launch_bounds__((RoleTile<TX, TY>::template launch<T>()), (RoleTile
       cs = pp.cs;
       __syncthreads();
       if (face) {
-        const Flux<T> F = face_from_sides_rt<T, RS>(P, PL::side(L, ax ? PL::SX : PL::SY, PL::SK, t.off(ax ? -1 : -BX)), lo, ax ? 0 : 1);
+        const SideData<T> below = PL::side(L, ax ? PL::SX : PL::SY, PL::SK, t.off(ax ? -1 : -BX));
+        const Flux<T> F = face_from_sides_rt<T, RS>(P, below, lo, ax ? 0 : 1);
         PL::put_flux(L, ax ? PL::FX : PL::FY, t, F);
       }
       __syncthreads();
