@@ -54,7 +54,8 @@ __device__ __forceinline__ float tabs(float a) { return __builtin_fabsf(a); }
 __device__ __forceinline__ double tabs(double a) { return __builtin_fabs(a); }
 // The same for operands that come from memory or LDS, where the compiler would first quiet each
 // one (v_max x, x) in case it is a signaling NaN: arithmetic makes none, and states are checked
-// finite when they are set
+// finite when they are set. (The compiler's hazard pass does not look at inline assembly's operands:
+// a test of the built code holds that none is a transcendental's result of the slot before.)
 __device__ __forceinline__ float raw_min(float a, float b) {
   float r;
   asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));

@@ -69,3 +69,34 @@ def test_kernels_stay_small(code_objects):
         most = 128 << 10 if src.startswith(("uniform", "ens")) else 160 << 10
         big = {k: v for k, v in sizes.items() if v >= most}
         assert not big, (src, big)
+
+
+def test_transcendentals_are_not_read_in_the_next_slot(code_objects):
+    """On gfx950 a vector instruction must not read the result of a transcendental one (v_rcp, v_sqrt, v_exp,
+    ...) right behind it. The compiler sees to that, but not for the operands of inline assembly
+    (raw_min, raw_max in hydro.hpp), so it is checked over the whole code."""
+    trans = re.compile(r"v_(rcp|sqrt|rsq|log|exp|sin|cos)_")
+
+    def regs(text):
+        out = {int(a) for a in re.findall(r"\bv(\d+)\b", text)}
+        for a, b in re.findall(r"\bv\[(\d+):(\d+)\]", text):
+            out |= set(range(int(a), int(b) + 1))
+        return out
+
+    seen, bad = 0, []
+    for src, co in code_objects.items():
+        text = subprocess.run([f"{LLVM}/llvm-objdump", "-d", "--no-show-raw-insn", "--no-leading-addr", co], check=True,
+                              capture_output=True, text=True).stdout
+        last = None
+        for line in text.splitlines():
+            op, _, rest = line.split("//")[0].strip().partition(" ")
+            if last and op.startswith("v_") and not trans.match(op):
+                first, _, others = rest.partition(",")
+                read = regs(others) | (regs(first) if op.startswith(("v_fmac", "v_cmp")) else set())
+                if last & read:
+                    bad.append((src, line.strip()))
+            last = None
+            if trans.match(op):
+                last = regs(rest.partition(",")[0])
+                seen += 1
+    assert seen > 10000 and not bad, bad[:5]
