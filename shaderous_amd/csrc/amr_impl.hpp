@@ -443,12 +443,19 @@ __device__ __forceinline__ T leaf_rate(const Params<T>& P, const Prim<T>& w) {
   else return rate_of(P, w);
 }
 
-// Workgroups of 256 per 3D block: 16 of cells, then two per face, a layer each (the edges and
-// corners are never assembled). Beside a coarser block the first wave of the first takes the whole
-// face, a lane per coarse cell and its eight texels from one set of slopes.
-// All of the 3D blast's 624 blocks (root 4): 131 us with every texel by itself in raster order, 88 us
-// so (240 MB at least: 47 us).
-constexpr int ASM_CELLS = AMR_CELLS / 256, ASM_CHUNKS = ASM_CELLS + 12;
+// Workgroups of 256 per 3D block: 25 of the cell planes with their x and y ghosts, then a layer of a z
+// face each (the edges and corners are never assembled). Beside a coarser block one wave takes the
+// whole face, a lane per coarse cell and its eight texels from one set of slopes: the first of a z
+// face's first layer, or one of the four of a last workgroup for the x and y faces. 32 in all, two of
+// them empty: workgroups go to the 8 XCDs in turn, so the planes of a block and of its x and y
+// neighbours, whose cells its ghosts are, meet in the same L2; the others take turns by block, so
+// that no XCD has all the coarse faces.
+// The 3D blast's substeps with per-block timesteps (root 4, 624 blocks), on average: 74 us with every
+// texel by itself in raster order, 60 with cells and faces a workgroup of their own each, 53 so; 216
+// unrefined blocks 29, 38, 28 (ghost layers of their own store a line per x ghost and read the
+// neighbour's cells through another L2).
+constexpr int ASM_PLANES = AMR_BS * AMR_PAD * AMR_PAD / 256, ASM_CHUNKS = 32;
+static_assert(ASM_PLANES * 256 == AMR_BS * AMR_PAD * AMR_PAD && ASM_PLANES + 5 <= ASM_CHUNKS, "assembly chunks");
 
 template <typename T, int LIM, int D, bool BINS>
 __global__ __launch_bounds__(256, D == 3 && sizeof(T) == 4 ? 4 : 1) void k_amr_assemble(
@@ -461,29 +468,32 @@ __global__ __launch_bounds__(256, D == 3 && sizeof(T) == 4 ? 4 : 1) void k_amr_a
     b = blockIdx.x / ASM_CHUNKS;
     const int c = blockIdx.x % ASM_CHUNKS;
     t = c * 256 + threadIdx.x;
-    if (c >= ASM_CELLS) {
-      const int s = list[b], f = (c - ASM_CELLS) >> 1, layer = (c - ASM_CELLS) & 1, axis = f >> 1;
+    if (c >= ASM_PLANES) {
+      const int s = list[b], g = (c - ASM_PLANES + b) % (ASM_CHUNKS - ASM_PLANES), wave = threadIdx.x >> 6;
+      if (g > 4) return;
+      const bool zface = g < 4;
+      const int f = zface ? 4 + (g >> 1) : wave, layer = zface ? g & 1 : 0, axis = f >> 1;
       const size_t at = (size_t)s * AmrGeo<D>::TEXELS;
       auto put = [&](int x, int y, int z, const Prim<T>& w) {
         W1[at + tex(x, y, z)] = v4<T>(w.rho, w.vx, w.vy, w.vz);
         W2[at + tex(x, y, z)] = v4<T>(w.p, w.cs, w.s, T(0));
       };
       if (bt(tab, s, BT_NB + f) == -1) {
-        if (layer > 0 || threadIdx.x >= 64) return;
+        if (layer > 0 || (zface && wave > 0)) return;
         // the coarse cell's first fine texel: even along every axis
-        const int n = (f & 1) ? AMR_BS : -2, i = 2 * (threadIdx.x & 7), j = 2 * (threadIdx.x >> 3);
+        const int n = (f & 1) ? AMR_BS : -2, i = 2 * (threadIdx.x & 7), j = 2 * ((threadIdx.x >> 3) & 7);
         const int x = axis == 0 ? n : i, y = axis == 1 ? n : (axis == 0 ? i : j), z = axis == 2 ? n : j;
         int par[3];
-        const Prolong<T> g = coarse_cell<T, LIM, D>(P, tab, U1, U2, s, x, y, z, bt(tab, s, BT_COARSE + f), par, B);
+        const Prolong<T> pr = coarse_cell<T, LIM, D>(P, tab, U1, U2, s, x, y, z, bt(tab, s, BT_COARSE + f), par, B);
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-          const Cons<T> u = g.child(k & 1, (k >> 1) & 1, k >> 2);
+          const Cons<T> u = pr.child(k & 1, (k >> 1) & 1, k >> 2);
           put(x + (k & 1), y + ((k >> 1) & 1), z + (k >> 2), prim_from_cons(P, u.a, u.b));
         }
         return;
       }
-      const int n = (f & 1) ? AMR_BS + layer : -1 - layer, i = threadIdx.x & 15, j = threadIdx.x >> 4;
-      const int x = axis == 0 ? n : i, y = axis == 1 ? n : (axis == 0 ? i : j), z = axis == 2 ? n : j;
+      if (!zface) return;
+      const int x = threadIdx.x & 15, y = threadIdx.x >> 4, z = (f & 1) ? AMR_BS + layer : -1 - layer;
       Prim<T> w;
       if (amr_texel<T, LIM, D, false>(P, tab, U1, U2, s, x, y, z, w, B)) put(x, y, z, w);
       return;
@@ -501,9 +511,12 @@ __global__ __launch_bounds__(256, D == 3 && sizeof(T) == 4 ? 4 : 1) void k_amr_a
   int x, y, z;
   bool any = t < AmrGeo<D>::TEXELS && b < count;
   if constexpr (D == 3) {
-    x = t % AMR_BS;
-    y = (t / AMR_BS) % AMR_BS;
-    z = t / (AMR_BS * AMR_BS);
+    x = t % AMR_PAD - AMR_NG;
+    y = (t / AMR_PAD) % AMR_PAD - AMR_NG;
+    z = t / (AMR_PAD * AMR_PAD);
+    // (a ghost beside a coarser block is another workgroup's)
+    const bool gx = x < 0 || x >= AMR_BS, gy = y < 0 || y >= AMR_BS;
+    any = gx != gy ? bt(tab, list[b], BT_NB + (gx ? x >= AMR_BS : 2 + (y >= AMR_BS))) != -1 : !gx;
   } else {
     // 2D: the cells' workgroups take only cells, the others the face ghosts face by face (-x,
     // +x, -y, +y; two layers of 16), so no wave mixes the cells' copy with a ghost's
