@@ -818,7 +818,9 @@ __device__ __forceinline__ Flux<T> fine_face(const Params<T>& P, const int* __re
   T sum[8], err[8];
 #pragma unroll
   for (int q = 0; q < 8; q++) { sum[q] = T(0); err[q] = T(0); }
-#pragma unroll
+  // (with bins in 3D one copy of the face for the two rows: the copies of the six sides otherwise
+  // outgrow the instruction cache, 103 KB with Koren + isentropic)
+#pragma unroll(BINS && D == 3 ? 1 : 2)
   for (int j = 0; j < 2; j++)
 #pragma unroll
     for (int i = 0; i < 2; i++) {
